@@ -120,14 +120,17 @@ struct ovl_ctx {
     double *staging = nullptr;
     size_t staging_bytes = 0;
 
-    // multi-shift CG
-    int ms_no = 0;
+    // multi-shift CG of the mode-block fields
     void *ms_ps = nullptr, *ms_r = nullptr, *ms_q = nullptr, *ms_w = nullptr, *ms_chi = nullptr;
     double *ms_coef = nullptr;
-    int *ms_active = nullptr;
+    ovl::CgMode *ms_modes = nullptr;
+    int *ms_active[2] = {nullptr, nullptr};
 
-    // Ritz vectors (one block)
-    void *rz[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+    // single vectors ([spin][colour][site]): links, the two vectors of a drop-in, CG work vectors,
+    // Ritz vectors, the start vector of the Ritz bounds, partial results and scalar states
+    void *s1_links = nullptr, *s1_vec = nullptr, *s1_cg = nullptr, *s1_ritz = nullptr, *s1_start = nullptr;
+    double *s1_part = nullptr;
+    void *s1_state = nullptr;
 
     // timing
     bool profiling = false;
@@ -1146,82 +1149,125 @@ int apply_h2(ovl_ctx *c, const Geom &g, const void *v, void *w, void *q, double 
     return hop(c, g, P64, P64, b);
 }
 
-// Zolotrr (OverlapU.cpp:5-149) for all modes of `in`: chi = sum_k bz_k (h^2 + dz_k)^{-1} in.
-// Per-mode scalars live on the host; the chi accumulation is folded into the shift update.
-int mscg(ovl_ctx *c, const Geom &g, const void *in, void *chi, const double *bz, const double *dz, int no,
-         double cgerr, int nitcgm, int *max_iter, int *nonconv)
+// tolerance and iteration cap of the reference's multi-shift CG (OverlapOperator.cpp:25-64)
+constexpr double CG_TOL = 1e-16;
+constexpr int CG_CAP = 1000;
+
+ovl::CgShifts zolotarev_shifts(double lmin, double lmax)
 {
-    const size_t fb = (size_t)g.nblk * c->blk64_elems * 16;      // stride of one shift vector for g
-    const size_t fmax = (size_t)c->g.nblk * c->blk64_elems * 16;  // allocation: the whole context
-    if (c->ms_no < no) {
-        dfree(c->ms_ps);
-        c->ms_no = no;
-    }
-    RETCHK(dalloc(c, &c->ms_ps, fmax * no));
-    RETCHK(dalloc(c, &c->ms_r, fmax));
-    RETCHK(dalloc(c, &c->ms_q, fmax));
-    RETCHK(dalloc(c, &c->ms_w, fmax));
-    const int nm = g.nblk * g.mb;
-    RETCHK(dalloc(c, (void **)&c->ms_coef, sizeof(double) * (size_t)c->g.nblk * c->g.mb * 3 * 32));
-    RETCHK(dalloc(c, (void **)&c->ms_active, sizeof(int) * (size_t)c->g.nblk * c->g.mb));
+    ovl::CgShifts sh;
+    ovl_zolotarev_coefficients(lmin, lmax, 1e-12, ovl::CG_SHIFTS, sh.bz, sh.dz);
+    return sh;
+}
+
+// Zolotrr (OverlapU.cpp:5-149) for all modes of `in`: chi = sum_k bz_k (h^2 + dz_k)^{-1} in.  The per-mode
+// scalars stay on the device; the host enqueues iterations and looks for the end of them once per
+// batch.  A finished mode is left alone by the later iterations, so a batch only costs time: it is one
+// iteration where an iteration moves more than CG_BATCH_BYTES (about 0.2 ms, ten times the 20 us that
+// the host's look costs) and eight of them below.
+constexpr double CG_BATCH_BYTES = 1e9;
+int mscg(ovl_ctx *c, const Geom &g, const void *in, void *chi, const ovl::CgShifts &sh, int *nonconv)
+{
+    constexpr int no = ovl::CG_SHIFTS;
+    const size_t fb = (size_t)g.nblk * c->blk64_elems * 16;
+    const int nm = g.nblk * g.mb, chunks = ovl::mode_dot_chunks();
+    RETCHK(dalloc(c, &c->ms_ps, fb * no));
+    RETCHK(dalloc(c, &c->ms_r, fb));
+    RETCHK(dalloc(c, &c->ms_q, fb));
+    RETCHK(dalloc(c, &c->ms_w, fb));
+    RETCHK(dalloc(c, (void **)&c->ms_coef, sizeof(double) * (size_t)nm * 3 * no));
+    RETCHK(dalloc(c, (void **)&c->ms_modes, sizeof(ovl::CgMode) * (size_t)nm));
+    for (auto &p : c->ms_active) RETCHK(dalloc(c, (void **)&p, sizeof(int) * (size_t)nm));
     HIPCHK(c, ovl::launch_lincomb(g, g.nblk, P64, c->ms_r, in, 1, 0, nullptr, 0, 0, c->st));
     for (int k = 0; k < no; ++k)
         HIPCHK(c, ovl::launch_lincomb(g, g.nblk, P64, (char *)c->ms_ps + k * fb, in, 1, 0, nullptr, 0, 0, c->st));
     HIPCHK(c, ovl::launch_lincomb(g, g.nblk, P64, chi, in, 0, 0, nullptr, 0, 0, c->st));
-    std::vector<cplx> d;
-    RETCHK(mode_dot(c, g, c->ms_r, c->ms_r, d));
-    std::vector<double> rn(nm), bn(nm), betam(nm, 1.0), a0(nm, 0.0);
-    std::vector<double> z((size_t)nm * no, 1.0), gc((size_t)nm * no, 1.0), be((size_t)nm * no, 0.0), al((size_t)nm * no, 0.0);
-    std::vector<int> act(nm), it(nm, 0);
-    std::vector<double> coefA(nm), coef((size_t)nm * 3 * no, 0.0);
-    for (int i = 0; i < nm; ++i) {
-        rn[i] = d[i].real();
-        bn[i] = std::sqrt(rn[i]);
-        act[i] = rn[i] > cgerr * bn[i];
-    }
-    *max_iter = 0;
-    *nonconv = 0;
-    while (std::any_of(act.begin(), act.end(), [](int v) { return v != 0; })) {
-        HIPCHK(c, hipMemcpyAsync(c->ms_active, act.data(), sizeof(int) * nm, hipMemcpyHostToDevice, c->st));
-        RETCHK(apply_h2(c, g, c->ms_ps, c->ms_w, c->ms_q, dz[0]));
-        std::vector<cplx> pq;
-        RETCHK(mode_dot(c, g, c->ms_ps, c->ms_q, pq));
-        for (int i = 0; i < nm; ++i) coefA[i] = act[i] ? rn[i] / pq[i].real() : 0.0;
-        HIPCHK(c, hipMemcpyAsync(c->ms_coef, coefA.data(), sizeof(double) * nm, hipMemcpyHostToDevice, c->st));
-        HIPCHK(c, ovl::launch_axpy_modes(g, c->ms_r, c->ms_q, c->ms_coef, 1, -1.0, c->ms_active, c->st));
-        std::vector<cplx> rr;
-        RETCHK(mode_dot(c, g, c->ms_r, c->ms_r, rr));
-        std::vector<int> nact(nm, 0);
-        for (int i = 0; i < nm; ++i) {
-            if (!act[i]) continue;
-            double *zi = &z[(size_t)i * no], *bi = &be[(size_t)i * no], *ai = &al[(size_t)i * no], *gi = &gc[(size_t)i * no];
-            bi[0] = coefA[i];
-            for (int k = 1; k < no; ++k) {
-                const double dr = bi[0] * a0[i] * (1.0 - zi[k]) + betam[i] * (1.0 + (dz[k] - dz[0]) * bi[0]);
-                zi[k] = betam[i] / dr;
-                bi[k] = bi[0] * zi[k];
-            }
-            a0[i] = rr[i].real() / rn[i];
-            rn[i] = rr[i].real();
-            for (int k = 0; k < no; ++k) {
-                ai[k] = a0[i] * zi[k] * bi[k] / bi[0];
-                gi[k] = gi[k] * zi[k];
-                coef[((size_t)i * no + k) * 3 + 0] = bz[k] * bi[k];
-                coef[((size_t)i * no + k) * 3 + 1] = ai[k];
-                coef[((size_t)i * no + k) * 3 + 2] = gi[k];
-            }
-            betam[i] = bi[0];
-            it[i]++;
-            nact[i] = (rn[i] > cgerr * bn[i]) && it[i] < nitcgm;
-            if (it[i] >= nitcgm && rn[i] > cgerr * bn[i]) (*nonconv)++;
-            *max_iter = std::max(*max_iter, it[i]);
+    HIPCHK(c, ovl::launch_mode_dot_partial(g, c->ms_r, c->ms_r, c->partial, c->st));
+    HIPCHK(c, ovl::launch_cgm_begin(g, c->partial, chunks, c->ms_modes, c->ms_active[0], CG_TOL, c->st));
+    const int batch = (2.0 * no + 9.0) * (double)fb > CG_BATCH_BYTES ? 1 : 8;
+    std::vector<int> act(nm);
+    for (int it = 0; it < CG_CAP; ++it) {
+        if (it % batch == 0) {
+            HIPCHK(c, hipMemcpyAsync(act.data(), c->ms_active[it & 1], sizeof(int) * nm, hipMemcpyDeviceToHost, c->st));
+            HIPCHK(c, hipStreamSynchronize(c->st));
+            if (std::none_of(act.begin(), act.end(), [](int v) { return v != 0; })) break;
         }
-        HIPCHK(c, hipMemcpyAsync(c->ms_coef, coef.data(), sizeof(double) * coef.size(), hipMemcpyHostToDevice, c->st));
+        const int *cur = c->ms_active[it & 1];
+        RETCHK(apply_h2(c, g, c->ms_ps, c->ms_w, c->ms_q, sh.dz[0]));
+        HIPCHK(c, ovl::launch_mode_dot_partial(g, c->ms_ps, c->ms_q, c->partial, c->st));
+        HIPCHK(c, ovl::launch_cgm_alpha(g, c->partial, chunks, c->ms_modes, cur, c->st));
+        HIPCHK(c, ovl::launch_cgm_residual(g, c->ms_r, c->ms_q, c->ms_modes, cur, c->partial, chunks, c->st));
+        HIPCHK(c, ovl::launch_cgm_scalars(g, c->partial, chunks, c->ms_modes, cur, c->ms_active[1 - (it & 1)], c->ms_coef,
+                                          sh, CG_TOL, CG_CAP, c->st));
         HIPCHK(c, ovl::launch_mscg_update(g, no, (double *)c->ms_ps, (double *)chi, (const double *)c->ms_r, c->ms_coef,
-                                          c->ms_active, c->st));
-        HIPCHK(c, hipStreamSynchronize(c->st));
-        act = nact;
+                                          cur, c->st));
     }
+    std::vector<ovl::CgMode> modes(nm);
+    HIPCHK(c, hipMemcpyAsync(modes.data(), c->ms_modes, sizeof(ovl::CgMode) * nm, hipMemcpyDeviceToHost, c->st));
+    HIPCHK(c, hipStreamSynchronize(c->st));
+    *nonconv = 0;
+    for (const ovl::CgMode &m : modes)
+        if (m.it >= CG_CAP && m.rn > CG_TOL * m.bn) (*nonconv)++;
+    return OVL_OK;
+}
+
+// ---- one vector ([spin][colour][site]) ----
+// links, partial results and states of the single-vector kernels
+int ensure_single(ovl_ctx *c)
+{
+    const size_t V = (size_t)c->g.V;
+    RETCHK(dalloc(c, &c->s1_links, 16 * 3 * V * c->g.nc * c->g.nc));
+    RETCHK(dalloc(c, (void **)&c->s1_part, sizeof(double) * ovl::single_partial_len(c->g)));
+    return dalloc(c, &c->s1_state, 2 * std::max(sizeof(ovl::CgMode), ovl::RITZ_SOLVES * sizeof(ovl::RitzState)) + sizeof(int) * 2);
+}
+size_t vec1_bytes(const ovl_ctx *c) { return (size_t)c->g.V * c->ncomp * 16; }
+// two ints after the states: non-finite flags of a drop-in's inputs
+int *single_flags(const ovl_ctx *c)
+{
+    return (int *)((char *)c->s1_state + 2 * std::max(sizeof(ovl::CgMode), ovl::RITZ_SOLVES * sizeof(ovl::RitzState)));
+}
+
+// the single-vector form of mscg: `in` and the links c->s1_links are set, *chi receives the solution
+int mscg1(ovl_ctx *c, const void *in, const ovl::CgShifts &sh, void **chi, int *nonconv)
+{
+    RETCHK(dalloc(c, &c->s1_cg, vec1_bytes(c) * (ovl::CG_SHIFTS + 4)));
+    ovl::Cg1Call k{};
+    k.work = c->s1_cg;
+    k.state = c->s1_state;
+    k.part = c->s1_part;
+    k.in = in;
+    k.links = c->s1_links;
+    k.amass = amass(c);
+    k.tol = CG_TOL;
+    k.sh = sh;
+    k.cap = CG_CAP;
+    HIPCHK(c, ovl::launch_cg1_start(c->g, k, c->st));
+    ovl::CgMode m{};
+    constexpr int batch = 8;  // an iteration is four short launches: look every eighth (20 us in 150 us)
+    for (int it = 0;; ++it) {
+        if (it % batch == 0 || it == CG_CAP) {
+            HIPCHK(c, hipMemcpyAsync(&m, (ovl::CgMode *)c->s1_state + (it & 1), sizeof m, hipMemcpyDeviceToHost, c->st));
+            HIPCHK(c, hipStreamSynchronize(c->st));
+            if (!m.act || it == CG_CAP) break;
+        }
+        HIPCHK(c, ovl::launch_cg1_iteration(c->g, k, it, c->st));
+    }
+    *nonconv = m.it >= CG_CAP && m.rn > CG_TOL * m.bn;
+    *chi = ovl::cg1_chi(c->g, c->s1_cg);
+    return OVL_OK;
+}
+
+int cg_result(ovl_ctx *c, int nonconv)
+{
+    if (nonconv)
+        return fail(c, OVL_E_CONVERGE, "multi-shift CG reached 1000 iterations for " + std::to_string(nonconv) + " mode(s)");
+    return OVL_OK;
+}
+
+int check_interval(ovl_ctx *c, double lmin, double lmax)
+{
+    if (!(lmin > 0.0) || !(lmax > lmin) || !std::isfinite(lmax))
+        return fail(c, OVL_E_SPECTRUM, "Zolotarev interval needs 0 < lmin < lmax");
     return OVL_OK;
 }
 
@@ -1231,17 +1277,11 @@ int ritz_bounds(ovl_ctx *c, double *lmin, double *lmax);
 int zolo_overlap(ovl_ctx *c, const Geom &g, const void *in, void *out, double lmin, double lmax, int axpy, double dt)
 {
     if (lmin == 0.0 && lmax == 0.0) RETCHK(ritz_bounds(c, &lmin, &lmax));
-    if (!(lmin > 0.0) || !(lmax > lmin) || !std::isfinite(lmax))
-        return fail(c, OVL_E_SPECTRUM, "Zolotarev interval needs 0 < lmin < lmax");
+    RETCHK(check_interval(c, lmin, lmax));
     RETCHK(ensure_stencil(c));
-    const int no = 25;
-    double bz[25], dz[25];
-    ovl_zolotarev_coefficients(lmin, lmax, 1e-12, no, bz, dz);
-    const size_t fb = (size_t)g.nblk * c->blk64_elems * 16;
-    RETCHK(dalloc(c, &c->ms_chi, (size_t)c->g.nblk * c->blk64_elems * 16));
-    int mx = 0, nc = 0;
-    RETCHK(mscg(c, g, in, c->ms_chi, bz, dz, no, 1e-16, 1000, &mx, &nc));
-    (void)fb;
+    RETCHK(dalloc(c, &c->ms_chi, (size_t)g.nblk * c->blk64_elems * 16));
+    int nc = 0;
+    RETCHK(mscg(c, g, in, c->ms_chi, zolotarev_shifts(lmin, lmax), &nc));
     // psi = -i h_W chi, combined as OverlapU.cpp:188-201
     const double M = c->prm.m_dw, m = c->prm.m_fermion, s = axpy ? dt : 1.0;
     HopArgs a = hop_args(c, P64);
@@ -1257,8 +1297,7 @@ int zolo_overlap(ovl_ctx *c, const Geom &g, const void *in, void *out, double lm
         a.st_r = 1.0;
     }
     RETCHK(hop(c, g, P64, P64, a));
-    if (nc) return fail(c, OVL_E_CONVERGE, "multi-shift CG reached 1000 iterations for " + std::to_string(nc) + " mode(s)");
-    return OVL_OK;
+    return cg_result(c, nc);
 }
 
 }  // namespace
@@ -1614,8 +1653,9 @@ int ovl_destroy(ovl_ctx *c)
     if (c->st) hipStreamSynchronize(c->st);
     void *ps[] = {c->links, c->efield, c->ul64, c->ul32, c->phase, c->field[0], c->field[1], c->field[2], c->w64, c->a64,
                   c->b64, c->x32, c->w32, c->a32, c->b32, c->partial, c->dout, c->gam, c->jv, c->ja, c->staging,
-                  c->ms_ps, c->ms_r, c->ms_q, c->ms_w, c->ms_chi, c->ms_coef, c->ms_active, c->rz[0], c->rz[1],
-                  c->rz[2], c->rz[3], c->rz[4], c->rz[5], c->d_sys, c->d_work, c->d_qwork, c->d_qoff, c->d_qctr,
+                  c->ms_ps, c->ms_r, c->ms_q, c->ms_w, c->ms_chi, c->ms_coef, c->ms_modes, c->ms_active[0],
+                  c->ms_active[1], c->s1_links, c->s1_vec, c->s1_cg, c->s1_ritz, c->s1_start, c->s1_part,
+                  c->s1_state, c->d_sys, c->d_work, c->d_qwork, c->d_qoff, c->d_qctr,
                   c->order[0], c->order[1],
                   c->order[2], c->order[3], c->x16, c->w16, c->a16, c->b16, c->x48, c->w48, c->a48, c->b48,
                   c->f32[0], c->f32[1], c->guard_buf[0], c->guard_buf[1]};
@@ -1992,39 +2032,39 @@ int ovl_sign_residual(ovl_ctx *c, int in, const ovl_sign_opts *o, double *rel)
     return OVL_OK;
 }
 
-// ---- single-mode drop-ins on the first mode block of the scratch field ----
+// ---- single-mode drop-ins: one vector in the layout of the single-vector kernels ----
+// (in a mode-block field the one mode would drag the other 15 lanes of its block through every load)
+// u_cc and phi from host arrays to c->s1_links and the first vector of c->s1_vec
 static int dropin_setup(ovl_ctx *c, const double *ucc, const double *phi)
 {
     if (!ucc || !phi) return fail(c, OVL_E_ARG, "null argument");
     RETCHK(single_lattice(c, "the single-mode drop-ins"));
     const size_t nu = (size_t)3 * c->g.V * c->g.nc * c->g.nc * 2, np = (size_t)c->g.V * c->ncomp * 2;
-    // the inputs are checked for Inf/NaN on the device after the upload (a host scan of the 8.6 MB
-    // of a 24^3 SU(3) call costs about as long as the copy itself)
-    bool ok = true;
-    RETCHK(stage(c, std::max(nu, np) * sizeof(double)));
+    RETCHK(stage(c, (nu + np) * sizeof(double)));
+    RETCHK(ensure_single(c));
+    RETCHK(dalloc(c, &c->s1_vec, 2 * vec1_bytes(c)));
+    int *flags = single_flags(c), bad[2] = {0, 0};
+    // the inputs are checked for Inf/NaN by the kernels that lay them out (a host scan of the 8.6 MB of a
+    // 24^3 SU(3) call costs about as long as the copy itself)
+    HIPCHK(c, hipMemsetAsync(flags, 0, sizeof bad, c->st));
     HIPCHK(c, hipMemcpyAsync(c->staging, ucc, nu * sizeof(double), hipMemcpyHostToDevice, c->st));
-    RETCHK(device_finite(c, c->staging, nullptr, (long)nu, &ok));
-    if (!ok) return fail(c, OVL_E_ARG, "non-finite input (u_cc)");
-    HIPCHK(c, ovl::launch_ucc_to_links(c->g, c->staging, c->ul64, c->ul32, c->st));
-    c->stencil_dirty = true;  // the next batched call re-derives the stencil from the master links
-    Geom g1 = c->g;
-    g1.nblk = 1;
-    HIPCHK(c, hipMemsetAsync(c->field[OVL_SCRATCH], 0, c->blk64_elems * 16, c->st));
+    HIPCHK(c, ovl::launch_links1(c->g, c->staging, c->s1_links, flags, c->st));
+    HIPCHK(c, hipMemcpyAsync(c->staging + nu, phi, np * sizeof(double), hipMemcpyHostToDevice, c->st));
+    HIPCHK(c, ovl::launch_vec1_in(c->g, c->staging + nu, c->s1_vec, flags + 1, c->st));
+    HIPCHK(c, hipMemcpyAsync(bad, flags, sizeof bad, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
-    HIPCHK(c, hipMemcpyAsync(c->staging, phi, np * sizeof(double), hipMemcpyHostToDevice, c->st));
-    RETCHK(device_finite(c, c->staging, nullptr, (long)np, &ok));
-    if (!ok) return fail(c, OVL_E_ARG, "non-finite input (phi)");
-    HIPCHK(c, ovl::launch_aos_to_soa(g1, c->staging, 0, 1, c->field[OVL_SCRATCH], c->st));
+    if (bad[0]) return fail(c, OVL_E_ARG, "non-finite input (u_cc)");
+    if (bad[1]) return fail(c, OVL_E_ARG, "non-finite input (phi)");
     return OVL_OK;
 }
 
-static int dropin_fetch(ovl_ctx *c, const void *field, double *psi)
+// sh h_W(in) + sx gamma0 x -> psi (host; x may be null)
+static int dropin_result(ovl_ctx *c, const void *in, double sh_i, const void *x, double sx_i, double *psi)
 {
-    Geom g1 = c->g;
-    g1.nblk = 1;
-    const size_t np = (size_t)c->g.V * c->ncomp * 2;
-    HIPCHK(c, ovl::launch_soa_to_aos(g1, field, 0, 1, c->staging, c->st));
-    HIPCHK(c, hipMemcpyAsync(psi, c->staging, np * sizeof(double), hipMemcpyDeviceToHost, c->st));
+    void *out = (char *)c->s1_vec + vec1_bytes(c);
+    HIPCHK(c, ovl::launch_hop1(c->g, amass(c), in, out, c->s1_links, 0.0, sh_i, x, 0.0, sx_i, 1, c->st));
+    HIPCHK(c, ovl::launch_vec1_out(c->g, out, c->staging, c->st));
+    HIPCHK(c, hipMemcpyAsync(psi, c->staging, vec1_bytes(c), hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
     return OVL_OK;
 }
@@ -2033,152 +2073,79 @@ int ovl_wilson_evo_compute(ovl_ctx *c, const double *ucc, const double *phi, dou
 {
     if (!c || !psi) return OVL_E_ARG;
     RETCHK(dropin_setup(c, ucc, phi));
-    RETCHK(ensure_work(c, 1, false));
-    Geom g1 = c->g;
-    g1.nblk = 1;
-    HopArgs a = hop_args(c, P64);
-    a.nblk = 1;
-    a.in = c->field[OVL_SCRATCH];
-    a.out = c->w64;
-    a.sh_i = -1.0;
-    RETCHK(hop(c, g1, P64, P64, a));
-    return dropin_fetch(c, c->w64, psi);
+    return dropin_result(c, c->s1_vec, -1.0, nullptr, 0.0, psi);
 }
 
 int ovl_overlap_operator_compute(ovl_ctx *c, const double *ucc, const double *phi, double *psi, double lmin,
                                  double lmax)
 {
     if (!c || !psi) return OVL_E_ARG;
-    if (!(lmin > 0.0) || !(lmax > lmin)) return fail(c, OVL_E_SPECTRUM, "Zolotarev interval needs 0 < lmin < lmax");
+    RETCHK(check_interval(c, lmin, lmax));
     RETCHK(dropin_setup(c, ucc, phi));
-    RETCHK(ensure_work(c, 1, false));
-    Geom g1 = c->g;
-    g1.nblk = 1;
-    // zolo_overlap's ensure_stencil() must not overwrite the uploaded u_cc links
-    const bool saved_set = c->links_set;
-    c->links_set = true;
-    c->stencil_dirty = false;
-    int r = zolo_overlap(c, g1, c->field[OVL_SCRATCH], c->w64, lmin, lmax, 0, 0.0);
-    c->links_set = saved_set;
-    c->stencil_dirty = true;
-    if (r != OVL_OK && r != OVL_E_CONVERGE) return r;
-    RETCHK(dropin_fetch(c, c->w64, psi));
-    return r;
+    void *chi = nullptr;
+    int nc = 0;
+    RETCHK(mscg1(c, c->s1_vec, zolotarev_shifts(lmin, lmax), &chi, &nc));
+    // psi = -i h_W chi, combined as OverlapU.cpp:188-201
+    const double M = c->prm.m_dw, m = c->prm.m_fermion;
+    RETCHK(dropin_result(c, chi, -M * (1.0 - 0.5 * m), c->s1_vec, -M * (1.0 + 0.5 * m), psi));
+    return cg_result(c, nc);
 }
 
-// ---- Ritz (RitzSolver.cpp:92-297), neigen = 1, on mode 0 of one block ----
+// ---- Ritz (RitzSolver.cpp:92-297), neigen = 1 ----
+// `solves` independent solves from the start vectors in the first Ritz vector of each (signs sign[]): they
+// advance in the same launches, so that two bounds cost the iterations of the longer one
+static int ritz_solve(ovl_ctx *c, int solves, const double *sign, double delitr, int nitlz, int nrestart, double *eig)
+{
+    if (nrestart < 1) return fail(c, OVL_E_ARG, "Ritz needs at least one iteration per restart");
+    ovl::RitzCall k{};
+    k.vec = c->s1_ritz;
+    k.state = c->s1_state;
+    k.part = c->s1_part;
+    k.links = c->s1_links;
+    k.amass = amass(c);
+    k.solves = solves;
+    for (int q = 0; q < solves; ++q) k.sign[q] = sign[q];
+    k.delitr = delitr;
+    k.nitlz = nitlz;
+    HIPCHK(c, ovl::launch_links1(c->g, c->ul64, c->s1_links, nullptr, c->st));
+    std::vector<ovl::RitzState> h((size_t)2 * solves);
+    HIPCHK(c, hipMemsetAsync(c->s1_state, 0, sizeof(ovl::RitzState) * h.size(), c->st));
+    HIPCHK(c, ovl::launch_ritz_start(c->g, k, c->st));
+    // an iteration is five short launches; once all solves are done they return at once
+    constexpr int batch = 16;
+    for (int it = 0;; ++it) {
+        if (it > 0 && it % batch == 0) {
+            HIPCHK(c, hipMemcpyAsync(h.data(), c->s1_state, sizeof(ovl::RitzState) * h.size(), hipMemcpyDeviceToHost, c->st));
+            HIPCHK(c, hipStreamSynchronize(c->st));
+            bool all = true;
+            for (int q = 0; q < solves; ++q) all = all && h[2 * q + (it & 1)].done;
+            if (all) {
+                for (int q = 0; q < solves; ++q) eig[q] = h[2 * q + (it & 1)].xy_r;
+                return OVL_OK;
+            }
+        }
+        HIPCHK(c, ovl::launch_ritz_iteration(c->g, k, it, it % nrestart == 0, c->st));
+        c->hop_launches += 2;
+    }
+}
+
+static int ritz_buffers(ovl_ctx *c)
+{
+    RETCHK(ensure_stencil(c));
+    RETCHK(ensure_single(c));
+    return dalloc(c, &c->s1_ritz, vec1_bytes(c) * ovl::RITZ_VECS * ovl::RITZ_SOLVES);
+}
+
 int ovl_ritz(ovl_ctx *c, const double *start_flat, double sign, double delitr, int nitlz, int nrestart,
              double *eigenvalue)
 {
     if (!c || !start_flat || !eigenvalue) return OVL_E_ARG;
     RETCHK(single_lattice(c, "ovl_ritz"));
-    RETCHK(ensure_stencil(c));
-    Geom g = c->g;
-    g.nblk = 1;
-    const size_t fb = c->blk64_elems * 16;
-    for (int i = 0; i < 6; ++i) RETCHK(dalloc(c, &c->rz[i], fb));
-    void *xr = c->rz[0], *yr = c->rz[1], *zr = c->rz[2], *gr = c->rz[3], *pr = c->rz[4], *w = c->rz[5];
-    // flat (m = s + V(spin + 4 colour)) -> AoS -> SoA mode 0
-    const int V = c->g.V, nc = c->g.nc;
-    std::vector<double> aos((size_t)V * c->ncomp * 2);
-    for (int s = 0; s < V; ++s)
-        for (int k = 0; k < 4; ++k)
-            for (int j = 0; j < nc; ++j) {
-                const size_t m = s + (size_t)V * (k + 4 * j);
-                aos[2 * ((s * nc + j) * 4 + k)] = start_flat[2 * m];
-                aos[2 * ((s * nc + j) * 4 + k) + 1] = start_flat[2 * m + 1];
-            }
-    RETCHK(stage(c, aos.size() * sizeof(double)));
-    for (void *v : {xr, yr, zr, gr, pr, w}) HIPCHK(c, hipMemsetAsync(v, 0, fb, c->st));
-    HIPCHK(c, hipMemcpyAsync(c->staging, aos.data(), aos.size() * sizeof(double), hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, ovl::launch_aos_to_soa(g, c->staging, 0, 1, xr, c->st));
-    auto dot = [&](const void *a, const void *b, cplx &res) -> int {
-        std::vector<cplx> d;
-        RETCHK(mode_dot(c, g, a, b, d));
-        res = d[0];
-        return OVL_OK;
-    };
-    auto lin = [&](void *out, const void *a, cplx ca, const void *b, cplx cb) -> int {
-        HIPCHK(c, ovl::launch_lincomb(g, 1, P64, out, a, ca.real(), ca.imag(), b, cb.real(), cb.imag(), c->st));
-        return OVL_OK;
-    };
-    auto uu = [&](const void *v, void *out) -> int {  // out = sign * h^2 v
-        RETCHK(apply_h2(c, g, v, w, out, 0.0));
-        return lin(out, out, sign, nullptr, 0.0);
-    };
-    cplx t;
-    RETCHK(dot(xr, xr, t));
-    double xnorm = 1.0 / std::sqrt(t.real());
-    RETCHK(lin(xr, xr, xnorm, nullptr, 0.0));
-    int ittot = 0;
-    bool done = false;
-    cplx xynorm = 0, oxynorm = 0, xpnorm = 0, amb = 0;
-    double gnorm = 0, gnormim = 0, pnorm = 0;
-    while (!done) {
-        RETCHK(uu(xr, yr));
-        RETCHK(dot(xr, yr, xynorm));
-        RETCHK(lin(gr, yr, 1.0, xr, -xynorm));
-        RETCHK(lin(pr, gr, 1.0, nullptr, 0.0));
-        RETCHK(dot(gr, gr, t));
-        gnormim = t.real();
-        pnorm = std::sqrt(gnormim);
-        RETCHK(lin(pr, pr, 1.0 / pnorm, nullptr, 0.0));
-        for (int itt = 1; itt <= nrestart; ++itt) {
-            ittot++;
-            RETCHK(uu(pr, zr));
-            amb = xynorm;
-            RETCHK(dot(pr, zr, t));
-            amb -= t.real();
-            RETCHK(dot(xr, zr, t));
-            const double ccc = t.real();
-            const double cox = 2.0 * ccc / amb.real();
-            const double sig1 = -std::copysign(1.0, amb.real());
-            const double sig2 = std::copysign(1.0, cox) * sig1;
-            const double cox2 = cox * cox;
-            double ct, stt;
-            if (cox2 <= 1.0e-3) {
-                // series of RitzSolver.cpp:199-200
-                const double sqp = 1.0 - 0.125 * cox2 + 0.0859375 * cox2 * cox2 - 0.0673828125 * cox2 * cox2 * cox2 +
-                                   0.0562439 * cox2 * cox2 * cox2 * cox2 + 0.0487 * cox2 * cox2 * cox2 * cox2 * cox2;
-                const double sqm = 0.5 * sig1 * sig2 * cox *
-                                   (1.0 - 0.375 * cox2 + 0.2421875 * cox2 * cox2 - 0.182617875 * cox2 * cox2 * cox2 +
-                                    0.1482849 * cox2 * cox2 * cox2 * cox2 - 0.12575 * cox2 * cox2 * cox2 * cox2 * cox2 +
-                                    0.1097 * cox2 * cox2 * cox2 * cox2 * cox2 * cox2);
-                if (sig1 < 0.0) { ct = sqm; stt = sig2 * sqp; }
-                else { ct = sqp; stt = sig2 * sqm; }
-            } else {
-                const double sox = sig1 / std::sqrt(1.0 + cox2);
-                ct = std::sqrt((1.0 + sox) * 0.5);
-                stt = std::sqrt((1.0 - sox) * 0.5) * sig2;
-            }
-            RETCHK(lin(xr, xr, ct, pr, stt));
-            RETCHK(lin(yr, yr, ct, zr, stt));
-            RETCHK(dot(xr, xr, t));
-            xnorm = t.real();
-            oxynorm = xynorm;
-            RETCHK(dot(xr, yr, xynorm));
-            xnorm = 1.0 / std::sqrt(xnorm);
-            xynorm *= xnorm;
-            RETCHK(lin(xr, xr, xnorm, nullptr, 0.0));
-            RETCHK(lin(gr, yr, 1.0, xr, -xynorm));
-            RETCHK(dot(gr, gr, t));
-            gnorm = t.real();
-            RETCHK(dot(xr, pr, xpnorm));
-            if (xynorm.real() > oxynorm.real()) { done = true; break; }
-            if (gnorm < delitr * sign * xynorm.real()) { done = true; break; }
-            const double beta = gnorm / gnormim * pnorm;
-            // pr = gr + beta (pr - xr xpnorm)
-            RETCHK(lin(pr, pr, beta, xr, -beta * xpnorm));
-            RETCHK(lin(pr, pr, 1.0, gr, 1.0));
-            RETCHK(dot(pr, pr, t));
-            pnorm = std::sqrt(t.real());
-            RETCHK(lin(pr, pr, 1.0 / pnorm, nullptr, 0.0));
-            gnormim = gnorm;
-            if (ittot >= nitlz) { done = true; break; }
-        }
-    }
-    *eigenvalue = xynorm.real();
-    return OVL_OK;
+    RETCHK(ritz_buffers(c));
+    RETCHK(stage(c, vec1_bytes(c)));
+    HIPCHK(c, hipMemcpyAsync(c->staging, start_flat, vec1_bytes(c), hipMemcpyHostToDevice, c->st));
+    HIPCHK(c, ovl::launch_vec1_flat(c->g, c->staging, c->s1_ritz, c->st));
+    return ritz_solve(c, 1, &sign, delitr, nitlz, nrestart, eigenvalue);
 }
 
 }  // extern "C"
@@ -2189,22 +2156,32 @@ namespace {
 // fixed-seed 64-bit Mersenne twister instead of the reference's GSL stream
 int ritz_bounds(ovl_ctx *c, double *lmin, double *lmax)
 {
-    const size_t n = (size_t)c->g.V * c->ncomp;
-    std::vector<double> v(2 * n);
-    unsigned long long st = 0x9E3779B97F4A7C15ull;
-    double nrm = 0;
-    for (size_t i = 0; i < 2 * n; ++i) {
-        st ^= st << 13; st ^= st >> 7; st ^= st << 17;  // xorshift64
-        v[i] = (double)(st >> 11) * (1.0 / 9007199254740992.0);
-        nrm += v[i] * v[i];
+    RETCHK(ritz_buffers(c));
+    const size_t fb = vec1_bytes(c);
+    if (!c->s1_start) {
+        std::vector<double> v(fb / sizeof(double));
+        unsigned long long st = 0x9E3779B97F4A7C15ull;
+        double nrm = 0;
+        for (auto &x : v) {
+            st ^= st << 13; st ^= st >> 7; st ^= st << 17;  // xorshift64
+            x = (double)(st >> 11) * (1.0 / 9007199254740992.0);
+            nrm += x * x;
+        }
+        nrm = std::sqrt(nrm);
+        for (auto &x : v) x /= nrm;
+        RETCHK(stage(c, fb));
+        HIPCHK(c, hipMemcpyAsync(c->staging, v.data(), fb, hipMemcpyHostToDevice, c->st));
+        HIPCHK(c, hipStreamSynchronize(c->st));
+        RETCHK(dalloc(c, &c->s1_start, fb));
+        HIPCHK(c, ovl::launch_vec1_flat(c->g, c->staging, c->s1_start, c->st));
     }
-    nrm = std::sqrt(nrm);
-    for (auto &x : v) x /= nrm;
-    double a = 0, b = 0;
-    RETCHK(ovl_ritz(c, v.data(), -1.0, 1e-16, 2000, 100, &a));
-    RETCHK(ovl_ritz(c, v.data(), 1.0, 1e-16, 2000, 100, &b));
-    *lmax = -1.05 * a;
-    *lmin = 0.95 * b;
+    for (int q = 0; q < 2; ++q)
+        HIPCHK(c, hipMemcpyAsync((char *)c->s1_ritz + q * ovl::RITZ_VECS * fb, c->s1_start, fb, hipMemcpyDeviceToDevice, c->st));
+    const double sign[2] = {-1.0, 1.0};
+    double eig[2] = {0, 0};
+    RETCHK(ritz_solve(c, 2, sign, 1e-16, 2000, 100, eig));
+    *lmax = -1.05 * eig[0];
+    *lmin = 0.95 * eig[1];
     return OVL_OK;
 }
 }  // namespace

@@ -153,11 +153,77 @@ size_t reduce_partial_len(const Geom &g);
 hipError_t launch_currents(const Geom &g, const void *psi, const void *hpsi, const double *gam, int first_mode,
                            double *partial, double *jv, double *ja, hipStream_t st);
 size_t currents_partial_len(const Geom &g);
-// multi-shift CG helpers (FP64 fields)
+// partial sums per (chunk, mode) of launch_mode_dot, before its fixed-order sum over the chunks
+hipError_t launch_mode_dot_partial(const Geom &g, const void *a, const void *b, double *partial, hipStream_t st);
+int mode_dot_chunks();
+
+// ---- Krylov solvers with device-resident scalars (ovl_solvers.hip) ----
+// number of poles of the Zolotarev sign (OverlapOperator.cpp:25-64)
+constexpr int CG_SHIFTS = 25;
+struct CgShifts {
+    double bz[CG_SHIFTS], dz[CG_SHIFTS];
+};
+// scalar state of one mode's multi-shift CG
+struct CgMode {
+    double rn, bn, a0, betam, alpha;
+    int it, act;
+    double z[CG_SHIFTS], gc[CG_SHIFTS];
+};
+// p_k, chi of every shift and mode from per-mode coefficients {bz beta, alpha, zeta} (FP64 fields)
 hipError_t launch_mscg_update(const Geom &g, int nshift, double *ps, double *chi, const double *r,
                               const double *coef, const int *active, hipStream_t st);
-hipError_t launch_axpy_modes(const Geom &g, void *y, const void *x, const double *coef, int coef_stride,
-                             double sign, const int *active, hipStream_t st);
+// one multi-shift CG iteration of many modes: hop, hop, launch_mode_dot_partial, alpha, residual (with
+// its partial |r|^2), scalars, launch_mscg_update
+hipError_t launch_cgm_begin(const Geom &g, const double *part, int chunks, CgMode *modes, int *act, double tol, hipStream_t st);
+hipError_t launch_cgm_alpha(const Geom &g, const double *part, int chunks, CgMode *modes, const int *act, hipStream_t st);
+hipError_t launch_cgm_residual(const Geom &g, void *r, const void *q, const CgMode *modes, const int *act, double *part,
+                               int chunks, hipStream_t st);
+hipError_t launch_cgm_scalars(const Geom &g, const double *part, int chunks, CgMode *modes, const int *act, int *act_next,
+                              double *coef, const CgShifts &sh, double tol, int cap, hipStream_t st);
+
+// One FP64 vector in the layout [spin][colour][site] with links [mu][i][j][site] (Geom: nc, n0..n2, V).
+// `bad` (device int, may be null) is set to 1 when an input entry is Inf or NaN.
+hipError_t launch_links1(const Geom &g, const void *links, void *out, int *bad, hipStream_t st);
+hipError_t launch_vec1_in(const Geom &g, const double *aos, void *out, int *bad, hipStream_t st);
+hipError_t launch_vec1_out(const Geom &g, const void *f, double *aos, hipStream_t st);
+hipError_t launch_vec1_flat(const Geom &g, const double *flat, void *out, hipStream_t st);
+// out = sh h_W(in) + sx G(x) (x may be null)
+hipError_t launch_hop1(const Geom &g, double amass, const void *in, void *out, const void *links, double sh_r, double sh_i,
+                       const void *x, double sx_r, double sx_i, int x_gamma0, hipStream_t st);
+size_t single_partial_len(const Geom &g);  // doubles of `part` below
+
+// Ritz: up to RITZ_SOLVES independent solves (signs sign[0..solves)) advance in the same launches.  `vec`:
+// RITZ_VECS vectors per solve, the first one the start vector; `state`: 2 RitzState per solve, zeroed;
+// iteration `iter` counts from 0, `restart` before the first and after every nrestart iterations.  The
+// result of iteration i is state[2 solve + (i + 1) % 2].
+constexpr int RITZ_VECS = 6, RITZ_SOLVES = 2, RITZ_PARTS = 5;
+struct RitzState {
+    double xy_r, xy_i, xyn_r, xyn_i, gnormim;
+    int iters, done, fresh, pad;
+};
+struct RitzCall {
+    void *vec, *state;
+    double *part;
+    const void *links;
+    double amass, sign[RITZ_SOLVES], delitr;
+    int solves, nitlz;
+};
+hipError_t launch_ritz_start(const Geom &g, const RitzCall &c, hipStream_t st);
+hipError_t launch_ritz_iteration(const Geom &g, const RitzCall &c, int iter, bool restart, hipStream_t st);
+
+// multi-shift CG of one vector: `work` holds CG_SHIFTS + 4 vectors, `state` 2 CgMode; the state after
+// iteration `iter` (from 0) is state[(iter + 1) % 2], the solution cg1_chi(work)
+struct Cg1Call {
+    void *work, *state;
+    double *part;
+    const void *in, *links;
+    double amass, tol;
+    CgShifts sh;
+    int cap;
+};
+hipError_t launch_cg1_start(const Geom &g, const Cg1Call &c, hipStream_t st);
+hipError_t launch_cg1_iteration(const Geom &g, const Cg1Call &c, int iter, hipStream_t st);
+void *cg1_chi(const Geom &g, void *work);
 
 // QED eigenbasis (FP64 fields): unit sources of one batch into a zeroed field (mode mm < cnt:
 // source k0 + mm, colour 0 of the z = 0 plane below dz = 4 n0 n1, colour 1 of site 0 above);

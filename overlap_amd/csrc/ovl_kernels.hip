@@ -1475,14 +1475,20 @@ __global__ __launch_bounds__(TPB) void k_mode_dot(const double2 *__restrict__ a,
     }
 }
 
-__global__ __launch_bounds__(TPB) void k_mode_dot_finish(const double2 *__restrict__ partial, double2 *__restrict__ out,
-                                                         int nmodes_pad)
+// sum over the chunks, one wavefront per mode (two partial results per lane, then the wave's tree)
+__global__ __launch_bounds__(64) void k_mode_dot_finish(const double2 *__restrict__ partial, double2 *__restrict__ out,
+                                                        int nmodes_pad)
 {
-    const int i = blockIdx.x * TPB + threadIdx.x;
-    if (i >= nmodes_pad) return;
+    const int i = blockIdx.x;
     double r = 0, im = 0;
-    for (int c = 0; c < DOT_CHUNKS; ++c) { r += partial[(size_t)c * nmodes_pad + i].x; im += partial[(size_t)c * nmodes_pad + i].y; }
-    out[i] = make_double2(r, im);
+    for (int c = threadIdx.x; c < DOT_CHUNKS; c += 64) {
+        const double2 p = partial[(size_t)c * nmodes_pad + i];
+        r += p.x;
+        im += p.y;
+    }
+    r = wave_sum(r);
+    im = wave_sum(im);
+    if (threadIdx.x == 0) out[i] = make_double2(r, im);
 }
 
 // currents (OverlapCurrents.cpp:137-228), per (site, mode) bilinears summed over the modes of a block.
@@ -1570,26 +1576,6 @@ __global__ __launch_bounds__(TPB) void k_mscg_update2(int nshift, double2 *__res
         ps[(size_t)k * nel + i] = p;
     }
     chi[i] = x;
-}
-
-// y += sign * coef[mode*stride] * x for active modes (FP64 fields)
-__global__ __launch_bounds__(TPB) void k_axpy_modes(double2 *__restrict__ y, const double2 *__restrict__ x,
-                                                    const double *__restrict__ coef, int stride, double sign,
-                                                    const int *__restrict__ active, long per_blk, int nblk, int mb)
-{
-    const long i = (long)blockIdx.x * TPB + threadIdx.x;
-    const long nel = per_blk * nblk * mb;
-    if (i >= nel) return;
-    const int m = (int)(i % mb);
-    const int blk = (int)(i / ((long)per_blk * mb));
-    const int mode = blk * mb + m;
-    if (active && !active[mode]) return;
-    const double c = sign * coef[(size_t)mode * stride];
-    const double2 xv = x[i];
-    double2 yv = y[i];
-    yv.x += c * xv.x;
-    yv.y += c * xv.y;
-    y[i] = yv;
 }
 
 inline unsigned nblocks(long n) { return (unsigned)((n + TPB - 1) / TPB); }
@@ -1998,7 +1984,9 @@ hipError_t launch_efield_update(const Geom &g, const double *links, double *efie
 
 size_t mode_dot_partial_len(const Geom &g) { return (size_t)DOT_CHUNKS * g.nblk * g.mb * 2; }
 
-hipError_t launch_mode_dot(const Geom &g, const void *a, const void *b, double *partial, double *out, hipStream_t st)
+int mode_dot_chunks() { return DOT_CHUNKS; }
+
+hipError_t launch_mode_dot_partial(const Geom &g, const void *a, const void *b, double *partial, hipStream_t st)
 {
     dim3 grid(DOT_CHUNKS, g.nblk);
     const auto A = (const double2 *)a;
@@ -2011,8 +1999,15 @@ hipError_t launch_mode_dot(const Geom &g, const void *a, const void *b, double *
         if (g.mb == 16) DOT(3, 16); else if (g.mb == 32) DOT(3, 32); else DOT(3, 64);
     }
 #undef DOT
+    return hipGetLastError();
+}
+
+hipError_t launch_mode_dot(const Geom &g, const void *a, const void *b, double *partial, double *out, hipStream_t st)
+{
+    const hipError_t e = launch_mode_dot_partial(g, a, b, partial, st);
+    if (e != hipSuccess) return e;
     const int np = g.nblk * g.mb;
-    k_mode_dot_finish<<<nblocks(np), TPB, 0, st>>>(P, (double2 *)out, np);
+    k_mode_dot_finish<<<np, 64, 0, st>>>((const double2 *)partial, (double2 *)out, np);
     return hipGetLastError();
 }
 
@@ -2088,16 +2083,6 @@ hipError_t launch_mscg_update(const Geom &g, int nshift, double *ps, double *chi
     const long nel = per_blk * g.nblk * g.mb;
     k_mscg_update2<<<nblocks(nel), TPB, 0, st>>>(nshift, (double2 *)ps, (double2 *)chi, (const double2 *)r, coef, active,
                                                  per_blk, g.nblk, g.mb);
-    return hipGetLastError();
-}
-
-hipError_t launch_axpy_modes(const Geom &g, void *y, const void *x, const double *coef, int coef_stride, double sign,
-                             const int *active, hipStream_t st)
-{
-    const long per_blk = (long)g.V * 4 * g.nc;
-    const long nel = per_blk * g.nblk * g.mb;
-    k_axpy_modes<<<nblocks(nel), TPB, 0, st>>>((double2 *)y, (const double2 *)x, coef, coef_stride, sign, active, per_blk,
-                                               g.nblk, g.mb);
     return hipGetLastError();
 }
 
