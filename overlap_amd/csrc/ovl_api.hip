@@ -2195,7 +2195,7 @@ int ovl_update_links(ovl_ctx *c, double dt)
     if (!c->links_set) return fail(c, OVL_E_STATE, "no gauge links uploaded");
     for (int s = 0; s < nsys(c); ++s)
         HIPCHK(c, ovl::launch_link_update(sys_geom(c, s), sys_links(c, s), sys_efield(c, s), dt, c->prm.reunitarize,
-                                          c->st));
+                                          nullptr, nullptr, nullptr, c->st));
     c->stencil_dirty = true;
     HIPCHK(c, hipStreamSynchronize(c->st));
     return OVL_OK;
@@ -2218,8 +2218,8 @@ static int gauge_half(ovl_ctx *c, int mode, double h)
         const Geom g = sys_geom(c, s);
         if (mode == OVL_GAUGE_FULL)
             HIPCHK(c, ovl::launch_efield_update(g, sys_links(c, s), sys_efield(c, s), h, c->st));
-        HIPCHK(c, ovl::launch_link_update(g, sys_links(c, s), sys_efield(c, s), h, c->prm.reunitarize, c->st));
-        HIPCHK(c, ovl::launch_link_setup(g, sys_links(c, s), sys_phase(c, s), sys_ul64(c, s), sys_ul32(c, s), c->st));
+        HIPCHK(c, ovl::launch_link_update(g, sys_links(c, s), sys_efield(c, s), h, c->prm.reunitarize, sys_phase(c, s),
+                                          sys_ul64(c, s), sys_ul32(c, s), c->st));
     }
     return OVL_OK;
 }
@@ -2493,47 +2493,30 @@ static int fetch_out(ovl_ctx *c, double *h, int n)
     return OVL_OK;
 }
 
-static int obs_energy(ovl_ctx *c, int s, double *e_el, double *e_mag)
+// the raw observables `what` (ovl::OBS_*) of system s, one synchronisation
+static int obs_raw(ovl_ctx *c, int s, int what, double *raw)
 {
     if (!c->sys_links_set[s]) return fail(c, OVL_E_STATE, "no gauge links uploaded");
-    HIPCHK(c, ovl::launch_energy(sys_geom(c, s), sys_links(c, s), sys_efield(c, s), c->partial, c->dout, c->st));
-    double h[2];
-    RETCHK(fetch_out(c, h, 2));
-    *e_el = h[0];
-    *e_mag = h[1];
-    return OVL_OK;
+    HIPCHK(c, ovl::launch_observables(sys_geom(c, s), sys_links(c, s), sys_efield(c, s), what, nullptr, c->partial,
+                                      c->dout, c->st));
+    return fetch_out(c, raw, ovl::OBS_RAW);
 }
 
-static int obs_gauss(ovl_ctx *c, int s, double *vmax, double *vrms)
+static double gauss_rms(const ovl_ctx *c, int s, const double *raw)
 {
-    if (!c->sys_links_set[s]) return fail(c, OVL_E_STATE, "no gauge links uploaded");
-    HIPCHK(c, ovl::launch_gauss(sys_geom(c, s), sys_links(c, s), sys_efield(c, s), c->partial, c->dout, nullptr,
-                                c->st));
-    double h[2];
-    RETCHK(fetch_out(c, h, 2));
-    *vmax = h[0];
-    *vrms = std::sqrt(h[1] / (n_adj(c) * (double)c->sys[s].V));
-    return OVL_OK;
+    return std::sqrt(raw[ovl::RAW_GSUM] / (n_adj(c) * (double)c->sys[s].V));
 }
-
-static int obs_unitarity(ovl_ctx *c, int s, double *vmax, double *vrms)
+static double unitarity_rms(const ovl_ctx *c, int s, const double *raw)
 {
-    if (!c->sys_links_set[s]) return fail(c, OVL_E_STATE, "no gauge links uploaded");
-    HIPCHK(c, ovl::launch_unitarity(sys_geom(c, s), sys_links(c, s), c->partial, c->dout, c->st));
-    double h[2];
-    RETCHK(fetch_out(c, h, 2));
-    *vmax = h[0];
-    *vrms = std::sqrt(h[1] / (3.0 * c->sys[s].V));
-    return OVL_OK;
+    return std::sqrt(raw[ovl::RAW_USUM] / (3.0 * c->sys[s].V));
 }
+static double ncs_dot_of(const double *raw) { return 0.125 * raw[ovl::RAW_EDOTB] / (M_PI * M_PI); }  // ChernSimonsDerivative.cpp:47
 
 static int obs_ncs_dot(ovl_ctx *c, int s, double *ncsdot)
 {
-    if (!c->sys_links_set[s]) return fail(c, OVL_E_STATE, "no gauge links uploaded");
-    HIPCHK(c, ovl::launch_edotb(sys_geom(c, s), sys_links(c, s), sys_efield(c, s), c->partial, c->dout, c->st));
-    double h[1];
-    RETCHK(fetch_out(c, h, 1));
-    *ncsdot = 0.125 * h[0] / (M_PI * M_PI);  // ChernSimonsDerivative.cpp:47
+    double h[ovl::OBS_RAW];
+    RETCHK(obs_raw(c, s, ovl::OBS_EDOTB, h));
+    *ncsdot = ncs_dot_of(h);
     return OVL_OK;
 }
 
@@ -2541,21 +2524,33 @@ int ovl_energy(ovl_ctx *c, double *e_el, double *e_mag)
 {
     if (!c || !e_el || !e_mag) return OVL_E_ARG;
     RETCHK(single_lattice(c, "ovl_energy"));
-    return obs_energy(c, 0, e_el, e_mag);
+    double h[ovl::OBS_RAW];
+    RETCHK(obs_raw(c, 0, ovl::OBS_LOCAL, h));
+    *e_el = h[ovl::RAW_EEL];
+    *e_mag = h[ovl::RAW_EMAG];
+    return OVL_OK;
 }
 
 int ovl_gauss_violation(ovl_ctx *c, double *vmax, double *vrms)
 {
     if (!c || !vmax || !vrms) return OVL_E_ARG;
     RETCHK(single_lattice(c, "ovl_gauss_violation"));
-    return obs_gauss(c, 0, vmax, vrms);
+    double h[ovl::OBS_RAW];
+    RETCHK(obs_raw(c, 0, ovl::OBS_GAUSS, h));
+    *vmax = h[ovl::RAW_GMAX];
+    *vrms = gauss_rms(c, 0, h);
+    return OVL_OK;
 }
 
 int ovl_unitarity_violation(ovl_ctx *c, double *vmax, double *vrms)
 {
     if (!c || !vmax || !vrms) return OVL_E_ARG;
     RETCHK(single_lattice(c, "ovl_unitarity_violation"));
-    return obs_unitarity(c, 0, vmax, vrms);
+    double h[ovl::OBS_RAW];
+    RETCHK(obs_raw(c, 0, ovl::OBS_LOCAL, h));
+    *vmax = h[ovl::RAW_UMAX];
+    *vrms = unitarity_rms(c, 0, h);
+    return OVL_OK;
 }
 
 int ovl_ncs_dot(ovl_ctx *c, double *ncsdot)
@@ -2569,10 +2564,16 @@ int ovl_system_observables(ovl_ctx *c, int sys, double *obs)
 {
     if (!c || !obs) return OVL_E_ARG;
     RETCHK(check_sys(c, sys));
-    RETCHK(obs_energy(c, sys, &obs[OVL_OBS_E_EL], &obs[OVL_OBS_E_MAG]));
-    RETCHK(obs_gauss(c, sys, &obs[OVL_OBS_GAUSS_MAX], &obs[OVL_OBS_GAUSS_RMS]));
-    RETCHK(obs_unitarity(c, sys, &obs[OVL_OBS_UNIT_MAX], &obs[OVL_OBS_UNIT_RMS]));
-    return obs_ncs_dot(c, sys, &obs[OVL_OBS_NCS_DOT]);
+    double h[ovl::OBS_RAW];
+    RETCHK(obs_raw(c, sys, ovl::OBS_LOCAL | ovl::OBS_EDOTB, h));
+    obs[OVL_OBS_E_EL] = h[ovl::RAW_EEL];
+    obs[OVL_OBS_E_MAG] = h[ovl::RAW_EMAG];
+    obs[OVL_OBS_GAUSS_MAX] = h[ovl::RAW_GMAX];
+    obs[OVL_OBS_GAUSS_RMS] = gauss_rms(c, sys, h);
+    obs[OVL_OBS_UNIT_MAX] = h[ovl::RAW_UMAX];
+    obs[OVL_OBS_UNIT_RMS] = unitarity_rms(c, sys, h);
+    obs[OVL_OBS_NCS_DOT] = ncs_dot_of(h);
+    return OVL_OK;
 }
 
 // ---- allocation-free observables ----
@@ -2651,10 +2652,7 @@ int ovl_observables_noalloc(int nc, const int *n, const double *links, const dou
     RETCHK(noalloc_scratch(&s));
     double *raw = s + NOALLOC_RAW;
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    hipError_t e = ovl::launch_energy(g, links, efield, s, raw + 0, st);
-    if (e == hipSuccess) e = ovl::launch_gauss(g, links, efield, s, raw + 2, nullptr, st);
-    if (e == hipSuccess) e = ovl::launch_unitarity(g, links, s, raw + 4, st);
-    if (e == hipSuccess) e = ovl::launch_edotb(g, links, efield, s, raw + 6, st);
+    hipError_t e = ovl::launch_observables(g, links, efield, ovl::OBS_LOCAL | ovl::OBS_EDOTB, nullptr, s, raw, st);
     if (e == hipSuccess) {
         k_obs_noalloc_finish<<<1, 64, 0, st>>>(raw, obs, (double)(nc * nc - 1) * (double)V, 3.0 * (double)V);
         e = hipGetLastError();
@@ -2677,11 +2675,11 @@ int ovl_gauss_restore(ovl_ctx *c, int sys, double tol, int max_iter, int *iters,
     const double *L = sys_links(c, sys);
     double *E = sys_efield(c, sys);
     auto deviation = [&](double *mx) -> int {
-        HIPCHK(c, ovl::launch_gauss(g, L, E, c->partial, c->dout, gf, c->st));
+        HIPCHK(c, ovl::launch_observables(g, L, E, ovl::OBS_GAUSS, gf, c->partial, mx ? c->dout : nullptr, c->st));
         if (mx) {
-            double h[2];
-            RETCHK(fetch_out(c, h, 2));
-            *mx = h[0];
+            double h[ovl::OBS_RAW];
+            RETCHK(fetch_out(c, h, ovl::OBS_RAW));
+            *mx = h[ovl::RAW_GMAX];
         }
         return OVL_OK;
     };

@@ -128,26 +128,26 @@ hipError_t launch_soa_to_aos(const Geom &g, const void *field, int first, int co
 hipError_t launch_link_setup(const Geom &g, const double *links, const double *phase, double *ul64, float *ul32,
                              hipStream_t st);
 hipError_t launch_ucc_to_links(const Geom &g, const double *ucc, double *ul64, float *ul32, hipStream_t st);
+// links <- exp(-i dt E) links; with ul64 (and ul32, phase or null) the stencil links of the new ones too
 hipError_t launch_link_update(const Geom &g, double *links, const double *efield, double dt, int reunit,
-                              hipStream_t st);
+                              const double *phase, double *ul64, float *ul32, hipStream_t st);
 hipError_t launch_efield_update(const Geom &g, const double *links, double *efield, double dt, hipStream_t st);
 // per-mode inner products <a,b> = sum conj(a) b over one field (FP64 fields), nmodes results
 // written as (re, im) pairs to `out` (device); `partial` scratch of partial_len doubles
 hipError_t launch_mode_dot(const Geom &g, const void *a, const void *b, double *partial, double *out,
                            hipStream_t st);
 size_t mode_dot_partial_len(const Geom &g);
-// global observables, written to device `out`
-hipError_t launch_energy(const Geom &g, const double *links, const double *efield, double *partial, double *out,
-                         hipStream_t st);
-// gfield (optional): G^a(x) stored as [site][a]
-hipError_t launch_gauss(const Geom &g, const double *links, const double *efield, double *partial, double *out,
-                        double *gfield, hipStream_t st);
+// Global observables, `what` a sum of OBS_*: the raw results of those asked for go to out[OBS_RAW] (device;
+// null: none) in the order (1/2) sum E^2, magnetic energy, max |G|, sum G^2, max and sum of squares of the
+// unitarity norm, sum E.B.  gfield (optional, with OBS_GAUSS or OBS_LOCAL): G^a(x) stored as [site][a].
+constexpr int OBS_RAW = 7;
+enum { OBS_LOCAL = 1, OBS_GAUSS = 2, OBS_EDOTB = 4 };
+enum { RAW_EEL = 0, RAW_EMAG, RAW_GMAX, RAW_GSUM, RAW_UMAX, RAW_USUM, RAW_EDOTB };
+hipError_t launch_observables(const Geom &g, const double *links, const double *efield, int what, double *gfield,
+                              double *partial, double *out, hipStream_t st);
 // E_mu(x) -= gamma (G(x) - U_mu(x) G(x+mu) U_mu(x)^+) from a stored G
 hipError_t launch_gauss_restore(const Geom &g, const double *links, const double *gfield, double *efield, double gamma,
                                 hipStream_t st);
-hipError_t launch_unitarity(const Geom &g, const double *links, double *partial, double *out, hipStream_t st);
-hipError_t launch_edotb(const Geom &g, const double *links, const double *efield, double *partial, double *out,
-                        hipStream_t st);
 size_t reduce_partial_len(const Geom &g);
 // per-site currents summed over modes: jv, ja [4*site + mu] (device); psi, hpsi FP64 fields
 hipError_t launch_currents(const Geom &g, const void *psi, const void *hpsi, const double *gam, int first_mode,

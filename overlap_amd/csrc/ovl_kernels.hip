@@ -882,8 +882,8 @@ template <int NC> __device__ __forceinline__ Mat<NC> alg_to_mat(const double *al
         m.e[2] = {0.5 * alpha[0], 0.5 * alpha[1]};
     } else {  // alpha_a lambda_a / 2
         const double r3 = 0.5 / sqrt(3.0);
-        m.e[0] = {0.5 * alpha[2] + r3 * alpha[7], 0};
-        m.e[4] = {-0.5 * alpha[2] + r3 * alpha[7], 0};
+        m.e[0] = {__builtin_fma(r3, alpha[7], 0.5 * alpha[2]), 0};
+        m.e[4] = {__builtin_fma(r3, alpha[7], -0.5 * alpha[2]), 0};
         m.e[8] = {-2.0 * r3 * alpha[7], 0};
         m.e[1] = {0.5 * alpha[0], -0.5 * alpha[1]};
         m.e[3] = {0.5 * alpha[0], 0.5 * alpha[1]};
@@ -895,36 +895,77 @@ template <int NC> __device__ __forceinline__ Mat<NC> alg_to_mat(const double *al
     return m;
 }
 
-// ReTr(i t^a V) for all generators
-template <int NC> __device__ __forceinline__ void retr_it(const Mat<NC> &v, double *out)
+// ReTr(i t^a V) = retr_factor(a) * out[a] for all generators: tr(t^a V) = sum_ij t_ij V_ji, ReTr(i X) = -Im tr X
+template <int NC> __device__ __forceinline__ void retr_sums(const Mat<NC> &v, double *out)
 {
-    // tr(t^a V) = sum_ij t_ij V_ji; ReTr(i X) = -Im tr(X)
     if constexpr (NC == 2) {
         // t0: (0,1)=(1,0)=1/2 -> tr = (V10 + V01)/2
-        out[0] = -0.5 * (v.e[2].i + v.e[1].i);
+        out[0] = v.e[2].i + v.e[1].i;
         // t1: (0,1)=-i/2, (1,0)=i/2 -> tr = (-i V10 + i V01)/2 ; Im = (V01.r - V10.r)/2
-        out[1] = -0.5 * (v.e[1].r - v.e[2].r);
-        out[2] = -0.5 * (v.e[0].i - v.e[3].i);
+        out[1] = v.e[1].r - v.e[2].r;
+        out[2] = v.e[0].i - v.e[3].i;
     } else {
-        out[0] = -0.5 * (v.e[3].i + v.e[1].i);
-        out[1] = -0.5 * (v.e[1].r - v.e[3].r);
-        out[2] = -0.5 * (v.e[0].i - v.e[4].i);
-        out[3] = -0.5 * (v.e[6].i + v.e[2].i);
-        out[4] = -0.5 * (v.e[2].r - v.e[6].r);
-        out[5] = -0.5 * (v.e[7].i + v.e[5].i);
-        out[6] = -0.5 * (v.e[5].r - v.e[7].r);
-        const double r3 = 0.5 / sqrt(3.0);
-        out[7] = -r3 * (v.e[0].i + v.e[4].i - 2.0 * v.e[8].i);
+        out[0] = v.e[3].i + v.e[1].i;
+        out[1] = v.e[1].r - v.e[3].r;
+        out[2] = v.e[0].i - v.e[4].i;
+        out[3] = v.e[6].i + v.e[2].i;
+        out[4] = v.e[2].r - v.e[6].r;
+        out[5] = v.e[7].i + v.e[5].i;
+        out[6] = v.e[5].r - v.e[7].r;
+        out[7] = v.e[0].i + v.e[4].i - 2.0 * v.e[8].i;
     }
 }
-
-// exp(i c alpha^a t^a): scaling and squaring of the Taylor series (FP64)
-template <int NC> __device__ Mat<NC> iexp(double c, const double *alpha)
+__device__ __forceinline__ double retr_factor(int a) { return a == 7 ? -0.5 / sqrt(3.0) : -0.5; }
+template <int NC> __device__ __forceinline__ void retr_it(const Mat<NC> &v, double *out)
 {
-    Mat<NC> a = alg_to_mat<NC>(alpha);
+    retr_sums<NC>(v, out);
+#pragma unroll
+    for (int a = 0; a < NC * NC - 1; ++a) out[a] *= retr_factor(a);
+}
+
+// column `col` of A B from A and the column of B: the sums of mmul, each complex product with two roundings
+// per part in a fixed form (AR: the imaginary part rounds a.i b.r first, else a.r b.i), so that a link does
+// not depend on how the compiler contracts the expression around it (an FP32 evolution amplifies the
+// last bit of a link to the size of its own rounding)
+template <bool AR> __device__ __forceinline__ void mcol(const Mat<3> &a, cd *b)
+{
+    cd r[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        cd s = {0, 0};
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const cd x = a.e[i * 3 + k], y = b[k];
+            s = cadd(s, {__builtin_fma(x.r, y.r, -(x.i * y.i)),
+                         AR ? __builtin_fma(x.r, y.i, x.i * y.r) : __builtin_fma(x.i, y.r, x.r * y.i)});
+        }
+        r[i] = s;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; ++i) b[i] = r[i];
+}
+
+// the matrix whose columns the lanes 4 q .. 4 q + 2 of a wavefront hold
+__device__ __forceinline__ Mat<3> gather_columns(const cd *c)
+{
+    Mat<3> m;
+    const int base = (int)(threadIdx.x & 60);
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) m.e[i * 3 + j] = {__shfl(c[i].r, base + j, 64), __shfl(c[i].i, base + j, 64)};
+    return m;
+}
+
+// column `col` of exp(i c alpha^a t^a): scaling and squaring of the Taylor series (FP64).  The columns of
+// the Horner form are independent, so three of four lanes walk one each: a third of the 20 matrix
+// products' chain per lane, the sums of the one-lane form unchanged.
+__device__ void iexp_column(double c, const double *alpha, int col, cd *r)
+{
+    Mat<3> a = alg_to_mat<3>(alpha);
     double nrm = 0;
 #pragma unroll
-    for (int i = 0; i < NC * NC; ++i) {
+    for (int i = 0; i < 9; ++i) {
         a.e[i] = {-c * a.e[i].i, c * a.e[i].r};  // i c A
         nrm += a.e[i].r * a.e[i].r + a.e[i].i * a.e[i].i;
     }
@@ -933,30 +974,22 @@ template <int NC> __device__ Mat<NC> iexp(double c, const double *alpha)
     while (nrm > 0.25 && sq < 64) { nrm *= 0.5; ++sq; }
     const double sc = ldexp(1.0, -sq);
 #pragma unroll
-    for (int i = 0; i < NC * NC; ++i) { a.e[i].r *= sc; a.e[i].i *= sc; }
+    for (int i = 0; i < 9; ++i) { a.e[i].r *= sc; a.e[i].i *= sc; }
     // Horner: I + a(1 + a/2(1 + a/3(...)))
-    Mat<NC> r = mid<NC>();
-    for (int k = 20; k >= 1; --k) {
-        Mat<NC> t = mmul<NC>(a, r);
+    const double one[3] = {col == 0 ? 1.0 : 0.0, col == 1 ? 1.0 : 0.0, col == 2 ? 1.0 : 0.0};
+#pragma unroll
+    for (int i = 0; i < 3; ++i) r[i] = {one[i], 0.0};
+#pragma unroll
+    for (int k = 20; k >= 1; --k) {  // unrolled: 1/k are constants
+        mcol<true>(a, r);
         const double f = 1.0 / k;
-        r = mid<NC>();
 #pragma unroll
-        for (int i = 0; i < NC * NC; ++i) { r.e[i].r += f * t.e[i].r; r.e[i].i += f * t.e[i].i; }
+        for (int i = 0; i < 3; ++i) r[i] = {__builtin_fma(f, r[i].r, one[i]), f * r[i].i};
     }
-    for (int k = 0; k < sq; ++k) r = mmul<NC>(r, r);
-    return r;
-}
-
-__device__ __forceinline__ void store_link3(double *links, int s, int mu, const Mat<3> &m)
-{
-    double *u = links + 18 * (mu + 3 * s);
-#pragma unroll
-    for (int i = 0; i < 3; ++i)
-#pragma unroll
-        for (int j = 0; j < 3; ++j) {
-            u[2 * (i + 3 * j)] = m.e[i * 3 + j].r;
-            u[2 * (i + 3 * j) + 1] = m.e[i * 3 + j].i;
-        }
+    for (int k = 0; k < sq; ++k) {  // sq is the same in the four lanes of a link
+        const Mat<3> m = gather_columns(r);
+        mcol<true>(m, r);
+    }
 }
 
 // project onto SU(3): the unitary polar factor P = V (V^+ V)^{-1/2} (the U(3) matrix closest to V,
@@ -1008,8 +1041,20 @@ __device__ Mat<3> reunit3(Mat<3> x)
     return x;
 }
 
-// stencil links from master links and U(1) phases (ConvertGaugeLinks,
-// OverlapEvolutionOperator.cpp:23-51, with the QED phase folded in)
+// one entry of the stencil links (ConvertGaugeLinks, OverlapEvolutionOperator.cpp:23-51, with the QED
+// phase folded in)
+__device__ __forceinline__ void put_stencil_entry(cd ph, cd m, double2 *__restrict__ u64, float2 *__restrict__ u32, size_t k)
+{
+    const cd v = cmul(ph, m);
+    u64[k] = make_double2(v.r, v.i);
+    u32[k] = make_float2((float)v.r, (float)v.i);
+}
+__device__ __forceinline__ cd phase_of(const double2 *__restrict__ phase, int i)
+{
+    if (!phase) return {1, 0};
+    return {phase[i].x, phase[i].y};
+}
+
 template <int NC>
 __global__ __launch_bounds__(TPB) void k_link_setup(const double *__restrict__ links, const double2 *__restrict__ phase,
                                                     double2 *__restrict__ u64, float2 *__restrict__ u32, int V)
@@ -1017,15 +1062,10 @@ __global__ __launch_bounds__(TPB) void k_link_setup(const double *__restrict__ l
     const int i = blockIdx.x * TPB + threadIdx.x;
     if (i >= 3 * V) return;
     const int mu = i / V, s = i - mu * V;
-    Mat<NC> m = get_link<NC>(links, s, mu);
-    cd ph = {1, 0};
-    if (phase) ph = {phase[i].x, phase[i].y};
+    const Mat<NC> m = get_link<NC>(links, s, mu);
+    const cd ph = phase_of(phase, i);
 #pragma unroll
-    for (int k = 0; k < NC * NC; ++k) {
-        cd v = cmul(ph, m.e[k]);
-        u64[(size_t)i * NC * NC + k] = make_double2(v.r, v.i);
-        u32[(size_t)i * NC * NC + k] = make_float2((float)v.r, (float)v.i);
-    }
+    for (int k = 0; k < NC * NC; ++k) put_stencil_entry(ph, m.e[k], u64, u32, (size_t)i * NC * NC + k);
 }
 
 // stencil links from a host-layout u_cc array (already in [mu*V+s][i][j] order)
@@ -1039,18 +1079,27 @@ __global__ __launch_bounds__(TPB) void k_ucc_setup(const double2 *__restrict__ u
     u32[i] = make_float2((float)v.x, (float)v.y);
 }
 
-// Dynamics.cpp:97-138: U <- exp(i cU E) U with cU = -dt
+// Dynamics.cpp:97-138: U <- exp(i cU E) U with cU = -dt.  With u64 the new stencil links are written in the
+// same pass (the leapfrog's half step: one launch instead of two, and the links are not read again).
+// A workgroup is one wavefront, so that a small lattice spreads over the CUs.  SU(3): four lanes per
+// link, the first three a column each (iexp_column).  With a lane per link and the stencil links apart:
+// 11.1 + 4.8 us on 15 x 12 x 10 (the serial chain in 22 workgroups) and 14.1 + 7.5 us on 24^3 SU(3); now
+// 5.7 and 15.7 us (24^3: 25 MB read and written in 144-byte strides).
+constexpr int LINK_TPB = 64;
 template <int NC>
-__global__ __launch_bounds__(TPB) void k_link_update(double *__restrict__ links, const double *__restrict__ e,
-                                                     double dt, int V, int reunit)
+__global__ __launch_bounds__(LINK_TPB) void k_link_update(double *__restrict__ links, const double *__restrict__ e,
+                                                          double dt, int V, int reunit,
+                                                          const double2 *__restrict__ phase, double2 *__restrict__ u64,
+                                                          float2 *__restrict__ u32)
 {
-    const int i = blockIdx.x * TPB + threadIdx.x;
-    if (i >= 3 * V) return;
+    constexpr int LPL = NC == 2 ? 1 : 4;  // lanes per link
+    const int i = (int)(blockIdx.x * (LINK_TPB / LPL) + threadIdx.x / LPL);
+    if (i >= 3 * V) return;  // the lanes of a link leave together
     const int s = i / 3, mu = i - 3 * s;  // link (s, mu) at index mu + 3 s
     constexpr int NG = NC * NC - 1;
     double al[NG];
 #pragma unroll
-    for (int a = 0; a < NG; ++a) al[a] = e[NG * (mu + 3 * s) + a];
+    for (int a = 0; a < NG; ++a) al[a] = e[(size_t)NG * i + a];
     const double c = -dt;
     if constexpr (NC == 2) {
         // MatrixIExp (SU2/AlgebraOperations.cpp:37-55) and UU (SU2/GroupOperations.cpp:103-110)
@@ -1062,7 +1111,7 @@ __global__ __launch_bounds__(TPB) void k_link_update(double *__restrict__ links,
         } else {
             up[0] = up[1] = up[2] = 0; up[3] = 1;
         }
-        double *u = links + 4 * (mu + 3 * s);
+        double *u = links + 4 * (size_t)i;
         const double o0 = u[0], o1 = u[1], o2 = u[2], o3 = u[3];
         double n0 = up[3] * o0 + up[0] * o3 - (up[1] * o2 - up[2] * o1);
         double n1 = up[3] * o1 + up[1] * o3 + (up[0] * o2 - up[2] * o0);
@@ -1073,12 +1122,38 @@ __global__ __launch_bounds__(TPB) void k_link_update(double *__restrict__ links,
             n0 /= nn; n1 /= nn; n2 /= nn; n3 /= nn;
         }
         u[0] = n0; u[1] = n1; u[2] = n2; u[3] = n3;
+        if (u64) {
+            const int iu = mu * V + s;
+            const cd ph = phase_of(phase, iu);
+            const cd m[4] = {{n3, n2}, {n1, n0}, {-n1, n0}, {n3, -n2}};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) put_stencil_entry(ph, m[k], u64, u32, (size_t)iu * 4 + k);
+        }
     } else {
-        Mat<3> ex = iexp<3>(c, al);
-        Mat<3> u = get_link<3>(links, s, mu);
-        Mat<3> r = mmul<3>(ex, u);
-        if (reunit) r = reunit3(r);
-        store_link3(links, s, mu, r);
+        const int col = threadIdx.x % 4 < 3 ? threadIdx.x % 4 : 0;  // the fourth lane repeats the first
+        double *u = links + 18 * (size_t)i + 6 * col;
+        cd ex[3], r[3];
+        iexp_column(c, al, col, ex);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) r[k] = {u[2 * k], u[2 * k + 1]};
+        mcol<false>(gather_columns(ex), r);
+        if (reunit) {
+            const Mat<3> m = reunit3(gather_columns(r));
+#pragma unroll
+            for (int k = 0; k < 3; ++k) r[k] = col == 0 ? m.e[3 * k] : (col == 1 ? m.e[3 * k + 1] : m.e[3 * k + 2]);
+        }
+        if (threadIdx.x % 4 == 3) return;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            u[2 * k] = r[k].r;
+            u[2 * k + 1] = r[k].i;
+        }
+        if (u64) {
+            const int iu = mu * V + s;
+            const cd ph = phase_of(phase, iu);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) put_stencil_entry(ph, r[k], u64, u32, (size_t)iu * 9 + 3 * k + col);
+        }
     }
 }
 
@@ -1094,43 +1169,52 @@ __device__ __forceinline__ int nbr(int s, int dmu, int step, int n0, int n1, int
 // E_mu(x) += dt * (-2) sum_{nu != mu} [ReTr(i t^a U_{mu nu}(x)) + ReTr(i t^a U_{mu,-nu}(x))]
 // (Hamilton's equation of H = 1/2 E^2 + 2 sum ReTr(1 - U_plaq) for U' = -i E U; the
 // reference's plaquette macros used by Dynamics.cpp:145-197 are absent)
+// Four lanes per link, one plaquette each (two planes, forward and backward), their components summed
+// from the four lanes: a lane's chain is three matrix products instead of twelve (SU(3): 14.1 -> 7.3 us on
+// 15 x 12 x 10, where a lane per link left most CUs without a wave, 17.8 -> 15.3 us on 24^3, where the
+// matrices' strided loads bound it).
 template <int NC>
-__global__ __launch_bounds__(TPB) void k_efield_update(const double *__restrict__ links, double *__restrict__ e,
-                                                       double dt, int n0, int n1, int n2)
+__global__ __launch_bounds__(LINK_TPB) void k_efield_update(const double *__restrict__ links, double *__restrict__ e,
+                                                            double dt, int n0, int n1, int n2)
 {
     const int V = n0 * n1 * n2;
-    const int i = blockIdx.x * TPB + threadIdx.x;
-    if (i >= 3 * V) return;
-    const int s = i / 3, mu = i - 3 * s;
+    const int j = threadIdx.x % 4;
+    const int i = (int)(blockIdx.x * (LINK_TPB / 4) + threadIdx.x / 4);
+    const bool ok = i < 3 * V;
+    const int il = ok ? i : 3 * V - 1;
+    const int s = il / 3, mu = il - 3 * s;
     constexpr int NG = NC * NC - 1;
-    double f[NG];
-#pragma unroll
-    for (int a = 0; a < NG; ++a) f[a] = 0;
-    const Mat<NC> umu = get_link<NC>(links, s, mu);
+    const int nu = j < 2 ? (mu == 0 ? 1 : 0) : (mu == 2 ? 1 : 2);  // the two other directions, ascending
+    const bool back = j & 1;
     const int sp = nbr(s, mu, 1, n0, n1, n2);
-    for (int nu = 0; nu < 3; ++nu) {
-        if (nu == mu) continue;
-        // forward: U_mu(x) U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
-        const int snu = nbr(s, nu, 1, n0, n1, n2);
-        Mat<NC> p = mmul<NC>(umu, get_link<NC>(links, sp, nu));
-        p = mmul<NC>(p, mdag<NC>(get_link<NC>(links, snu, mu)));
+    // forward:  U_mu(x) U_nu(x+mu) U_mu(x+nu)^+ U_nu(x)^+
+    // backward: U_mu(x) U_nu(x+mu-nu)^+ U_mu(x-nu)^+ U_nu(x-nu)
+    Mat<NC> p = get_link<NC>(links, s, mu);
+    if (back) {
+        const int sn = nbr(s, nu, -1, n0, n1, n2);
+        p = mmul<NC>(p, mdag<NC>(get_link<NC>(links, nbr(sp, nu, -1, n0, n1, n2), nu)));
+        p = mmul<NC>(p, mdag<NC>(get_link<NC>(links, sn, mu)));
+        p = mmul<NC>(p, get_link<NC>(links, sn, nu));
+    } else {
+        p = mmul<NC>(p, get_link<NC>(links, sp, nu));
+        p = mmul<NC>(p, mdag<NC>(get_link<NC>(links, nbr(s, nu, 1, n0, n1, n2), mu)));
         p = mmul<NC>(p, mdag<NC>(get_link<NC>(links, s, nu)));
-        double t[NG];
-        retr_it<NC>(p, t);
-#pragma unroll
-        for (int a = 0; a < NG; ++a) f[a] += t[a];
-        // backward: U_mu(x) U_nu(x+mu-nu)^+ U_mu(x-nu)^+ U_nu(x-nu)
-        const int smn = nbr(sp, nu, -1, n0, n1, n2);
-        const int sm = nbr(s, nu, -1, n0, n1, n2);
-        Mat<NC> q = mmul<NC>(umu, mdag<NC>(get_link<NC>(links, smn, nu)));
-        q = mmul<NC>(q, mdag<NC>(get_link<NC>(links, sm, mu)));
-        q = mmul<NC>(q, get_link<NC>(links, sm, nu));
-        retr_it<NC>(q, t);
-#pragma unroll
-        for (int a = 0; a < NG; ++a) f[a] += t[a];
     }
+    double f[NG];
+    retr_sums<NC>(p, f);
+    const int base = (int)(threadIdx.x & 60);
 #pragma unroll
-    for (int a = 0; a < NG; ++a) e[NG * (mu + 3 * s) + a] += -2.0 * dt * f[a];
+    for (int k = 0; k < NG; ++k) {  // in the order of the planes
+        double t = 0;
+#pragma unroll
+        for (int l = 0; l < 4; ++l) t = __builtin_fma(retr_factor(k), __shfl(f[k], base + l, 64), t);
+        f[k] = t;
+    }
+    if (!ok) return;
+    double *o = e + (size_t)NG * i;
+#pragma unroll
+    for (int k = 0; k < NG; ++k)
+        if (k % 4 == j) o[k] += -2.0 * dt * f[k];
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1151,10 +1235,11 @@ __device__ __forceinline__ double wave_max(double v)
     return v;
 }
 
-// block reduction of NV values (sum or max per value); result valid in thread 0
-template <int NV> __device__ void block_reduce(double *v, const int *is_max)
+// block reduction of NV values (sum or max per value) in a workgroup of NT threads; result valid in
+// thread 0
+template <int NV, int NT = TPB> __device__ void block_reduce(double *v, const int *is_max)
 {
-    __shared__ double sh[TPB / 64][NV];
+    __shared__ double sh[NT / 64][NV];
     const int w = threadIdx.x / 64, l = threadIdx.x % 64;
 #pragma unroll
     for (int k = 0; k < NV; ++k) v[k] = is_max[k] ? wave_max(v[k]) : wave_sum(v[k]);
@@ -1166,63 +1251,10 @@ template <int NV> __device__ void block_reduce(double *v, const int *is_max)
 #pragma unroll
         for (int k = 0; k < NV; ++k) {
             double r = sh[0][k];
-            for (int j = 1; j < TPB / 64; ++j) r = is_max[k] ? fmax(r, sh[j][k]) : r + sh[j][k];
+            for (int j = 1; j < NT / 64; ++j) r = is_max[k] ? fmax(r, sh[j][k]) : r + sh[j][k];
             v[k] = r;
         }
     }
-}
-
-template <int NV>
-__global__ __launch_bounds__(TPB) void k_finish(const double *__restrict__ partial, int nblocks, double *out, int m0,
-                                                int m1, int m2, int m3)
-{
-    const int is_max[4] = {m0, m1, m2, m3};
-    double v[NV];
-#pragma unroll
-    for (int k = 0; k < NV; ++k) {
-        double r = is_max[k] ? 0.0 : 0.0;
-        for (int b = threadIdx.x; b < nblocks; b += TPB) {
-            const double p = partial[(size_t)b * NV + k];
-            r = is_max[k] ? fmax(r, p) : r + p;
-        }
-        v[k] = r;
-    }
-    block_reduce<NV>(v, is_max);
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int k = 0; k < NV; ++k) out[k] = v[k];
-}
-
-template <int NC> __device__ double plaq_retr_1mu(const double *links, int s, int mu, int nu, int n0, int n1, int n2)
-{
-    const int sp = nbr(s, mu, 1, n0, n1, n2), snu = nbr(s, nu, 1, n0, n1, n2);
-    Mat<NC> p = mmul<NC>(get_link<NC>(links, s, mu), get_link<NC>(links, sp, nu));
-    p = mmul<NC>(p, mdag<NC>(get_link<NC>(links, snu, mu)));
-    p = mmul<NC>(p, mdag<NC>(get_link<NC>(links, s, nu)));
-    double tr = 0;
-#pragma unroll
-    for (int i = 0; i < NC; ++i) tr += 1.0 - p.e[i * NC + i].r;
-    return tr;
-}
-
-// energy: (1/2) sum E^2 and (1/2) sum_planes 4 ReTr(1 - U_plaq)   (BulkObservables.cpp:29-31,84-86)
-template <int NC>
-__global__ __launch_bounds__(TPB) void k_energy(const double *__restrict__ links, const double *__restrict__ e,
-                                                double *partial, int n0, int n1, int n2)
-{
-    const int V = n0 * n1 * n2;
-    constexpr int NG = NC * NC - 1;
-    double v[2] = {0, 0};
-    for (int s = blockIdx.x * TPB + threadIdx.x; s < V; s += RED_BLOCKS * TPB) {
-        for (int k = 0; k < 3 * NG; ++k) { const double q = e[(size_t)3 * NG * s + k]; v[0] += q * q; }
-        v[1] += 4.0 * (plaq_retr_1mu<NC>(links, s, 1, 2, n0, n1, n2) + plaq_retr_1mu<NC>(links, s, 2, 0, n0, n1, n2) +
-                       plaq_retr_1mu<NC>(links, s, 0, 1, n0, n1, n2));
-    }
-    v[0] *= 0.5;
-    v[1] *= 0.5;
-    const int ism[2] = {0, 0};
-    block_reduce<2>(v, ism);
-    if (threadIdx.x == 0) { partial[2 * blockIdx.x] = v[0]; partial[2 * blockIdx.x + 1] = v[1]; }
 }
 
 // components X^a = 2 tr(t^a X) of a Hermitian traceless matrix, via ReTr(i t^a (-i X))
@@ -1236,49 +1268,114 @@ template <int NC> __device__ __forceinline__ void alg_components(const Mat<NC> &
     for (int a = 0; a < NC * NC - 1; ++a) out[a] *= 2.0;
 }
 
-// Gauss law G(x) = sum_mu E_mu(x) - U_mu(x-mu)^+ E_mu(x-mu) U_mu(x-mu), components G^a
-template <int NC>
-__device__ void gauss_site(const double *__restrict__ links, const double *__restrict__ e, int s, int n0, int n1,
-                           int n2, double *comp)
-{
-    constexpr int NG = NC * NC - 1;
-    Mat<NC> G;
-#pragma unroll
-    for (int k = 0; k < NC * NC; ++k) G.e[k] = {0, 0};
-    for (int mu = 0; mu < 3; ++mu) {
-        const int sm = nbr(s, mu, -1, n0, n1, n2);
-        Mat<NC> e0 = alg_to_mat<NC>(e + NG * (mu + 3 * s));
-        Mat<NC> e1 = alg_to_mat<NC>(e + NG * (mu + 3 * sm));
-        Mat<NC> u = get_link<NC>(links, sm, mu);
-        Mat<NC> t = mmul<NC>(mmul<NC>(mdag<NC>(u), e1), u);
-#pragma unroll
-        for (int k = 0; k < NC * NC; ++k) G.e[k] = {G.e[k].r + e0.e[k].r - t.e[k].r, G.e[k].i + e0.e[k].i - t.e[k].i};
-    }
-    alg_components<NC>(G, comp);
-}
-
-// max |G^a| and sum G^2 (GaussLawViolation.cpp:13-61); with g != null also stores G^a(x)
-template <int NC>
-__global__ __launch_bounds__(TPB) void k_gauss(const double *__restrict__ links, const double *__restrict__ e,
-                                               double *partial, double *__restrict__ g, int n0, int n1, int n2)
+// The site-local observables in one pass, four lanes per site (lane mu < 3 has direction mu, the plane
+// (mu + 1, mu + 2) and the link (s, mu); lane 3 idles):
+//   (1/2) sum E^2 and (1/2) sum_planes 4 ReTr(1 - U_plaq)     (BulkObservables.cpp:29-31,84-86)
+//   max |G^a| and sum G^2 of G(x) = sum_mu E_mu(x) - U_mu(x-mu)^+ E_mu(x-mu) U_mu(x-mu)
+//                                                             (GaussLawViolation.cpp:13-61)
+//   max and sum of the squares of ||U U^+ - 1||               (UnitarityViolation.cpp:13-51)
+// g (optional): G^a(x) stored as [site][a]; GAUSS_ONLY leaves the other two out.  24^3 SU(3): 9.7 us where
+// three kernels and their finishing passes took 37 us.
+enum { LOC_EEL = 0, LOC_EMAG, LOC_GMAX, LOC_GSUM, LOC_UMAX, LOC_USUM, LOC_COUNT };
+template <int NC, bool GAUSS_ONLY>
+__global__ __launch_bounds__(TPB) void k_obs_local(const double *__restrict__ links, const double *__restrict__ e,
+                                                   double *partial, double *__restrict__ g, int n0, int n1, int n2)
 {
     const int V = n0 * n1 * n2;
     constexpr int NG = NC * NC - 1;
-    double v[2] = {0, 0};
-    for (int s = blockIdx.x * TPB + threadIdx.x; s < V; s += RED_BLOCKS * TPB) {
+    double v[LOC_COUNT] = {0, 0, 0, 0, 0, 0};
+    const int mu = threadIdx.x % 4;
+    const bool dir = mu < 3;
+    const int stride = (int)gridDim.x * (TPB / 4);
+    // the four lanes of a site share the loop condition
+    for (int s = (int)blockIdx.x * (TPB / 4) + threadIdx.x / 4; s < V; s += stride) {
         double comp[NG];
-        gauss_site<NC>(links, e, s, n0, n1, n2, comp);
+#pragma unroll
+        for (int a = 0; a < NG; ++a) comp[a] = 0;
+        if (dir) {
+            const int sm = nbr(s, mu, -1, n0, n1, n2);
+            const Mat<NC> e0 = alg_to_mat<NC>(e + (size_t)NG * (mu + 3 * (size_t)s));
+            const Mat<NC> e1 = alg_to_mat<NC>(e + (size_t)NG * (mu + 3 * (size_t)sm));
+            const Mat<NC> ub = get_link<NC>(links, sm, mu);
+            Mat<NC> t = mmul<NC>(mmul<NC>(mdag<NC>(ub), e1), ub);
+#pragma unroll
+            for (int k = 0; k < NC * NC; ++k) t.e[k] = {e0.e[k].r - t.e[k].r, e0.e[k].i - t.e[k].i};
+            alg_components<NC>(t, comp);
+            if constexpr (!GAUSS_ONLY) {
+                for (int a = 0; a < NG; ++a) {
+                    const double q = e[(size_t)NG * (mu + 3 * (size_t)s) + a];
+                    v[LOC_EEL] += q * q;
+                }
+                const int a = (mu + 1) % 3, b = (mu + 2) % 3;
+                Mat<NC> p = mmul<NC>(get_link<NC>(links, s, a), get_link<NC>(links, nbr(s, a, 1, n0, n1, n2), b));
+                p = mmul<NC>(p, mdag<NC>(get_link<NC>(links, nbr(s, b, 1, n0, n1, n2), a)));
+                p = mmul<NC>(p, mdag<NC>(get_link<NC>(links, s, b)));
+                double tr = 0;
+#pragma unroll
+                for (int i = 0; i < NC; ++i) tr += 1.0 - p.e[i * NC + i].r;
+                v[LOC_EMAG] += 4.0 * tr;
+                double nrm;
+                if constexpr (NC == 2) {  // UnitarityNorm (SU2/GroupOperations.cpp:172-184)
+                    const double *u = links + 4 * (mu + 3 * (size_t)s);
+                    const double c3 = u[3] * u[3] + u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
+                    nrm = fabs(c3 - 1.0);
+                } else {
+                    const Mat<3> u = get_link<3>(links, s, mu);
+                    const Mat<3> q = mmul<3>(u, mdag<3>(u));
+                    nrm = 0;
+                    for (int i = 0; i < 3; ++i)
+                        for (int k = 0; k < 3; ++k) {
+                            const double re = q.e[i * 3 + k].r - (i == k ? 1.0 : 0.0), im = q.e[i * 3 + k].i;
+                            nrm += re * re + im * im;
+                        }
+                    nrm = sqrt(nrm);
+                }
+                v[LOC_UMAX] = fmax(v[LOC_UMAX], nrm);
+                v[LOC_USUM] += nrm * nrm;
+            }
+        }
 #pragma unroll
         for (int a = 0; a < NG; ++a) {
-            if (g) g[(size_t)NG * s + a] = comp[a];
-            const double q = fabs(comp[a]);
-            v[0] = fmax(v[0], q);
-            v[1] += q * q;
+            comp[a] += __shfl_xor(comp[a], 1, 64);
+            comp[a] += __shfl_xor(comp[a], 2, 64);
+            if (a % 4 == mu) {  // every lane of the site holds G^a: each keeps its share
+                if (g) g[(size_t)NG * s + a] = comp[a];
+                const double q = fabs(comp[a]);
+                v[LOC_GMAX] = fmax(v[LOC_GMAX], q);
+                v[LOC_GSUM] += q * q;
+            }
         }
     }
-    const int ism[2] = {1, 0};
-    block_reduce<2>(v, ism);
-    if (threadIdx.x == 0) { partial[2 * blockIdx.x] = v[0]; partial[2 * blockIdx.x + 1] = v[1]; }
+    v[LOC_EEL] *= 0.5;
+    v[LOC_EMAG] *= 0.5;
+    const int ism[LOC_COUNT] = {0, 0, 1, 0, 1, 0};
+    block_reduce<LOC_COUNT>(v, ism);
+    if (threadIdx.x == 0)
+#pragma unroll
+        for (int k = 0; k < LOC_COUNT; ++k) partial[(size_t)blockIdx.x * LOC_COUNT + k] = v[k];
+}
+
+// the partial results of k_obs_local (nl of them; none when 0) and of k_edotb (ne; likewise), summed in a
+// fixed order: out[0 .. LOC_COUNT) and out[LOC_COUNT]
+__global__ __launch_bounds__(TPB) void k_obs_finish(const double *__restrict__ local, int nl,
+                                                    const double *__restrict__ edotb, int ne, double *out)
+{
+    const int ism[LOC_COUNT + 1] = {0, 0, 1, 0, 1, 0, 0};
+    double v[LOC_COUNT + 1] = {0, 0, 0, 0, 0, 0, 0};
+    for (int b = threadIdx.x; b < nl; b += TPB)
+#pragma unroll
+        for (int k = 0; k < LOC_COUNT; ++k) {
+            const double p = local[(size_t)b * LOC_COUNT + k];
+            v[k] = ism[k] ? fmax(v[k], p) : v[k] + p;
+        }
+    for (int b = threadIdx.x; b < ne; b += TPB) v[LOC_COUNT] += edotb[b];
+    block_reduce<LOC_COUNT + 1>(v, ism);
+    if (threadIdx.x == 0) {
+        if (nl > 0)
+#pragma unroll
+            for (int k = 0; k < LOC_COUNT; ++k) out[k] = v[k];
+        if (ne > 0) out[LOC_COUNT] = v[LOC_COUNT];
+    }
 }
 
 // one relaxation step of GaussLawRestoration::UpdateElectricFields (GaussRestore.cpp:74-112):
@@ -1302,147 +1399,185 @@ __global__ __launch_bounds__(TPB) void k_gauss_restore(const double *__restrict_
     for (int a = 0; a < NG; ++a) e[(size_t)NG * (mu + 3 * s) + a] -= gamma * (g[(size_t)NG * s + a] - up[a]);
 }
 
-template <int NC>
-__global__ __launch_bounds__(TPB) void k_unitarity(const double *__restrict__ links, double *partial, int V)
+// improved sum_x E.B (ChernSimonsOperators.cpp:228-439): per site and direction mu, with (a, b) the plane
+// across mu,
+//   E = 7/12 E(0) - 1/12 U E(1) U^+ + 7/12 U(-1)^+ E(-1) U(-1) - 1/12 (..)^+ E(-2) (..)
+//   B = 5/12 sum of the four plaquettes at the site - 1/24 sum of the eight 2 x 1 rectangles
+// with every loop and E transported to the site; the sum is 4 sum_c ReTr(t^c E) ReTr(i t^c B) =
+// 4 ReTr(i E' B) with E' the traceless Hermitian half of E.
+//
+// A lane holds one row of one quadrant's loops (a plaquette and two rectangles) or of E and walks it
+// along their links, a row times a matrix per link; loops that share their first or last links are added
+// before the shared ones (10 or 17 products per quadrant instead of 16 and 24).  A wavefront is one
+// quadrant (or E) of 64 / Nc (site, mu) pairs, so its lanes run the same products; the five wavefronts
+// of a workgroup meet in LDS.  FP64 issue bounds it on large lattices (62 products of about 80
+// instructions per Nc lanes), the chain of 17 on small ones.  One lane per site making 675 matrix
+// products took 328 us on 24^3 SU(3) and 94 us on 8^3 SU(2); this form 55 and 5 us.
+template <int NC, bool DAG>
+__device__ __forceinline__ void row_step(cd *v, const double *__restrict__ links, int s, int mu)
 {
-    double v[2] = {0, 0};
-    for (int i = blockIdx.x * TPB + threadIdx.x; i < 3 * V; i += RED_BLOCKS * TPB) {
-        const int s = i / 3, mu = i - 3 * s;
-        double nrm;
-        if constexpr (NC == 2) {  // UnitarityNorm (SU2/GroupOperations.cpp:172-184)
-            const double *u = links + 4 * (mu + 3 * s);
-            const double c3 = u[3] * u[3] + u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
-            nrm = fabs(c3 - 1.0);
-        } else {
-            Mat<3> u = get_link<3>(links, s, mu);
-            Mat<3> p = mmul<3>(u, mdag<3>(u));
-            nrm = 0;
-            for (int a = 0; a < 3; ++a)
-                for (int b = 0; b < 3; ++b) {
-                    const double re = p.e[a * 3 + b].r - (a == b ? 1.0 : 0.0), im = p.e[a * 3 + b].i;
-                    nrm += re * re + im * im;
-                }
-            nrm = sqrt(nrm);
-        }
-        v[0] = fmax(v[0], nrm);
-        v[1] += nrm * nrm;
+    const Mat<NC> m = get_link<NC>(links, s, mu);
+    cd r[NC];
+#pragma unroll
+    for (int j = 0; j < NC; ++j) {
+        cd t = {0, 0};
+#pragma unroll
+        for (int k = 0; k < NC; ++k)
+            t = cadd(t, DAG ? cmul(v[k], cd{m.e[j * NC + k].r, -m.e[j * NC + k].i}) : cmul(v[k], m.e[k * NC + j]));
+        r[j] = t;
     }
-    const int ism[2] = {1, 0};
-    block_reduce<2>(v, ism);
-    if (threadIdx.x == 0) { partial[2 * blockIdx.x] = v[0]; partial[2 * blockIdx.x + 1] = v[1]; }
+#pragma unroll
+    for (int j = 0; j < NC; ++j) v[j] = r[j];
 }
 
-// improved sum_x E.B (ChernSimonsOperators.cpp:228-439)
-template <int NC> __device__ __forceinline__ Mat<NC> L_(const double *links, int s, int mu) { return get_link<NC>(links, s, mu); }
-
-template <int NC> __device__ __forceinline__ Mat<NC> transport(const Mat<NC> &u, const Mat<NC> &q)
+// v <- v E of the site's field e[0 .. Nc^2 - 1)
+template <int NC> __device__ __forceinline__ void row_field(cd *v, const double *__restrict__ e)
 {
-    return mmul<NC>(mmul<NC>(u, q), mdag<NC>(u));
-}
-
-template <int NC>
-__device__ __forceinline__ void acc(Mat<NC> &a, const Mat<NC> &b, double w)
-{
+    const Mat<NC> m = alg_to_mat<NC>(e);
+    cd r[NC];
 #pragma unroll
-    for (int k = 0; k < NC * NC; ++k) { a.e[k].r += w * b.e[k].r; a.e[k].i += w * b.e[k].i; }
-}
-
-template <int NC>
-__device__ double edotb_site(const double *links, const double *e, int s, int n0, int n1, int n2)
-{
-    constexpr int NG = NC * NC - 1;
-    double total = 0;
-    for (int mu = 0; mu < 3; ++mu) {
-        const int a = (mu + 1) % 3, b = (mu + 2) % 3;
-        // site at (i along a, j along b)
-        auto at = [&](int i, int j) {
-            int t = s;
-            if (i) t = nbr(t, a, i, n0, n1, n2);
-            if (j) t = nbr(t, b, j, n0, n1, n2);
-            return t;
-        };
-        auto atm = [&](int k) { return nbr(s, mu, k, n0, n1, n2); };
-        // E_mu transported average
-        Mat<NC> ea;
+    for (int j = 0; j < NC; ++j) {
+        cd t = {0, 0};
 #pragma unroll
-        for (int k = 0; k < NC * NC; ++k) ea.e[k] = {0, 0};
-        acc<NC>(ea, alg_to_mat<NC>(e + NG * (mu + 3 * s)), 7.0 / 12.0);
-        acc<NC>(ea, transport<NC>(L_<NC>(links, s, mu), alg_to_mat<NC>(e + NG * (mu + 3 * atm(1)))), -1.0 / 12.0);
-        const Mat<NC> um = mdag<NC>(L_<NC>(links, atm(-1), mu));
-        acc<NC>(ea, transport<NC>(um, alg_to_mat<NC>(e + NG * (mu + 3 * atm(-1)))), 7.0 / 12.0);
-        const Mat<NC> um2 = mmul<NC>(um, mdag<NC>(L_<NC>(links, atm(-2), mu)));
-        acc<NC>(ea, transport<NC>(um2, alg_to_mat<NC>(e + NG * (mu + 3 * atm(-2)))), -1.0 / 12.0);
-        // E^a = 2 tr(t^a E) = 2 ReTr(i t^a (-i E))
-        Mat<NC> mie;
-#pragma unroll
-        for (int k = 0; k < NC * NC; ++k) mie.e[k] = {ea.e[k].i, -ea.e[k].r};
-        double Ea[NG];
-        retr_it<NC>(mie, Ea);
-
-        // B from the (a, b) plane
-        const Mat<NC> uaM = mdag<NC>(L_<NC>(links, at(-1, 0), a));
-        const Mat<NC> ubM = mdag<NC>(L_<NC>(links, at(0, -1), b));
-        const Mat<NC> ua2M = mmul<NC>(uaM, mdag<NC>(L_<NC>(links, at(-2, 0), a)));
-        const Mat<NC> ub2M = mmul<NC>(ubM, mdag<NC>(L_<NC>(links, at(0, -2), b)));
-        Mat<NC> ub;
-#pragma unroll
-        for (int k = 0; k < NC * NC; ++k) ub.e[k] = {0, 0};
-        auto box = [&](int i, int j, int dag12) {  // UUDD from (i,j) or DDUU
-            (void)dag12;
-            return mmul<NC>(mmul<NC>(L_<NC>(links, at(i, j), a), L_<NC>(links, at(i + 1, j), b)),
-                            mmul<NC>(mdag<NC>(L_<NC>(links, at(i, j + 1), a)), mdag<NC>(L_<NC>(links, at(i, j), b))));
-        };
-        acc<NC>(ub, box(0, 0, 0), 5.0 / 12.0);
-        acc<NC>(ub, transport<NC>(uaM, box(-1, 0, 0)), 5.0 / 12.0);
-        {  // lower left: U_a(-1,0)^+ U_b(-1,-1)^+ U_a(-1,-1) U_b(0,-1)
-            Mat<NC> p = mmul<NC>(mdag<NC>(L_<NC>(links, at(-1, 0), a)), mdag<NC>(L_<NC>(links, at(-1, -1), b)));
-            p = mmul<NC>(p, mmul<NC>(L_<NC>(links, at(-1, -1), a), L_<NC>(links, at(0, -1), b)));
-            acc<NC>(ub, p, 5.0 / 12.0);
-        }
-        acc<NC>(ub, transport<NC>(ubM, box(0, -1, 0)), 5.0 / 12.0);
-        // rectangles: six links (offset i, offset j, direction b?, dagger?)
-        struct R6 { signed char o[6][2]; unsigned char d[6]; unsigned char g[6]; unsigned char t; };
-        const R6 R[8] = {
-            {{{0, 0}, {1, 0}, {2, 0}, {1, 1}, {0, 1}, {0, 0}}, {0, 0, 1, 0, 0, 1}, {0, 0, 0, 1, 1, 1}, 0},
-            {{{0, 0}, {1, 0}, {1, 1}, {0, 2}, {0, 1}, {0, 0}}, {0, 1, 1, 0, 1, 1}, {0, 0, 0, 1, 1, 1}, 0},
-            {{{-1, 0}, {0, 0}, {0, 1}, {-1, 2}, {-1, 1}, {-1, 0}}, {0, 1, 1, 0, 1, 1}, {0, 0, 0, 1, 1, 1}, 1},
-            {{{-2, 0}, {-1, 0}, {0, 0}, {-1, 1}, {-2, 1}, {-2, 0}}, {0, 0, 1, 0, 0, 1}, {0, 0, 0, 1, 1, 1}, 2},
-            {{{-1, 0}, {-1, -1}, {-1, -2}, {-1, -2}, {0, -2}, {0, -1}}, {0, 1, 1, 0, 1, 1}, {1, 1, 1, 0, 0, 0}, 0},
-            {{{-1, 0}, {-2, 0}, {-2, -1}, {-2, -1}, {-1, -1}, {0, -1}}, {0, 0, 1, 0, 0, 1}, {1, 1, 1, 0, 0, 0}, 0},
-            {{{0, -1}, {1, -1}, {2, -1}, {1, 0}, {0, 0}, {0, -1}}, {0, 0, 1, 0, 0, 1}, {0, 0, 0, 1, 1, 1}, 3},
-            {{{0, -2}, {1, -2}, {1, -1}, {0, 0}, {0, -1}, {0, -2}}, {0, 1, 1, 0, 1, 1}, {0, 0, 0, 1, 1, 1}, 4},
-        };
-        for (int r = 0; r < 8; ++r) {
-            Mat<NC> p = mid<NC>();
-            for (int k = 0; k < 6; ++k) {
-                Mat<NC> l = L_<NC>(links, at(R[r].o[k][0], R[r].o[k][1]), R[r].d[k] ? b : a);
-                p = mmul<NC>(p, R[r].g[k] ? mdag<NC>(l) : l);
-            }
-            if (R[r].t == 1) p = transport<NC>(uaM, p);
-            if (R[r].t == 2) p = transport<NC>(ua2M, p);
-            if (R[r].t == 3) p = transport<NC>(ubM, p);
-            if (R[r].t == 4) p = transport<NC>(ub2M, p);
-            acc<NC>(ub, p, -1.0 / 24.0);
-        }
-        double Bb[NG];
-        retr_it<NC>(ub, Bb);
-#pragma unroll
-        for (int c = 0; c < NG; ++c) total += 2.0 * Ea[c] * 2.0 * Bb[c];
+        for (int k = 0; k < NC; ++k) t = cadd(t, cmul(v[k], m.e[k * NC + j]));
+        r[j] = t;
     }
-    return total;
+#pragma unroll
+    for (int j = 0; j < NC; ++j) v[j] = r[j];
 }
 
-template <int NC>
-__global__ __launch_bounds__(TPB) void k_edotb(const double *__restrict__ links, const double *__restrict__ e,
-                                               double *partial, int n0, int n1, int n2)
+template <int NC> struct Row {
+    cd e[NC];
+};
+template <int NC> __device__ __forceinline__ Row<NC> row_add(const Row<NC> &x, double wx, const Row<NC> &y, double wy)
 {
+    Row<NC> r;
+#pragma unroll
+    for (int k = 0; k < NC; ++k) r.e[k] = {wx * x.e[k].r + wy * y.e[k].r, wx * x.e[k].i + wy * y.e[k].i};
+    return r;
+}
+
+__device__ __forceinline__ int wrap(int c, int n) { return c < 0 ? c + n : (c >= n ? c - n : c); }  // |offset| <= 2 < n
+
+constexpr int EB_TPB = 5 * 64;  // four quadrants and E
+template <int NC>
+__global__ __launch_bounds__(EB_TPB) void k_edotb(const double *__restrict__ links, const double *__restrict__ e,
+                                                  double *partial, int n0, int n1, int n2)
+{
+    constexpr int NG = NC * NC - 1, PAIRS = 64 / NC;
+    constexpr double W4 = 5.0 / 12.0, W6 = -1.0 / 24.0;
+    __shared__ cd er[PAIRS][NC][NC];
     const int V = n0 * n1 * n2;
-    double v[1] = {0};
-    for (int s = blockIdx.x * TPB + threadIdx.x; s < V; s += RED_BLOCKS * TPB)
-        v[0] += edotb_site<NC>(links, e, s, n0, n1, n2);
+    const int part = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64;
+    const bool used = lane < PAIRS * NC;
+    const int pair = used ? lane / NC : PAIRS - 1, row = used ? lane % NC : 0;
+    double acc[1] = {0.0};
+    const int npairs = 3 * V;
+    for (int base = (int)blockIdx.x * PAIRS; base < npairs; base += (int)gridDim.x * PAIRS) {
+        const int gi = base + pair;
+        const int gc = gi < npairs ? gi : npairs - 1;  // spare lanes repeat the last pair's work
+        const bool ok = used && gi < npairs;
+        const int s = gc / 3, mu = gc - 3 * s;
+        const int z = s / (n0 * n1), rem = s - z * n0 * n1, y = rem / n0, x = rem - y * n0;
+        const int a = mu == 2 ? 0 : mu + 1, b = mu == 0 ? 2 : mu - 1;
+        auto pick = [](int d, int v0, int v1, int v2) { return d == 0 ? v0 : (d == 1 ? v1 : v2); };
+        const int ca = pick(a, x, y, z), na = pick(a, n0, n1, n2), sa = pick(a, 1, n0, n0 * n1);
+        const int cb = pick(b, x, y, z), nb = pick(b, n0, n1, n2), sb = pick(b, 1, n0, n0 * n1);
+        const int origin = s - ca * sa - cb * sb;
+        auto at = [&](int i, int j) { return origin + wrap(ca + i, na) * sa + wrap(cb + j, nb) * sb; };
+        Row<NC> v;
+#pragma unroll
+        for (int k = 0; k < NC; ++k) v.e[k] = {k == row ? 1.0 : 0.0, 0.0};
+        // v <- v U, v U^+ for the links A (direction a) and B at the offsets (i, j)
+        auto A = [&](Row<NC> &r, int i, int j) { row_step<NC, false>(r.e, links, at(i, j), a); };
+        auto Ad = [&](Row<NC> &r, int i, int j) { row_step<NC, true>(r.e, links, at(i, j), a); };
+        auto B = [&](Row<NC> &r, int i, int j) { row_step<NC, false>(r.e, links, at(i, j), b); };
+        auto Bd = [&](Row<NC> &r, int i, int j) { row_step<NC, true>(r.e, links, at(i, j), b); };
+        if (part == 0) {  // quadrant (+a, +b)
+            A(v, 0, 0);
+            Row<NC> t = v, q = v;
+            B(t, 1, 0);
+            A(q, 1, 0); B(q, 2, 0); Ad(q, 1, 1);
+            q = row_add<NC>(t, W4, q, W6);
+            Ad(q, 0, 1);
+            B(t, 1, 1); Ad(t, 0, 2); Bd(t, 0, 1);
+            v = row_add<NC>(q, 1.0, t, W6);
+            Bd(v, 0, 0);
+        } else if (part == 1) {  // quadrant (-a, +b), transported along a
+            Ad(v, -1, 0);
+            Row<NC> q = v;
+            A(v, -1, 0); B(v, 0, 0);
+            Row<NC> t = v;
+            Ad(v, -1, 1);
+            B(t, 0, 1); Ad(t, -1, 2); Bd(t, -1, 1);
+            v = row_add<NC>(v, W4, t, W6);
+            Bd(v, -1, 0);
+            Ad(q, -2, 0); A(q, -2, 0); A(q, -1, 0); B(q, 0, 0); Ad(q, -1, 1); Ad(q, -2, 1); Bd(q, -2, 0); A(q, -2, 0);
+            v = row_add<NC>(v, 1.0, q, W6);
+            A(v, -1, 0);
+        } else if (part == 2) {  // quadrant (-a, -b)
+            Ad(v, -1, 0);
+            Row<NC> t = v, q = v;
+            Bd(t, -1, -1);
+            Ad(q, -2, 0); Bd(q, -2, -1); A(q, -2, -1);
+            q = row_add<NC>(t, W4, q, W6);
+            A(q, -1, -1);
+            Bd(t, -1, -2); A(t, -1, -2); B(t, 0, -2);
+            v = row_add<NC>(q, 1.0, t, W6);
+            B(v, 0, -1);
+        } else if (part == 3) {  // quadrant (+a, -b), transported along b
+            Bd(v, 0, -1);
+            Row<NC> q = v;
+            A(v, 0, -1);
+            Row<NC> t = v;
+            B(v, 1, -1);
+            A(t, 1, -1); B(t, 2, -1); Ad(t, 1, 0);
+            v = row_add<NC>(v, W4, t, W6);
+            Ad(v, 0, 0); Bd(v, 0, -1);
+            Bd(q, 0, -2); A(q, 0, -2); B(q, 1, -2); B(q, 1, -1); Ad(q, 0, 0); Bd(q, 0, -1); Bd(q, 0, -2); B(q, 0, -2);
+            v = row_add<NC>(v, 1.0, q, W6);
+            B(v, 0, -1);
+        } else {
+            const int cm = pick(mu, x, y, z), nm = pick(mu, n0, n1, n2), sm = pick(mu, 1, n0, n0 * n1);
+            const int line = s - cm * sm;
+            const int sp = line + wrap(cm + 1, nm) * sm, s1 = line + wrap(cm - 1, nm) * sm, s2 = line + wrap(cm - 2, nm) * sm;
+            auto E = [&](Row<NC> &r, int site) { row_field<NC>(r.e, e + (size_t)NG * (mu + 3 * (size_t)site)); };
+            Row<NC> t = v, q = v;
+            E(v, s);
+            row_step<NC, false>(t.e, links, s, mu);
+            E(t, sp);
+            row_step<NC, true>(t.e, links, s, mu);
+            v = row_add<NC>(v, 7.0 / 12.0, t, -1.0 / 12.0);
+            row_step<NC, true>(q.e, links, s1, mu);
+            t = q;
+            E(q, s1);
+            row_step<NC, true>(t.e, links, s2, mu);
+            E(t, s2);
+            row_step<NC, false>(t.e, links, s2, mu);
+            q = row_add<NC>(q, 7.0 / 12.0, t, -1.0 / 12.0);
+            row_step<NC, false>(q.e, links, s1, mu);
+            v = row_add<NC>(v, 1.0, q, 1.0);
+            if (used)
+#pragma unroll
+                for (int k = 0; k < NC; ++k) er[pair][row][k] = v.e[k];
+        }
+        __syncthreads();
+        if (ok && part < 4) {
+            double tr = 0, im = 0;
+            for (int k = 0; k < NC; ++k) tr += er[pair][k][k].r;
+#pragma unroll
+            for (int k = 0; k < NC; ++k) {  // Im of (B E')_{row,row}
+                const cd p = er[pair][k][row], q = er[pair][row][k];
+                const cd h = {0.25 * (p.r + q.r) - (k == row ? 0.5 * tr / NC : 0.0), 0.25 * (p.i - q.i)};
+                im += cmul(v.e[k], h).i;
+            }
+            acc[0] -= 4.0 * im;
+        }
+        __syncthreads();
+    }
     const int ism[1] = {0};
-    block_reduce<1>(v, ism);
-    if (threadIdx.x == 0) partial[blockIdx.x] = v[0];
+    block_reduce<1, EB_TPB>(acc, ism);
+    if (threadIdx.x == 0) partial[blockIdx.x] = acc[0];
 }
 
 // per-mode inner products: partial[chunk][mode] then a fixed-order sum over chunks
@@ -1966,19 +2101,22 @@ hipError_t launch_ucc_to_links(const Geom &g, const double *ucc, double *ul64, f
 }
 
 hipError_t launch_link_update(const Geom &g, double *links, const double *efield, double dt, int reunit,
-                              hipStream_t st)
+                              const double *phase, double *ul64, float *ul32, hipStream_t st)
 {
-    const unsigned nb = nblocks(3L * g.V);
-    if (g.nc == 2) k_link_update<2><<<nb, TPB, 0, st>>>(links, efield, dt, g.V, reunit);
-    else k_link_update<3><<<nb, TPB, 0, st>>>(links, efield, dt, g.V, reunit);
+    const unsigned nb = (unsigned)((3L * g.V * (g.nc == 2 ? 1 : 4) + LINK_TPB - 1) / LINK_TPB);
+    const auto ph = (const double2 *)phase;
+    if (g.nc == 2)
+        k_link_update<2><<<nb, LINK_TPB, 0, st>>>(links, efield, dt, g.V, reunit, ph, (double2 *)ul64, (float2 *)ul32);
+    else
+        k_link_update<3><<<nb, LINK_TPB, 0, st>>>(links, efield, dt, g.V, reunit, ph, (double2 *)ul64, (float2 *)ul32);
     return hipGetLastError();
 }
 
 hipError_t launch_efield_update(const Geom &g, const double *links, double *efield, double dt, hipStream_t st)
 {
-    const unsigned nb = nblocks(3L * g.V);
-    if (g.nc == 2) k_efield_update<2><<<nb, TPB, 0, st>>>(links, efield, dt, g.n0, g.n1, g.n2);
-    else k_efield_update<3><<<nb, TPB, 0, st>>>(links, efield, dt, g.n0, g.n1, g.n2);
+    const unsigned nb = (unsigned)((12L * g.V + LINK_TPB - 1) / LINK_TPB);
+    if (g.nc == 2) k_efield_update<2><<<nb, LINK_TPB, 0, st>>>(links, efield, dt, g.n0, g.n1, g.n2);
+    else k_efield_update<3><<<nb, LINK_TPB, 0, st>>>(links, efield, dt, g.n0, g.n1, g.n2);
     return hipGetLastError();
 }
 
@@ -2011,23 +2149,31 @@ hipError_t launch_mode_dot(const Geom &g, const void *a, const void *b, double *
     return hipGetLastError();
 }
 
-size_t reduce_partial_len(const Geom &) { return (size_t)RED_BLOCKS * 4; }
+// partial results of the observables: LOC_BLOCKS x LOC_COUNT of k_obs_local, then EB_BLOCKS of k_edotb
+// (fixed upper limits: the static scratch of ovl_observables_noalloc holds them too)
+constexpr int LOC_BLOCKS = 256, EB_BLOCKS = 2048;
+static_assert(LOC_COUNT + 1 == OBS_RAW, "raw observables");
+size_t reduce_partial_len(const Geom &) { return (size_t)LOC_BLOCKS * LOC_COUNT + EB_BLOCKS; }
 
-hipError_t launch_energy(const Geom &g, const double *links, const double *efield, double *partial, double *out,
-                         hipStream_t st)
+hipError_t launch_observables(const Geom &g, const double *links, const double *efield, int what, double *gfield,
+                              double *partial, double *out, hipStream_t st)
 {
-    if (g.nc == 2) k_energy<2><<<RED_BLOCKS, TPB, 0, st>>>(links, efield, partial, g.n0, g.n1, g.n2);
-    else k_energy<3><<<RED_BLOCKS, TPB, 0, st>>>(links, efield, partial, g.n0, g.n1, g.n2);
-    k_finish<2><<<1, TPB, 0, st>>>(partial, RED_BLOCKS, out, 0, 0, 0, 0);
-    return hipGetLastError();
-}
-
-hipError_t launch_gauss(const Geom &g, const double *links, const double *efield, double *partial, double *out,
-                        double *gfield, hipStream_t st)
-{
-    if (g.nc == 2) k_gauss<2><<<RED_BLOCKS, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
-    else k_gauss<3><<<RED_BLOCKS, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
-    k_finish<2><<<1, TPB, 0, st>>>(partial, RED_BLOCKS, out, 1, 0, 0, 0);
+    const int nl = (int)std::min<long>(LOC_BLOCKS, (4L * g.V + TPB - 1) / TPB);
+    const int ne = (int)std::min<long>(EB_BLOCKS, (3L * g.V + 64 / g.nc - 1) / (64 / g.nc));
+    double *pe = partial + (size_t)LOC_BLOCKS * LOC_COUNT;
+    if (what & OBS_EDOTB) {
+        if (g.nc == 2) k_edotb<2><<<ne, EB_TPB, 0, st>>>(links, efield, pe, g.n0, g.n1, g.n2);
+        else k_edotb<3><<<ne, EB_TPB, 0, st>>>(links, efield, pe, g.n0, g.n1, g.n2);
+    }
+    if (what & OBS_LOCAL) {
+        if (g.nc == 2) k_obs_local<2, false><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
+        else k_obs_local<3, false><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
+    } else if (what & OBS_GAUSS) {
+        if (g.nc == 2) k_obs_local<2, true><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
+        else k_obs_local<3, true><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
+    }
+    if (out)
+        k_obs_finish<<<1, TPB, 0, st>>>(partial, what & (OBS_LOCAL | OBS_GAUSS) ? nl : 0, pe, what & OBS_EDOTB ? ne : 0, out);
     return hipGetLastError();
 }
 
@@ -2037,23 +2183,6 @@ hipError_t launch_gauss_restore(const Geom &g, const double *links, const double
     const unsigned nb = nblocks(3L * g.V);
     if (g.nc == 2) k_gauss_restore<2><<<nb, TPB, 0, st>>>(links, gfield, efield, gamma, g.n0, g.n1, g.n2);
     else k_gauss_restore<3><<<nb, TPB, 0, st>>>(links, gfield, efield, gamma, g.n0, g.n1, g.n2);
-    return hipGetLastError();
-}
-
-hipError_t launch_unitarity(const Geom &g, const double *links, double *partial, double *out, hipStream_t st)
-{
-    if (g.nc == 2) k_unitarity<2><<<RED_BLOCKS, TPB, 0, st>>>(links, partial, g.V);
-    else k_unitarity<3><<<RED_BLOCKS, TPB, 0, st>>>(links, partial, g.V);
-    k_finish<2><<<1, TPB, 0, st>>>(partial, RED_BLOCKS, out, 1, 0, 0, 0);
-    return hipGetLastError();
-}
-
-hipError_t launch_edotb(const Geom &g, const double *links, const double *efield, double *partial, double *out,
-                        hipStream_t st)
-{
-    if (g.nc == 2) k_edotb<2><<<RED_BLOCKS, TPB, 0, st>>>(links, efield, partial, g.n0, g.n1, g.n2);
-    else k_edotb<3><<<RED_BLOCKS, TPB, 0, st>>>(links, efield, partial, g.n0, g.n1, g.n2);
-    k_finish<1><<<1, TPB, 0, st>>>(partial, RED_BLOCKS, out, 0, 0, 0, 0);
     return hipGetLastError();
 }
 
