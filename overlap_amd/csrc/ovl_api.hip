@@ -1394,33 +1394,29 @@ static int ctx_init(ovl_ctx *c)
         }
     }
     if (c->ensemble) {
-        // Work table of the ensemble stencil: the hardware hands workgroup b to XCD b % 8, so
-        // placing a system's workgroups at b = k + 8 j keeps the whole system (and the L2 reuse
-        // of its neighbour loads) on XCD k.  Systems go largest first to the least loaded XCD;
-        // shorter XCD lists are padded with idle entries.
+        // Work table of the ensemble stencil: the hardware hands workgroup b to XCD b % 8, so the
+        // workgroups at b = k + 8 j are XCD k's.  All systems' workgroups in order (system by system, each
+        // block-major with z slowest) are cut into eight equal runs, one per XCD: a system is spread over
+        // the XCDs it takes to keep them even, and a cut costs the two z planes on either side of it a
+        // second fetch.  (Whole systems per XCD leave the XCDs uneven whenever one system is more than an
+        // eighth of the work: six SU(2) systems of 8^3 to 20^3 with 32 modes, 47% of them in one, ran
+        // 105 ms per mixed step that way and 43 ms cut; 32 systems of 12^3 to 24^3, which
+        // whole systems balance to 1.7%, 368 and 367 ms.)
         const int ns = nsys(c);
-        std::vector<long> wg(ns);
-        std::vector<int> idx(ns);
+        std::vector<int2> tiles;
         for (int s = 0; s < ns; ++s) {
             const SysDesc &d = c->sys[s];
-            wg[s] = ((long)d.V * d.nblk * mb + ovl::STENCIL_TPB - 1) / ovl::STENCIL_TPB;
-            idx[s] = s;
+            const long wg = ((long)d.V * d.nblk * mb + ovl::STENCIL_TPB - 1) / ovl::STENCIL_TPB;
+            if ((long)tiles.size() + wg > (1L << 30)) return fail(c, OVL_E_ARG, "ensemble too large for one launch");
+            for (long j = 0; j < wg; ++j) tiles.push_back(make_int2(s, (int)j));
         }
-        std::stable_sort(idx.begin(), idx.end(), [&](int x, int y) { return wg[x] > wg[y]; });
-        std::vector<std::vector<int2>> bins(ovl::NUM_XCD);
-        std::vector<long> load(ovl::NUM_XCD, 0);
-        for (int s : idx) {
-            const int k = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-            for (long j = 0; j < wg[s]; ++j) bins[k].push_back(make_int2(s, (int)j));
-            load[k] += wg[s];
-        }
-        const long lmax = *std::max_element(load.begin(), load.end());
-        long ltot = 0;
-        for (long l : load) ltot += l;
-        if ((long)ovl::NUM_XCD * lmax > (1L << 30)) return fail(c, OVL_E_ARG, "ensemble too large for one launch");
+        const long ltot = (long)tiles.size(), lmax = (ltot + ovl::NUM_XCD - 1) / ovl::NUM_XCD;
+        std::vector<int> qoff(ovl::NUM_XCD + 1, 0);
         std::vector<int2> tab((size_t)ovl::NUM_XCD * lmax, make_int2(-1, 0));
-        for (int k = 0; k < ovl::NUM_XCD; ++k)
-            for (size_t j = 0; j < bins[k].size(); ++j) tab[(size_t)k + ovl::NUM_XCD * j] = bins[k][j];
+        for (int k = 0; k < ovl::NUM_XCD; ++k) {
+            qoff[k + 1] = (int)(ltot * (k + 1) / ovl::NUM_XCD);
+            for (int j = qoff[k]; j < qoff[k + 1]; ++j) tab[(size_t)k + ovl::NUM_XCD * (size_t)(j - qoff[k])] = tiles[j];
+        }
         c->ens_grid = (int)tab.size();
         c->ens_imbalance = (double)lmax * ovl::NUM_XCD / (double)ltot;
         RETCHK(dalloc(c, (void **)&c->d_work, sizeof(int2) * tab.size()));
@@ -1432,17 +1428,10 @@ static int ctx_init(ovl_ctx *c)
         }
         HIPCHK(c, hipMemcpy(c->d_work, tab.data(), sizeof(int2) * tab.size(), hipMemcpyHostToDevice));
         // the work queues: the same tiles, XCD k's in one run
-        std::vector<int2> qw;
-        std::vector<int> qoff(ovl::NUM_XCD + 1, 0);
-        for (int k = 0; k < ovl::NUM_XCD; ++k) {
-            qoff[k] = (int)qw.size();
-            qw.insert(qw.end(), bins[k].begin(), bins[k].end());
-        }
-        qoff[ovl::NUM_XCD] = (int)qw.size();
-        RETCHK(dalloc(c, (void **)&c->d_qwork, sizeof(int2) * std::max<size_t>(1, qw.size())));
+        RETCHK(dalloc(c, (void **)&c->d_qwork, sizeof(int2) * tiles.size()));
         RETCHK(dalloc(c, (void **)&c->d_qoff, sizeof(int) * qoff.size()));
         RETCHK(dalloc(c, (void **)&c->d_qctr, sizeof(int) * 2 * ovl::NUM_XCD));
-        HIPCHK(c, hipMemcpy(c->d_qwork, qw.data(), sizeof(int2) * qw.size(), hipMemcpyHostToDevice));
+        HIPCHK(c, hipMemcpy(c->d_qwork, tiles.data(), sizeof(int2) * tiles.size(), hipMemcpyHostToDevice));
         HIPCHK(c, hipMemcpy(c->d_qoff, qoff.data(), sizeof(int) * qoff.size(), hipMemcpyHostToDevice));
         HIPCHK(c, hipMemset(c->d_qctr, 0, sizeof(int) * 2 * ovl::NUM_XCD));
         HIPCHK(c, hipMemcpy(c->d_sys, c->sys.data(), sizeof(SysDesc) * c->sys.size(), hipMemcpyHostToDevice));
