@@ -104,7 +104,10 @@ struct ovl_ctx {
     bool order_set[NUM_PREC] = {false, false, false, false};
     int trav[NUM_PREC] = {ovl::TRAV_LEX, ovl::TRAV_LEX, ovl::TRAV_LEX, ovl::TRAV_LEX};  // lane traversal
     int slabs[NUM_PREC] = {1, 1, 1, 1};         // y slabs (TRAV_MODES) or sub-slabs per box (TRAV_BOXES)
-    int nt_out[NUM_PREC] = {0, 0, 0, 0};        // streaming output stores
+    // streaming output stores: on from the start in FP64, where they leave the L2 to the neighbours (24^3
+    // SU(3), 64 modes, one Clenshaw step 272 -> 236 us; 16^3 SU(2) 53 -> 51); FP32 loses 1% with them
+    // and the other two do not care
+    int nt_out[NUM_PREC] = {1, 0, 0, 0};
     int wpe[NUM_PREC] = {1, 1, 1, 1};           // occupancy variant
     bool tuned = false;                         // ovl_set_tuning or ovl_autotune has run
     double step_xmax = 0.0;  // bound of the mode norms during ovl_fermion_update (FP16 scales)
@@ -1442,8 +1445,13 @@ static int ctx_init(ovl_ctx *c)
 
 static int pick_mode_block(int mode_block, int n_modes)
 {
+    // the smallest padding, and of equal paddings the larger block: 33 to 63 modes fill two blocks of 32
+    // with as many slots as one of 64, whose sites read their links through scalar loads (40 modes of
+    // 11 x 14 x 9 SU(3), one Clenshaw step: 46.8 / 36.8 / 25.4 / 19.9 us in FP64 / 48-bit / FP32 / FP16
+    // against 53.2 / 43.3 / 26.7 / 20.5); up to 32 modes a block of 64 would be half empty (32 modes of
+    // 24^3 SU(3): 270 us against 156 in FP64)
     if (mode_block > 0) return mode_block;
-    return n_modes >= 64 ? 64 : (n_modes > 16 ? 32 : 16);
+    return n_modes > 32 ? 64 : (n_modes > 16 ? 32 : 16);
 }
 
 // mode_block = -1: each block size (16, 32, 64 modes; not one whose padding would double the lanes)
