@@ -7,7 +7,7 @@ import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 LIB = os.path.join(HERE, "libovl.so")
-SOURCES = [os.path.join(HERE, "csrc", f) for f in ("ovl_kernels.hip", "ovl_solvers.hip", "ovl_api.hip")]
+SOURCES = [os.path.join(HERE, "csrc", f) for f in ("ovl_kernels.hip", "ovl_solvers.hip", "ovl_hostcopy.cpp", "ovl_api.hip")]
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
          # keep hipcc from forming packed FP32 instructions
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]

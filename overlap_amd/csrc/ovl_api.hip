@@ -2,6 +2,7 @@
 // leapfrog.  Scalar recurrences (Clenshaw coefficients, multi-shift CG and Ritz scalars) run on
 // the host in FP64; every vector operation runs in the gfx950 kernels of ovl_kernels.hip.
 #include "../../include/ovl.h"
+#include "ovl_hostcopy.hpp"
 #include "ovl_internal.hpp"
 
 #include <hip/hip_runtime.h>
@@ -122,6 +123,7 @@ struct ovl_ctx {
     double *jv = nullptr, *ja = nullptr;
     double *staging = nullptr;
     size_t staging_bytes = 0;
+    bool holds_copies = false;  // this context counts as a holder of the host copy ring
 
     // multi-shift CG of the mode-block fields
     void *ms_ps = nullptr, *ms_r = nullptr, *ms_q = nullptr, *ms_w = nullptr, *ms_chi = nullptr;
@@ -1350,6 +1352,8 @@ int ovl_device_name(char *buf, int len)
 // c->link_sites are filled in.  On failure the caller destroys c.
 static int ctx_init(ovl_ctx *c)
 {
+    ovl::hostcopy_hold();
+    c->holds_copies = true;
     const int mb = c->g.mb, nc = c->g.nc;
     c->ncomp = 4 * nc;
     c->blk64_elems = (size_t)c->g.V * c->ncomp * mb;
@@ -1659,6 +1663,7 @@ int ovl_destroy(ovl_ctx *c)
     if (c->step_exec) hipGraphExecDestroy(c->step_exec);
     for (void *p : ps)
         if (p) hipFree(p);
+    if (c->holds_copies) ovl::hostcopy_release();
     for (auto e : c->evpool) hipEventDestroy(e);
     if (c->t0) hipEventDestroy(c->t0);
     if (c->t1) hipEventDestroy(c->t1);
@@ -1685,13 +1690,6 @@ static int stage(ovl_ctx *c, size_t bytes)
     return OVL_OK;
 }
 
-static bool all_finite(const double *p, size_t n)
-{
-    for (size_t i = 0; i < n; ++i)
-        if (!std::isfinite(p[i])) return false;
-    return true;
-}
-
 // *ok = no Inf/NaN among the n doubles at device address x, nor at y when given (one streaming
 // reduction over both, then a synchronisation)
 static int device_finite(ovl_ctx *c, const void *x, const void *y, long n, bool *ok)
@@ -1712,19 +1710,40 @@ static void refresh_links_set(ovl_ctx *c)
     for (char f : c->sys_links_set) c->links_set = c->links_set && f;
 }
 
-// host <-> device copies of `n` doubles at device offset `off` (elements)
+// Uploads are checked for Inf/NaN before they reach a field: up to HOST_SCAN doubles by a scan on the host,
+// larger ones in the staging buffer by a streaming pass on the device (about 50 us with its
+// synchronisation, as long as the host takes for 256 KB; a host scan of a 24^3 SU(3) mode costs more than
+// its copy).
+constexpr size_t HOST_SCAN = 32768;
+static bool all_finite(const double *p, size_t n)
+{
+    for (size_t i = 0; i < n; ++i)
+        if (!std::isfinite(p[i])) return false;
+    return true;
+}
+
+// host <-> device copies of `n` doubles
 static int put_doubles(ovl_ctx *c, double *dst, const double *src, size_t n, const char *what)
 {
-    if (!all_finite(src, n)) return fail(c, OVL_E_ARG, std::string("non-finite ") + what);
-    HIPCHK(c, hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, c->st));
+    bool ok = true;
+    if (n <= HOST_SCAN) {
+        if (!all_finite(src, n)) return fail(c, OVL_E_ARG, std::string("non-finite ") + what);
+        HIPCHK(c, hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, c->st));
+        HIPCHK(c, hipStreamSynchronize(c->st));
+        return OVL_OK;
+    }
+    RETCHK(stage(c, n * sizeof(double)));
+    HIPCHK(c, hipMemcpyAsync(c->staging, src, n * sizeof(double), hipMemcpyHostToDevice, c->st));
+    RETCHK(device_finite(c, c->staging, nullptr, (long)n, &ok));
+    if (!ok) return fail(c, OVL_E_ARG, std::string("non-finite ") + what);
+    HIPCHK(c, hipMemcpyAsync(dst, c->staging, n * sizeof(double), hipMemcpyDeviceToDevice, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
     return OVL_OK;
 }
 
 static int get_doubles(ovl_ctx *c, double *dst, const double *src, size_t n)
 {
-    HIPCHK(c, hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
+    HIPCHK(c, ovl::copy_to_host(dst, src, n * sizeof(double), c->st));
     return OVL_OK;
 }
 
@@ -1861,14 +1880,16 @@ static int modes_io(ovl_ctx *c, int sys, int field, double *aos, int first, int 
     const size_t n = (size_t)count * g.V * c->ncomp * 2;
     RETCHK(stage(c, n * sizeof(double)));
     if (upload) {
-        if (!all_finite(aos, n)) return fail(c, OVL_E_ARG, "non-finite spinor component");
-        HIPCHK(c, hipMemcpyAsync(c->staging, aos, n * sizeof(double), hipMemcpyHostToDevice, c->st));
+        bool ok = n > HOST_SCAN || all_finite(aos, n);
+        if (ok) HIPCHK(c, hipMemcpyAsync(c->staging, aos, n * sizeof(double), hipMemcpyHostToDevice, c->st));
+        if (n > HOST_SCAN) RETCHK(device_finite(c, c->staging, nullptr, (long)n, &ok));
+        if (!ok) return fail(c, OVL_E_ARG, "non-finite spinor component");
         HIPCHK(c, ovl::launch_aos_to_soa(g, c->staging, first, count, f, c->st));
+        HIPCHK(c, hipStreamSynchronize(c->st));
     } else {
         HIPCHK(c, ovl::launch_soa_to_aos(g, f, first, count, c->staging, c->st));
-        HIPCHK(c, hipMemcpyAsync(aos, c->staging, n * sizeof(double), hipMemcpyDeviceToHost, c->st));
+        HIPCHK(c, ovl::copy_to_host(aos, c->staging, n * sizeof(double), c->st));
     }
-    HIPCHK(c, hipStreamSynchronize(c->st));
     return OVL_OK;
 }
 
@@ -2061,8 +2082,7 @@ static int dropin_result(ovl_ctx *c, const void *in, double sh_i, const void *x,
     void *out = (char *)c->s1_vec + vec1_bytes(c);
     HIPCHK(c, ovl::launch_hop1(c->g, amass(c), in, out, c->s1_links, 0.0, sh_i, x, 0.0, sx_i, 1, c->st));
     HIPCHK(c, ovl::launch_vec1_out(c->g, out, c->staging, c->st));
-    HIPCHK(c, hipMemcpyAsync(psi, c->staging, vec1_bytes(c), hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
+    HIPCHK(c, ovl::copy_to_host(psi, c->staging, vec1_bytes(c), c->st));
     return OVL_OK;
 }
 

@@ -1,0 +1,22 @@
+// Copies from device memory to pageable host arrays (the C ABI's borrowed result pointers).
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include <cstddef>
+
+namespace ovl {
+
+// Ordered after the work queued on `st`; returns when the copy is complete.  Arrays of at least HOSTCOPY_MIN
+// bytes whose pages do not exist yet go through a ring of pinned buffers that a few host threads empty
+// while the DMA engine fills the next ones; all others, and copies that find the ring in use by another
+// host thread, are a plain hipMemcpyAsync and a synchronisation.
+hipError_t copy_to_host(void *host, const void *dev, size_t bytes, hipStream_t st);
+
+// The ring and its threads belong to the process: made by the first copy that wants them, given back when
+// the last holder lets go (every context holds it from its creation to its end).
+void hostcopy_hold();
+void hostcopy_release();
+
+constexpr size_t HOSTCOPY_MIN = (size_t)1 << 20;
+
+}  // namespace ovl
