@@ -99,7 +99,8 @@ struct ovl_ctx {
     // reductions / small scratch
     double *partial = nullptr;
     size_t partial_len = 0;
-    bool boxes_ok = false;     // the lattice splits into 8 equal boxes (TRAV_BOXES possible)
+    bool boxes_ok = false;     // the lattice splits into 8 equal boxes (TRAV_BOXES possible): `box`
+    ovl::XcdBoxes box{};
     // per input precision (P64, P32, P16, P48) of the stencil, set by ovl_autotune:
     int *order[NUM_PREC] = {nullptr, nullptr, nullptr, nullptr};  // device site order (null: lexicographic)
     bool order_set[NUM_PREC] = {false, false, false, false};
@@ -360,6 +361,7 @@ HopArgs hop_args(const ovl_ctx *c, int prec)
     a.trav = c->trav[prec];
     a.nt_out = c->nt_out[prec];
     a.order = c->order[prec];
+    if (c->boxes_ok) a.box = c->box;
     if (c->ensemble) {
         a.trav = c->trav[prec] == ovl::TRAV_QUEUE ? ovl::TRAV_QUEUE : ovl::TRAV_LEX;
         a.order = nullptr;
@@ -377,44 +379,46 @@ HopArgs hop_args(const ovl_ctx *c, int prec)
 }
 
 // Site traversal for the XCD-aware stencil launches: the lattice is cut into 8 boxes (one per XCD,
-// px*py*pz = 8 dividing the extents); inside a box the shorter of the y/z box extents is cut into
-// `sub` slabs, each walked with x fastest, then that extent, then the other one, so the three
-// planes a site's neighbours span (b_x * slab sites each) fit the XCD's L2.  Empty when no split fits.
-std::vector<int> xcd_site_order(int n0, int n1, int n2, int sub = 1)
+// px*py*pz = 8 dividing the extents, the split of the smallest box surface); inside a box the shorter of
+// the y/z box extents is cut into `sub` slabs, each walked with x fastest, then that extent, then the
+// other one, so the three planes a site's neighbours span (b_x * slab sites each) fit the XCD's L2.
+// Whole boxes (sub = 1) are computed by the kernel from `box`; slabs have a table.
+bool xcd_boxes(int n0, int n1, int n2, ovl::XcdBoxes *out)
 {
-    const int n[3] = {n0, n1, n2};
-    int best[3] = {0, 0, 0};
     long best_cost = -1;
-    for (int px = 1; px <= 8; px *= 2)
-        for (int py = 1; px * py <= 8; py *= 2) {
-            const int pz = 8 / (px * py);
+    for (int lx = 0; lx <= 3; ++lx)
+        for (int ly = 0; lx + ly <= 3; ++ly) {
+            const int px = 1 << lx, py = 1 << ly, pz = 8 >> (lx + ly);
             if (n0 % px || n1 % py || n2 % pz) continue;
-            // prefer compact boxes: minimise the box surface
             const long bx = n0 / px, by = n1 / py, bz = n2 / pz;
             const long cost = bx * by + by * bz + bz * bx;
-            if (best_cost < 0 || cost < best_cost) {
-                best_cost = cost;
-                best[0] = px; best[1] = py; best[2] = pz;
-            }
+            if (best_cost >= 0 && cost >= best_cost) continue;
+            best_cost = cost;
+            const bool y_mid = by <= bz;
+            *out = ovl::XcdBoxes{lx, ly, (int)by, (int)bz, y_mid, ovl::make_fastdiv((unsigned)bx),
+                                 ovl::make_fastdiv((unsigned)(bx * (y_mid ? by : bz)))};
         }
+    return best_cost >= 0;
+}
+
+std::vector<int> xcd_site_order(int n0, int n1, int n2, int sub)
+{
     std::vector<int> order;
-    if (best_cost < 0) return order;
-    const int b[3] = {n[0] / best[0], n[1] / best[1], n[2] / best[2]};
-    const bool y_mid = b[1] <= b[2];
-    const int slow = y_mid ? b[2] : b[1], mid = y_mid ? b[1] : b[2];
+    ovl::XcdBoxes q;
+    if (!xcd_boxes(n0, n1, n2, &q)) return order;
+    const int bx = (int)q.dv_x.d, slow = q.y_mid ? q.bz : q.by, mid = q.y_mid ? q.by : q.bz;
     sub = std::max(1, std::min(sub, mid));
     order.reserve((size_t)n0 * n1 * n2);
-    for (int kz = 0; kz < best[2]; ++kz)
-        for (int ky = 0; ky < best[1]; ++ky)
-            for (int kx = 0; kx < best[0]; ++kx)
-                for (int t = 0; t < sub; ++t)
-                    for (int i = 0; i < slow; ++i)
-                        for (int j = t * mid / sub; j < (t + 1) * mid / sub; ++j)
-                            for (int x = 0; x < b[0]; ++x) {
-                                const int y = y_mid ? j : i, z = y_mid ? i : j;
-                                const int gx = kx * b[0] + x, gy = ky * b[1] + y, gz = kz * b[2] + z;
-                                order.push_back(gx + n0 * (gy + n1 * gz));
-                            }
+    for (int k = 0; k < ovl::NUM_XCD; ++k) {
+        const int kx = k & ((1 << q.lx) - 1), ky = (k >> q.lx) & ((1 << q.ly) - 1), kz = k >> (q.lx + q.ly);
+        for (int t = 0; t < sub; ++t)
+            for (int i = 0; i < slow; ++i)
+                for (int j = t * mid / sub; j < (t + 1) * mid / sub; ++j)
+                    for (int x = 0; x < bx; ++x) {
+                        const int y = q.y_mid ? j : i, z = q.y_mid ? i : j;
+                        order.push_back(kx * bx + x + n0 * (ky * q.by + y + n1 * (kz * q.bz + z)));
+                    }
+    }
     return order;
 }
 
@@ -467,7 +471,7 @@ int set_traversal(ovl_ctx *c, int prec, int trav, int slabs)
     c->slabs[prec] = slabs;
     c->order_set[prec] = true;
     std::vector<int> ord;
-    if (trav == ovl::TRAV_BOXES) ord = xcd_site_order(c->g.n0, c->g.n1, c->g.n2, slabs);
+    if (trav == ovl::TRAV_BOXES && slabs > 1) ord = xcd_site_order(c->g.n0, c->g.n1, c->g.n2, slabs);
     else if (trav == ovl::TRAV_MODES && slabs > 1) ord = slab_site_order(c->g.n0, c->g.n1, c->g.n2, slabs);
     if (ord.empty()) return OVL_OK;
     RETCHK(dalloc(c, (void **)&c->order[prec], sizeof(int) * ord.size()));
@@ -1388,7 +1392,7 @@ static int ctx_init(ovl_ctx *c)
     RETCHK(dalloc(c, (void **)&c->partial, sizeof(double) * c->partial_len));
     RETCHK(dalloc(c, (void **)&c->dout, sizeof(double) * (16 + 2 * (size_t)maxblk * mb)));
     if (!c->ensemble && (c->prm.traversal == 0 || c->prm.traversal == 2))
-        c->boxes_ok = !xcd_site_order(c->g.n0, c->g.n1, c->g.n2).empty();
+        c->boxes_ok = xcd_boxes(c->g.n0, c->g.n1, c->g.n2, &c->box);
     if (!c->ensemble) {
         // traversal 0 (automatic): mode split where the mode blocks divide over the XCDs, else
         // boxes; ovl_autotune may change it
@@ -1711,10 +1715,10 @@ static void refresh_links_set(ovl_ctx *c)
 }
 
 // Uploads are checked for Inf/NaN before they reach a field: up to HOST_SCAN doubles by a scan on the host,
-// larger ones in the staging buffer by a streaming pass on the device (about 50 us with its
-// synchronisation, as long as the host takes for 256 KB; a host scan of a 24^3 SU(3) mode costs more than
+// larger ones in the staging buffer by a streaming pass on the device (about 100 us with its
+// synchronisation, as long as the host takes for 1 MB or two; a host scan of a 24^3 SU(3) mode costs more than
 // its copy).
-constexpr size_t HOST_SCAN = 32768;
+constexpr size_t HOST_SCAN = 262144;
 static bool all_finite(const double *p, size_t n)
 {
     for (size_t i = 0; i < n; ++i)

@@ -56,6 +56,14 @@ struct Geom {
     int nblk;    // mode blocks held per field
 };
 
+// the eight XCD boxes of a lattice: 2^lx x 2^ly x 2^lz of them (lx + ly + lz = 3), each walked x fastest, then
+// the shorter of its y and z extents (y_mid: y), then the other; dv_x: box extent in x, dv_plane: sites
+// of a plane (x, mid)
+struct XcdBoxes {
+    int lx, ly, by, bz, y_mid;
+    FastDiv dv_x, dv_plane;
+};
+
 // pointwise epilogue of the stencil kernel:
 //   out = sh * h_W(in) + sx * G(x) + s1 * b1 + s2 * b2 + st * tgt      (G = 1 or gamma0)
 // the five operands are block-relative pointers (already offset to the first block launched);
@@ -76,8 +84,9 @@ struct HopArgs {
     double out2_scale;
     int nblk;         // blocks covered by this launch
     int trav;         // lane traversal, TRAV_* (falls back to TRAV_LEX where the launch does not split evenly)
-    const int *order; // TRAV_BOXES: XCD k's box is order[k V/8 .. (k+1) V/8); TRAV_MODES: site order
-                      // inside a mode block (null = lexicographic)
+    const int *order; // TRAV_BOXES: XCD k's box is order[k V/8 .. (k+1) V/8) (null = `box`, computed);
+                      // TRAV_MODES: site order inside a mode block (null = lexicographic)
+    XcdBoxes box;     // TRAV_BOXES without a table
     // ensemble launch (null = one lattice): system table and per-workgroup work table
     // (int2 {system, workgroup within the system}, system -1 = idle), ens_grid workgroups
     const SysDesc *ens_sys;

@@ -307,8 +307,11 @@ __device__ __forceinline__ unsigned fdiv(unsigned n, const FastDiv &f)
     return f.d <= 1 ? n : (__umulhi(n, f.mul) >> f.shift);
 }
 
+struct Site {
+    int s, x, y, z;
+};
 template <int MB>
-__device__ __forceinline__ bool lane_coords(const HopArgs &a, int V, int &m, int &s, int &blk)
+__device__ __forceinline__ bool lane_coords(const HopArgs &a, int n0, int n1, int V, int &m, Site &p, int &blk)
 {
     const unsigned total = (unsigned)a.nblk * (unsigned)V * MB;  // < 2^31, checked by the launcher
     unsigned lb = blockIdx.x;
@@ -318,18 +321,39 @@ __device__ __forceinline__ bool lane_coords(const HopArgs &a, int V, int &m, int
     m = (int)(gl % MB);
     unsigned r = gl / MB;
     if constexpr (MB == 64) r = __builtin_amdgcn_readfirstlane(r);  // one site per wavefront
+    int s;
     if (a.trav == TRAV_BOXES) {
         const unsigned xc = fdiv(r, a.dv_per);  // XCD of the traversal slot (nblk V / 8 slots each)
         const unsigned rr = r - xc * a.dv_per.d;
         const unsigned b = fdiv(rr, a.dv_v8);
+        const unsigned i = rr - b * a.dv_v8.d;
         blk = (int)b;
-        s = a.order[xc * a.dv_v8.d + (rr - b * a.dv_v8.d)];
+        if (!a.order) {
+            // whole boxes: the site follows from the slot (no table to read before the first load: 1 to 1.5 us
+            // of every launch's chain)
+            const unsigned slow = fdiv(i, a.box.dv_plane), ip = i - slow * a.box.dv_plane.d;
+            const unsigned mid = fdiv(ip, a.box.dv_x);
+            const unsigned kx = xc & ((1u << a.box.lx) - 1), ky = (xc >> a.box.lx) & ((1u << a.box.ly) - 1);
+            const unsigned kz = xc >> (a.box.lx + a.box.ly);
+            p.x = (int)(kx * a.box.dv_x.d + (ip - mid * a.box.dv_x.d));
+            p.y = (int)(ky * a.box.by + (a.box.y_mid ? mid : slow));
+            p.z = (int)(kz * a.box.bz + (a.box.y_mid ? slow : mid));
+            p.s = p.x + n0 * (p.y + n1 * p.z);
+            return true;
+        }
+        s = a.order[xc * a.dv_v8.d + i];
     } else {
         const unsigned b = fdiv(r, a.dv_V);
         const unsigned i = r - b * (unsigned)V;
         blk = (int)b;
         s = (a.trav == TRAV_MODES && a.order) ? a.order[i] : (int)i;
     }
+    if constexpr (MB == 64) s = __builtin_amdgcn_readfirstlane(s);
+    p.s = s;
+    p.z = (int)fdiv((unsigned)s, a.dv_n01);
+    const int rem = s - p.z * (int)a.dv_n01.d;
+    p.y = (int)fdiv((unsigned)rem, a.dv_n0);
+    p.x = rem - p.y * n0;
     return true;
 }
 
@@ -437,17 +461,43 @@ __device__ __forceinline__ void hop_dir(const TP *pr, const TP *pi, const LT *__
 // (WilsonOperator.cpp:30-114 computes -i h_W of one mode; here every mode of every block).
 // The site s lives on an n0 x n1 x n2 lattice; its spinors are site-block q0 + s of the fields
 // (q0 = first site-block of this lane's mode block), its links start at site index l0.
-// EPI = false: a pure launch (out = sh h_W(in)); the pointwise operands are then known to be absent
-// at compile time, which frees the registers their arguments would hold
-template <int NC, typename TI, typename TO, int MB, bool EPI = true>
-__device__ __forceinline__ void hop_site(const HopArgs &a, int n0, int n1, int n2, int s, int x, int y, int z, int q0,
-                                         int l0, int m)
+// Kinds of launch, known at compile time so that a launch carries no arguments, tests or products of
+// terms it does not have (a complex factor with a zero part costs two instructions per real part more):
+//   EPI_PURE      out = sh h_W(in), sh real: w of a Clenshaw step
+//   EPI_ANY       every term, each present if its pointer is
+//   EPI_CLENSHAW  out = sh h_W(in) + sx x + s1 b1 + s2 b2, all factors real
+//   EPI_AXPY      out = i sh h_W(in) + tgt: a leapfrog step
+// The products and sums of the last two round as EPI_ANY's do (the zero parts only add zeros).
+enum { EPI_PURE = 0, EPI_ANY = 1, EPI_CLENSHAW = 2, EPI_AXPY = 3 };
+
+// an operand of the epilogue as loaded: FP16 stays in halves until the product widens it
+template <typename T> using OpT = typename std::conditional<std::is_same<T, _Float16>::value, _Float16, typename Vec<T>::C>::type;
+
+// -0 in a register the compiler cannot see through: f * v + (-0) is the rounded product, as one
+// mixed-precision FMA when v is a half (no conversion)
+__device__ __forceinline__ float opaque_minus_zero()
+{
+    float z;
+    asm("s_mov_b32 %0, 0x80000000" : "=s"(z));
+    return z;
+}
+// acc + f * v with two roundings, as the complex form with a zero imaginary factor has
+template <typename T>
+__device__ __forceinline__ typename Vec<T>::C add_scaled(typename Vec<T>::C acc, typename Vec<T>::C f, OpT<T> v, float mz)
+{
+#pragma clang fp contract(off)
+    if constexpr (std::is_same<T, _Float16>::value) return acc + __builtin_fmaf((float)v, f, mz);
+    else return acc + f * v;
+}
+
+template <int NC, typename TI, typename TO, int MB, int EPI = EPI_ANY>
+__device__ __forceinline__ void hop_site(const HopArgs &a, int n0, int n1, int n2, const Site &p, int q0, int l0, int m)
 {
     constexpr int NCOMP = 4 * NC;
     using LT = typename Vec<TI>::L;
     using CI = typename Vec<TI>::C;  // arithmetic type of the stencil
     using CO = typename Vec<TO>::C;  // arithmetic type of the epilogue
-    const int V = n0 * n1 * n2;
+    const int V = n0 * n1 * n2, s = p.s;
 
     const LT *__restrict__ L = reinterpret_cast<const LT *>(a.links) + (size_t)l0 * NC * NC;
     constexpr int NN = NC * NC;
@@ -462,24 +512,24 @@ __device__ __forceinline__ void hop_site(const HopArgs &a, int n0, int n1, int n
     for (int c = 0; c < NCOMP; ++c) { xr[c] = am * (CI)pr[c]; xi[c] = am * (CI)pi[c]; }
 
     {  // x direction
-        const int sp = s + ((x + 1 == n0) ? 1 - n0 : 1);
-        const int sm = s + ((x == 0) ? n0 - 1 : -1);
+        const int sp = s + ((p.x + 1 == n0) ? 1 - n0 : 1);
+        const int sm = s + ((p.x == 0) ? n0 - 1 : -1);
         load_sp<NC, MB, TI>(a.in, 0, 0, q0 + sp, m, pr, pi);
         hop_dir<NC, 0, 1>(pr, pi, L + ((size_t)0 * V + s) * NN, xr, xi);
         load_sp<NC, MB, TI>(a.in, 0, 0, q0 + sm, m, pr, pi);
         hop_dir<NC, 0, -1>(pr, pi, L + ((size_t)0 * V + sm) * NN, xr, xi);
     }
     {  // y direction
-        const int sp = s + ((y + 1 == n1) ? (1 - n1) * n0 : n0);
-        const int sm = s + ((y == 0) ? (n1 - 1) * n0 : -n0);
+        const int sp = s + ((p.y + 1 == n1) ? (1 - n1) * n0 : n0);
+        const int sm = s + ((p.y == 0) ? (n1 - 1) * n0 : -n0);
         load_sp<NC, MB, TI>(a.in, 0, 0, q0 + sp, m, pr, pi);
         hop_dir<NC, 1, 1>(pr, pi, L + ((size_t)1 * V + s) * NN, xr, xi);
         load_sp<NC, MB, TI>(a.in, 0, 0, q0 + sm, m, pr, pi);
         hop_dir<NC, 1, -1>(pr, pi, L + ((size_t)1 * V + sm) * NN, xr, xi);
     }
     {  // z direction
-        const int sp = s + ((z + 1 == n2) ? (1 - n2) * n0 * n1 : n0 * n1);
-        const int sm = s + ((z == 0) ? (n2 - 1) * n0 * n1 : -n0 * n1);
+        const int sp = s + ((p.z + 1 == n2) ? (1 - n2) * n0 * n1 : n0 * n1);
+        const int sm = s + ((p.z == 0) ? (n2 - 1) * n0 * n1 : -n0 * n1);
         load_sp<NC, MB, TI>(a.in, 0, 0, q0 + sp, m, pr, pi);
         hop_dir<NC, 2, 1>(pr, pi, L + ((size_t)2 * V + s) * NN, xr, xi);
         load_sp<NC, MB, TI>(a.in, 0, 0, q0 + sm, m, pr, pi);
@@ -487,7 +537,45 @@ __device__ __forceinline__ void hop_site(const HopArgs &a, int n0, int n1, int n
     }
 
     // h_W = (1/2) gamma0 X, then the epilogue in the output precision
+    const int q = q0 + s;
     CO orr[NCOMP], oi[NCOMP];
+    if constexpr (EPI == EPI_PURE || EPI == EPI_CLENSHAW) {
+        const CO f = (CO)0.5 * (CO)a.sh_r;
+#pragma unroll
+        for (int c = 0; c < NCOMP; ++c) {
+            const CO g = (c < 2 * NC) ? f : -f;
+            orr[c] = g * (CO)xr[c];
+            oi[c] = g * (CO)xi[c];
+        }
+    }
+    if constexpr (EPI == EPI_CLENSHAW) {
+        OpT<TO> tr[NCOMP], ti[NCOMP];
+        const float mz = std::is_same<TO, _Float16>::value ? opaque_minus_zero() : -0.0f;
+        auto term = [&](const void *v, double factor) {
+            load_sp_nt<NC, MB, TO>(v, 0, 0, q, m, tr, ti);
+            const CO f = (CO)factor;
+#pragma unroll
+            for (int c = 0; c < NCOMP; ++c) {
+                orr[c] = add_scaled<TO>(orr[c], f, tr[c], mz);
+                oi[c] = add_scaled<TO>(oi[c], f, ti[c], mz);
+            }
+        };
+        term(a.x, a.sx_r);
+        term(a.b1, a.s1_r);
+        term(a.b2, a.s2_r);
+    }
+    if constexpr (EPI == EPI_AXPY) {
+        CO tr[NCOMP], ti[NCOMP];
+        load_sp_nt<NC, MB, TO>(a.tgt, 0, 0, q, m, tr, ti);
+        const CO f = (CO)0.5 * (CO)a.sh_i;
+#pragma unroll
+        for (int c = 0; c < NCOMP; ++c) {
+            const CO g = (c < 2 * NC) ? f : -f;
+            orr[c] = add_scaled<TO>(tr[c], -g, (CO)xi[c], -0.0f);
+            oi[c] = add_scaled<TO>(ti[c], g, (CO)xr[c], -0.0f);
+        }
+    }
+    if constexpr (EPI == EPI_ANY) {
     const CO shr = (CO)a.sh_r, shi = (CO)a.sh_i;
 #pragma unroll
     for (int c = 0; c < NCOMP; ++c) {
@@ -496,8 +584,6 @@ __device__ __forceinline__ void hop_site(const HopArgs &a, int n0, int n1, int n
         orr[c] = shr * hr - shi * hi;
         oi[c] = shr * hi + shi * hr;
     }
-    const int q = q0 + s;
-    if constexpr (EPI) {
     CO tr[NCOMP], ti[NCOMP];
     if (a.x) {
         load_sp_nt<NC, MB, TO>(a.x, 0, 0, q, m, tr, ti);
@@ -537,38 +623,31 @@ __device__ __forceinline__ void hop_site(const HopArgs &a, int n0, int n1, int n
     }
     }
     // the pure launch's output w is an intermediate of the step: 48-bit storage truncates it
-    if (a.nt_out) store_sp_nt<NC, MB, TO, !EPI>(a.out, 0, 0, q, m, orr, oi);
-    else store_sp<NC, MB, TO, !EPI>(a.out, 0, 0, q, m, orr, oi);
+    constexpr bool TRUNC = EPI == EPI_PURE;
+    if (a.nt_out) store_sp_nt<NC, MB, TO, TRUNC>(a.out, 0, 0, q, m, orr, oi);
+    else store_sp<NC, MB, TO, TRUNC>(a.out, 0, 0, q, m, orr, oi);
 }
 
 // WPE: minimum waves per SIMD the register allocation must allow (1 = compiler's choice); the
 // stencil hoists its neighbour loads, so this trades memory-level parallelism per wave against
 // waves in flight.  The host picks the variant per problem shape (autotune).
-template <int NC, typename TI, typename TO, int MB, int WPE, bool EPI>
+template <int NC, typename TI, typename TO, int MB, int WPE, int EPI>
 __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(WPE))) void k_hop(HopArgs a, int n0, int n1,
                                                                                        int n2)
 {
     const int V = n0 * n1 * n2;
-    int m, s, blk;
-    if (!lane_coords<MB>(a, V, m, s, blk)) return;
-    if constexpr (MB == 64) {
-        // one site per wavefront: make the site wave-uniform so that the links (shared by all
-        // modes of the site) come through scalar loads instead of 64 identical vector lanes
-        s = __builtin_amdgcn_readfirstlane(s);
-        blk = __builtin_amdgcn_readfirstlane(blk);
-    }
-    // site coordinates (s = x + n0 (y + n1 z))
-    const int z = (int)fdiv((unsigned)s, a.dv_n01);
-    const int rem = s - z * (int)a.dv_n01.d;
-    const int y = (int)fdiv((unsigned)rem, a.dv_n0);
-    const int x = rem - y * n0;
-    hop_site<NC, TI, TO, MB, EPI>(a, n0, n1, n2, s, x, y, z, blk * V, 0, m);
+    int m, blk;
+    Site p;
+    // 64-mode blocks have one site per wavefront: site and block are wave-uniform there, so that the links
+    // (shared by all modes of the site) come through scalar loads instead of 64 identical vector lanes
+    if (!lane_coords<MB>(a, n0, n1, V, m, p, blk)) return;
+    hop_site<NC, TI, TO, MB, EPI>(a, n0, n1, n2, p, blk * V, 0, m);
 }
 
 // Ensemble launch: many independent lattices of different sizes in one grid.  One tile = TPB lanes
 // of one system: workgroup w.y of system w.x (lanes (site, mode) in block-major order, as k_hop's
 // lexicographic traversal).
-template <int NC, typename TI, typename TO, int MB, bool EPI>
+template <int NC, typename TI, typename TO, int MB, int EPI>
 __device__ __forceinline__ void hop_ens_tile(const HopArgs &a, int2 w)
 {
     const SysDesc d = a.ens_sys[w.x];
@@ -582,7 +661,7 @@ __device__ __forceinline__ void hop_ens_tile(const HopArgs &a, int2 w)
     const int z = (int)fdiv((unsigned)s, d.dv_n01);
     const int rem = s - z * d.n0 * d.n1;
     const int y = (int)fdiv((unsigned)rem, d.dv_n0);
-    hop_site<NC, TI, TO, MB, EPI>(a, d.n0, d.n1, d.n2, s, rem - y * d.n0, y, z, d.q0 + blk * d.V, d.l0, m);
+    hop_site<NC, TI, TO, MB, EPI>(a, d.n0, d.n1, d.n2, Site{s, rem - y * d.n0, y, z}, d.q0 + blk * d.V, d.l0, m);
 }
 
 // Static table (ens_qctr null): workgroup b runs tile ens_work[b]; the host lays the table out so
@@ -591,7 +670,7 @@ __device__ __forceinline__ void hop_ens_tile(const HopArgs &a, int2 w)
 // queue of XCD b % 8 until it is empty, so the tiles of an XCD's systems go to whichever of its
 // workgroups is free.  Every workgroup leaves when its queue is exhausted (no workgroup waits on
 // another); the last one of each queue to leave resets the queue's counters for the next launch.
-template <int NC, typename TI, typename TO, int MB, int WPE, bool EPI>
+template <int NC, typename TI, typename TO, int MB, int WPE, int EPI>
 __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(WPE))) void k_hop_ens(HopArgs a)
 {
     if (!a.ens_qctr) {
@@ -1728,7 +1807,7 @@ hipError_t reserve_lds(const void *kernel)
     return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_ONE_WG);
 }
 
-template <int NC, typename TI, typename TO, int MB, bool EPI>
+template <int NC, typename TI, typename TO, int MB, int EPI>
 void hop_wpe_epi(const HopArgs &b, unsigned nb, int wpe, const Geom &g, hipStream_t st)
 {
     switch (wpe) {
@@ -1743,15 +1822,36 @@ void hop_wpe_epi(const HopArgs &b, unsigned nb, int wpe, const Geom &g, hipStrea
     }
 }
 
+// the kind of launch (EPI_*) that a set of operands and factors is
+int epi_kind(const HopArgs &b)
+{
+    const bool none = !b.x && !b.b1 && !b.b2 && !b.out2;
+    if (none && !b.tgt && b.sh_i == 0.0) return EPI_PURE;
+    if (none && b.tgt && b.sh_r == 0.0 && b.st_r == 1.0 && b.st_i == 0.0) return EPI_AXPY;
+    if (b.x && b.b1 && b.b2 && !b.tgt && !b.out2 && !b.x_gamma0 && b.sh_i == 0.0 && b.sx_i == 0.0 && b.s1_i == 0.0 &&
+        b.s2_i == 0.0)
+        return EPI_CLENSHAW;
+    return EPI_ANY;
+}
+
 template <int NC, typename TI, typename TO, int MB>
 void hop_wpe(const HopArgs &b, unsigned nb, int wpe, const Geom &g, hipStream_t st)
 {
-    // the pure launch of the Clenshaw step (no pointwise operand) has a variant of its own
-    if (b.x || b.b1 || b.b2 || b.tgt || b.out2) hop_wpe_epi<NC, TI, TO, MB, true>(b, nb, wpe, g, st);
-    else hop_wpe_epi<NC, TI, TO, MB, false>(b, nb, wpe, g, st);
+    if constexpr (std::is_same<TI, TO>::value) {
+        switch (epi_kind(b)) {
+        case EPI_PURE: return hop_wpe_epi<NC, TI, TO, MB, EPI_PURE>(b, nb, wpe, g, st);
+        case EPI_CLENSHAW: return hop_wpe_epi<NC, TI, TO, MB, EPI_CLENSHAW>(b, nb, wpe, g, st);
+        case EPI_AXPY:
+            // the leapfrog's fields are FP64 or FP32
+            if constexpr (sizeof(TI) == 8 || sizeof(TI) == 4) return hop_wpe_epi<NC, TI, TO, MB, EPI_AXPY>(b, nb, wpe, g, st);
+            break;
+        default: break;
+        }
+    }
+    hop_wpe_epi<NC, TI, TO, MB, EPI_ANY>(b, nb, wpe, g, st);
 }
 
-template <int NC, typename TI, typename TO, int MB, bool EPI>
+template <int NC, typename TI, typename TO, int MB, int EPI>
 void hop_ens_wpe_epi(const HopArgs &b, int wpe, hipStream_t st)
 {
     unsigned nb = (unsigned)b.ens_grid;
@@ -1783,9 +1883,17 @@ void hop_ens_wpe_epi(const HopArgs &b, int wpe, hipStream_t st)
 template <int NC, typename TI, typename TO, int MB>
 void hop_ens_wpe(const HopArgs &b, int wpe, hipStream_t st)
 {
-    // the pure launch of the Clenshaw step (no pointwise operand) has a variant of its own
-    if (b.x || b.b1 || b.b2 || b.tgt || b.out2) hop_ens_wpe_epi<NC, TI, TO, MB, true>(b, wpe, st);
-    else hop_ens_wpe_epi<NC, TI, TO, MB, false>(b, wpe, st);
+    if constexpr (std::is_same<TI, TO>::value) {
+        switch (epi_kind(b)) {
+        case EPI_PURE: return hop_ens_wpe_epi<NC, TI, TO, MB, EPI_PURE>(b, wpe, st);
+        case EPI_CLENSHAW: return hop_ens_wpe_epi<NC, TI, TO, MB, EPI_CLENSHAW>(b, wpe, st);
+        case EPI_AXPY:
+            if constexpr (sizeof(TI) == 8 || sizeof(TI) == 4) return hop_ens_wpe_epi<NC, TI, TO, MB, EPI_AXPY>(b, wpe, st);
+            break;
+        default: break;
+        }
+    }
+    hop_ens_wpe_epi<NC, TI, TO, MB, EPI_ANY>(b, wpe, st);
 }
 
 template <int NC, typename TI, typename TO>
@@ -1812,7 +1920,7 @@ hipError_t hop_mb(const Geom &g, const HopArgs &a, int wpe, hipStream_t st)
     b.dv_n0 = make_fastdiv((unsigned)g.n0);
     // the XCD traversals need whole workgroups spread evenly over the XCDs
     const bool even = total % ((long)TPB * NUM_XCD) == 0;
-    if (b.trav == TRAV_BOXES && (!even || g.V % NUM_XCD != 0 || !b.order)) b.trav = TRAV_LEX;
+    if (b.trav == TRAV_BOXES && (!even || g.V % NUM_XCD != 0 || (!b.order && b.box.dv_x.d == 0))) b.trav = TRAV_LEX;
     if (b.trav == TRAV_MODES && !even) b.trav = TRAV_LEX;
     switch (g.mb) {
     case 16: hop_wpe<NC, TI, TO, 16>(b, nb, wpe, g, st); break;
