@@ -67,6 +67,10 @@ struct ovl_ctx {
     double *links = nullptr, *efield = nullptr;  // master FP64, reference layout
     double *ul64 = nullptr;                      // stencil links FP64 (double2)
     float *ul32 = nullptr;                       // stencil links FP32 (float2)
+    // the other stencil links of a Wilson leapfrog whose link update shares a launch with the stencil
+    // (allocated on first use; a full step swaps them twice)
+    double *ul64_next = nullptr;
+    float *ul32_next = nullptr;
     double *phase = nullptr;                     // U(1) phases double2[3V] or null
     int nb = 0;
     double q = 1.0;
@@ -327,7 +331,8 @@ double hop_alg_bytes(const ovl_ctx *c, const HopArgs &a, int pin, int pout)
     return b;
 }
 
-int hop(ovl_ctx *c, const Geom &g, int pin, int pout, const HopArgs &a)
+// gauge: a gauge half step to run in the same launch
+int hop(ovl_ctx *c, const Geom &g, int pin, int pout, const HopArgs &a, const ovl::GaugeHalf *gauge = nullptr)
 {
     const int var = (pin == P64) ? 0 : (pin == P16 ? 3 : (pin == P48 ? 4 : (pout == P32 ? 1 : 2)));
     hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -342,7 +347,8 @@ int hop(ovl_ctx *c, const Geom &g, int pin, int pout, const HopArgs &a)
             c->evused--;  // an unpaired event stays unused
         }
     }
-    HIPCHK(c, ovl::launch_hop(g, pin, pout, a, c->wpe[pin], c->st));
+    if (gauge) HIPCHK(c, ovl::launch_hop_gauge(g, pin, a, *gauge, c->st));
+    else HIPCHK(c, ovl::launch_hop(g, pin, pout, a, c->wpe[pin], c->st));
     if (e1) HIPCHK(c, hipEventRecord(e1, c->st));
     const double b = hop_alg_bytes(c, a, pin, pout);
     c->hop_launches++;
@@ -1656,7 +1662,7 @@ int ovl_destroy(ovl_ctx *c)
 {
     if (!c) return OVL_OK;
     if (c->st) hipStreamSynchronize(c->st);
-    void *ps[] = {c->links, c->efield, c->ul64, c->ul32, c->phase, c->field[0], c->field[1], c->field[2], c->w64, c->a64,
+    void *ps[] = {c->links, c->efield, c->ul64, c->ul32, c->ul64_next, c->ul32_next, c->phase, c->field[0], c->field[1], c->field[2], c->w64, c->a64,
                   c->b64, c->x32, c->w32, c->a32, c->b32, c->partial, c->dout, c->gam, c->jv, c->ja, c->staging,
                   c->ms_ps, c->ms_r, c->ms_q, c->ms_w, c->ms_chi, c->ms_coef, c->ms_modes, c->ms_active[0],
                   c->ms_active[1], c->s1_links, c->s1_vec, c->s1_cg, c->s1_ritz, c->s1_start, c->s1_part,
@@ -2210,13 +2216,19 @@ int ritz_bounds(ovl_ctx *c, double *lmin, double *lmax)
 extern "C" {
 
 // ---- dynamics ----
+// a gauge half step of system s; with ul64 / ul32 (those of the system) a link update writes the stencil links
+static ovl::GaugeHalf gauge_half_of(const ovl_ctx *c, int s, int what, double dt, double *ul64, float *ul32)
+{
+    return ovl::gauge_half_args(sys_geom(c, s), what, sys_links(c, s), sys_efield(c, s), dt, c->prm.reunitarize,
+                                sys_phase(c, s), ul64, ul32);
+}
+
 int ovl_update_links(ovl_ctx *c, double dt)
 {
     if (!c || !std::isfinite(dt)) return OVL_E_ARG;
     if (!c->links_set) return fail(c, OVL_E_STATE, "no gauge links uploaded");
     for (int s = 0; s < nsys(c); ++s)
-        HIPCHK(c, ovl::launch_link_update(sys_geom(c, s), sys_links(c, s), sys_efield(c, s), dt, c->prm.reunitarize,
-                                          nullptr, nullptr, nullptr, c->st));
+        HIPCHK(c, ovl::launch_gauge_half(sys_geom(c, s), gauge_half_of(c, s, ovl::GAUGE_LINKS_HALF, dt, nullptr, nullptr), c->st));
     c->stencil_dirty = true;
     HIPCHK(c, hipStreamSynchronize(c->st));
     return OVL_OK;
@@ -2227,7 +2239,7 @@ int ovl_update_efield(ovl_ctx *c, double dt)
     if (!c || !std::isfinite(dt)) return OVL_E_ARG;
     if (!c->links_set) return fail(c, OVL_E_STATE, "no gauge links uploaded");
     for (int s = 0; s < nsys(c); ++s)
-        HIPCHK(c, ovl::launch_efield_update(sys_geom(c, s), sys_links(c, s), sys_efield(c, s), dt, c->st));
+        HIPCHK(c, ovl::launch_gauge_half(sys_geom(c, s), gauge_half_of(c, s, ovl::GAUGE_EFIELD_HALF, dt, nullptr, nullptr), c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
     return OVL_OK;
 }
@@ -2238,9 +2250,8 @@ static int gauge_half(ovl_ctx *c, int mode, double h)
     for (int s = 0; s < nsys(c); ++s) {
         const Geom g = sys_geom(c, s);
         if (mode == OVL_GAUGE_FULL)
-            HIPCHK(c, ovl::launch_efield_update(g, sys_links(c, s), sys_efield(c, s), h, c->st));
-        HIPCHK(c, ovl::launch_link_update(g, sys_links(c, s), sys_efield(c, s), h, c->prm.reunitarize, sys_phase(c, s),
-                                          sys_ul64(c, s), sys_ul32(c, s), c->st));
+            HIPCHK(c, ovl::launch_gauge_half(g, gauge_half_of(c, s, ovl::GAUGE_EFIELD_HALF, h, nullptr, nullptr), c->st));
+        HIPCHK(c, ovl::launch_gauge_half(g, gauge_half_of(c, s, ovl::GAUGE_LINKS_HALF, h, sys_ul64(c, s), sys_ul32(c, s)), c->st));
     }
     return OVL_OK;
 }
@@ -2248,21 +2259,52 @@ static int gauge_half(ovl_ctx *c, int mode, double h)
 // the Wilson leapfrog steps FP32 spinor fields unless the options ask for FP64
 static bool wilson_fp32(const ovl_step_opts *o) { return o->kind == OVL_WILSON && o->sign.precision != OVL_PREC_FP64; }
 
+// target += dt * (-i h_W src): one stencil launch with the axpy in its epilogue, on the FP64 fields or the
+// FP32 copies (3S + L/M bytes per site-mode at S = 96 B for SU(3) instead of 192)
+static int wilson_half(ovl_ctx *c, const ovl_step_opts *o, int src, int tgt, const ovl::GaugeHalf *gauge)
+{
+    const int pr = wilson_fp32(o) ? P32 : P64;
+    HopArgs a = hop_args(c, pr);
+    a.in = pr == P32 ? c->f32[src] : c->field[src];
+    a.out = pr == P32 ? c->f32[tgt] : c->field[tgt];
+    a.tgt = a.out;
+    a.st_r = 1.0;
+    a.sh_i = -o->dt;
+    return hop(c, c->g, pr, pr, a, gauge);
+}
+
+// Whether a step's stencil and gauge half steps share launches: the Wilson steps of one lattice.  It always
+// pays there, most on small lattices, where a launch leaves most of the chip idle (us per step with moving
+// links, apart and shared: SU(2) 8^3, 16 modes FP64 24.1 and 16.8; SU(3) 24^3, 64 modes FP64 236 and 219;
+// SU(3) 32^3, 256 modes FP32 1081 and 1057); an overlap step has hundreds of launches per gauge half step.
+static bool shares_launches(const ovl_ctx *c, const ovl_step_opts *o)
+{
+    return o->kind == OVL_WILSON && o->gauge != OVL_GAUGE_FROZEN && !c->ensemble;
+}
+
+// a Wilson half step with its gauge half step in shared launches.  Links alone: the stencil reads the present
+// stencil links while the update writes the next ones.  With E: the stencil and the E update share one
+// launch (E follows from the present links), the link update needs the new E and follows in place.
+static int shared_half(ovl_ctx *c, const ovl_step_opts *o, int src, int tgt)
+{
+    const double h = 0.5 * o->dt;
+    if (o->gauge == OVL_GAUGE_FULL) {
+        const ovl::GaugeHalf e = gauge_half_of(c, 0, ovl::GAUGE_EFIELD_HALF, h, nullptr, nullptr);
+        RETCHK(wilson_half(c, o, src, tgt, &e));
+        HIPCHK(c, ovl::launch_gauge_half(c->g, gauge_half_of(c, 0, ovl::GAUGE_LINKS_HALF, h, c->ul64, c->ul32), c->st));
+        return OVL_OK;
+    }
+    const ovl::GaugeHalf u = gauge_half_of(c, 0, ovl::GAUGE_LINKS_HALF, h, c->ul64_next, c->ul32_next);
+    RETCHK(wilson_half(c, o, src, tgt, &u));
+    std::swap(c->ul64, c->ul64_next);
+    std::swap(c->ul32, c->ul32_next);
+    return OVL_OK;
+}
+
 // target += dt * (-i h src)   (OverlapUpdate.cpp:85-124, WILSON/Update.cpp:6-45)
 static int fermion_half(ovl_ctx *c, const ovl_step_opts *o, int src, int tgt, void *hpsi = nullptr)
 {
-    if (o->kind == OVL_WILSON) {
-        // one stencil launch with the axpy in its epilogue: FP64 fields, or the FP32 copies (3S + L/M
-        // bytes per site-mode at S = 96 B for SU(3) instead of 192)
-        const int pr = wilson_fp32(o) ? P32 : P64;
-        HopArgs a = hop_args(c, pr);
-        a.in = pr == P32 ? c->f32[src] : c->field[src];
-        a.out = pr == P32 ? c->f32[tgt] : c->field[tgt];
-        a.tgt = a.out;
-        a.st_r = 1.0;
-        a.sh_i = -o->dt;
-        return hop(c, c->g, pr, pr, a);
-    }
+    if (o->kind == OVL_WILSON) return wilson_half(c, o, src, tgt, nullptr);
     if (o->sign.method == OVL_SIGN_ZOLOTAREV)
         return zolo_overlap(c, c->g, c->field[src], c->field[tgt], o->sign.lmin, o->sign.lmax, 1, o->dt);
     return sign_driver(c, &o->sign, c->field[src], c->field[tgt], FIN_OVERLAP_AXPY, o->dt, c->step_xmax, hpsi);
@@ -2292,7 +2334,7 @@ static StepKey make_step_key(const ovl_ctx *c, const ovl_step_opts *o, const Sig
         k.sk = pl->sk;
         k.sw = pl->sw;
     }
-    k.ptrs = {c->links, c->efield, c->ul64, c->ul32, c->phase, c->field[0], c->field[1], c->field[2],
+    k.ptrs = {c->links, c->efield, c->ul64, c->ul32, c->ul64_next, c->ul32_next, c->phase, c->field[0], c->field[1], c->field[2],
               c->w64, c->a64, c->b64, c->x32, c->w32, c->a32, c->b32, c->x16, c->w16, c->a16, c->b16,
               c->x48, c->w48, c->a48, c->b48, c->partial, c->d_sys, c->d_work, c->d_qwork, c->d_qoff, c->d_qctr,
               c->order[0], c->order[1],
@@ -2323,6 +2365,10 @@ static void drop_step_graph(ovl_ctx *c)
 // observe: the second half step also leaves -i h_ov[U(t + dt/2)] Psi(t + dt) in the scratch field
 static int one_step(ovl_ctx *c, const ovl_step_opts *o, bool observe = false)
 {
+    if (shares_launches(c, o)) {
+        RETCHK(shared_half(c, o, OVL_PSIMID, OVL_PSI));
+        return shared_half(c, o, OVL_PSI, OVL_PSIMID);
+    }
     RETCHK(fermion_half(c, o, OVL_PSIMID, OVL_PSI));
     RETCHK(gauge_half(c, o->gauge, 0.5 * o->dt));
     RETCHK(fermion_half(c, o, OVL_PSI, OVL_PSIMID, observe ? c->field[OVL_SCRATCH] : nullptr));
@@ -2401,6 +2447,11 @@ static int update_impl(ovl_ctx *c, const ovl_step_opts *o, int nsteps, bool obse
     if (w32)
         for (int f = 0; f < 2; ++f)
             if (!c->f32[f]) RETCHK(dalloc(c, &c->f32[f], c->field32_bytes));
+    if (shares_launches(c, o) && o->gauge == OVL_GAUGE_LINKS) {
+        const size_t entries = 3 * (size_t)c->link_sites * c->g.nc * c->g.nc;
+        RETCHK(dalloc(c, (void **)&c->ul64_next, 16 * entries));
+        RETCHK(dalloc(c, (void **)&c->ul32_next, 8 * entries));
+    }
     begin_timing(c);
     if (observe_last && nsteps > 0) {
         RETCHK(update_impl(c, req, nsteps - 1, false));

@@ -137,10 +137,24 @@ hipError_t launch_soa_to_aos(const Geom &g, const void *field, int first, int co
 hipError_t launch_link_setup(const Geom &g, const double *links, const double *phase, double *ul64, float *ul32,
                              hipStream_t st);
 hipError_t launch_ucc_to_links(const Geom &g, const double *ucc, double *ul64, float *ul32, hipStream_t st);
-// links <- exp(-i dt E) links; with ul64 (and ul32, phase or null) the stencil links of the new ones too
-hipError_t launch_link_update(const Geom &g, double *links, const double *efield, double dt, int reunit,
-                              const double *phase, double *ul64, float *ul32, hipStream_t st);
-hipError_t launch_efield_update(const Geom &g, const double *links, double *efield, double dt, hipStream_t st);
+// One gauge half step of one lattice: GAUGE_LINKS_HALF: links <- exp(-i dt efield) links and, with ul64, the
+// stencil links of the new ones (phase may be null); GAUGE_EFIELD_HALF: efield += dt force(links)
+enum { GAUGE_LINKS_HALF = 1, GAUGE_EFIELD_HALF = 2 };
+struct GaugeHalf {
+    double *links, *efield;
+    const double *phase;
+    double *ul64;
+    float *ul32;
+    double dt;
+    int reunit, n0, n1, n2, V, what;
+    int blocks;  // workgroups of a shared launch
+};
+GaugeHalf gauge_half_args(const Geom &g, int what, double *links, double *efield, double dt, int reunit, const double *phase,
+                          double *ul64, float *ul32);
+hipError_t launch_gauge_half(const Geom &g, const GaugeHalf &h, hipStream_t st);
+// a leapfrog stencil step (out = i sh_i h_W(in) + tgt, FP64 or FP32 fields of one lattice) and the gauge half
+// step in one launch; they must not touch the same stencil links
+hipError_t launch_hop_gauge(const Geom &g, int prec, const HopArgs &a, const GaugeHalf &h, hipStream_t st);
 // per-mode inner products <a,b> = sum conj(a) b over one field (FP64 fields), nmodes results
 // written as (re, im) pairs to `out` (device); `partial` scratch of partial_len doubles
 hipError_t launch_mode_dot(const Geom &g, const void *a, const void *b, double *partial, double *out,

@@ -311,11 +311,13 @@ struct Site {
     int s, x, y, z;
 };
 template <int MB>
-__device__ __forceinline__ bool lane_coords(const HopArgs &a, int n0, int n1, int V, int &m, Site &p, int &blk)
+__device__ __forceinline__ bool lane_coords(const HopArgs &a, unsigned wg, unsigned wgs, int n0, int n1, int V, int &m,
+                                            Site &p, int &blk)
 {
+    // workgroup wg of the wgs of the stencil
     const unsigned total = (unsigned)a.nblk * (unsigned)V * MB;  // < 2^31, checked by the launcher
-    unsigned lb = blockIdx.x;
-    if (a.trav != TRAV_LEX) lb = (blockIdx.x % NUM_XCD) * (gridDim.x / NUM_XCD) + blockIdx.x / NUM_XCD;
+    unsigned lb = wg;
+    if (a.trav != TRAV_LEX) lb = (wg % NUM_XCD) * (wgs / NUM_XCD) + wg / NUM_XCD;
     const unsigned gl = lb * TPB + threadIdx.x;
     if (gl >= total) return false;
     m = (int)(gl % MB);
@@ -640,7 +642,7 @@ __global__ __launch_bounds__(TPB) __attribute__((amdgpu_waves_per_eu(WPE))) void
     Site p;
     // 64-mode blocks have one site per wavefront: site and block are wave-uniform there, so that the links
     // (shared by all modes of the site) come through scalar loads instead of 64 identical vector lanes
-    if (!lane_coords<MB>(a, n0, n1, V, m, p, blk)) return;
+    if (!lane_coords<MB>(a, blockIdx.x, gridDim.x, n0, n1, V, m, p, blk)) return;
     hop_site<NC, TI, TO, MB, EPI>(a, n0, n1, n2, p, blk * V, 0, m);
 }
 
@@ -1036,6 +1038,11 @@ __device__ __forceinline__ Mat<3> gather_columns(const cd *c)
     return m;
 }
 
+// 1/k of the Taylor series (a division would be as long as the product it scales)
+__device__ const double inverse_of[21] = {0.0,      1.0,      1.0 / 2,  1.0 / 3,  1.0 / 4,  1.0 / 5,  1.0 / 6,
+                                          1.0 / 7,  1.0 / 8,  1.0 / 9,  1.0 / 10, 1.0 / 11, 1.0 / 12, 1.0 / 13,
+                                          1.0 / 14, 1.0 / 15, 1.0 / 16, 1.0 / 17, 1.0 / 18, 1.0 / 19, 1.0 / 20};
+
 // column `col` of exp(i c alpha^a t^a): scaling and squaring of the Taylor series (FP64).  The columns of
 // the Horner form are independent, so three of four lanes walk one each: a third of the 20 matrix
 // products' chain per lane, the sums of the one-lane form unchanged.
@@ -1058,10 +1065,9 @@ __device__ void iexp_column(double c, const double *alpha, int col, cd *r)
     const double one[3] = {col == 0 ? 1.0 : 0.0, col == 1 ? 1.0 : 0.0, col == 2 ? 1.0 : 0.0};
 #pragma unroll
     for (int i = 0; i < 3; ++i) r[i] = {one[i], 0.0};
-#pragma unroll
-    for (int k = 20; k >= 1; --k) {  // unrolled: 1/k are constants
+    for (int k = 20; k >= 1; --k) {
         mcol<true>(a, r);
-        const double f = 1.0 / k;
+        const double f = inverse_of[k];
 #pragma unroll
         for (int i = 0; i < 3; ++i) r[i] = {__builtin_fma(f, r[i].r, one[i]), f * r[i].i};
     }
@@ -1121,10 +1127,13 @@ __device__ Mat<3> reunit3(Mat<3> x)
 }
 
 // one entry of the stencil links (ConvertGaugeLinks, OverlapEvolutionOperator.cpp:23-51, with the QED
-// phase folded in)
+// phase folded in).  The products round in a fixed form, so that every kernel that writes a stencil link
+// writes the same bits: PI: the imaginary part rounds ph.i m.r first, else ph.r m.i
+template <bool PI>
 __device__ __forceinline__ void put_stencil_entry(cd ph, cd m, double2 *__restrict__ u64, float2 *__restrict__ u32, size_t k)
 {
-    const cd v = cmul(ph, m);
+    const cd v = {__builtin_fma(ph.r, m.r, -(ph.i * m.i)),
+                  PI ? __builtin_fma(ph.r, m.i, ph.i * m.r) : __builtin_fma(ph.i, m.r, ph.r * m.i)};
     u64[k] = make_double2(v.r, v.i);
     u32[k] = make_float2((float)v.r, (float)v.i);
 }
@@ -1144,7 +1153,10 @@ __global__ __launch_bounds__(TPB) void k_link_setup(const double *__restrict__ l
     const Mat<NC> m = get_link<NC>(links, s, mu);
     const cd ph = phase_of(phase, i);
 #pragma unroll
-    for (int k = 0; k < NC * NC; ++k) put_stencil_entry(ph, m.e[k], u64, u32, (size_t)i * NC * NC + k);
+    for (int k = 0; k < NC * NC; ++k) {
+        if (NC == 2 && (k == 1 || k == 2)) put_stencil_entry<true>(ph, m.e[k], u64, u32, (size_t)i * NC * NC + k);
+        else put_stencil_entry<false>(ph, m.e[k], u64, u32, (size_t)i * NC * NC + k);
+    }
 }
 
 // stencil links from a host-layout u_cc array (already in [mu*V+s][i][j] order)
@@ -1166,13 +1178,12 @@ __global__ __launch_bounds__(TPB) void k_ucc_setup(const double2 *__restrict__ u
 // 5.7 and 15.7 us (24^3: 25 MB read and written in 144-byte strides).
 constexpr int LINK_TPB = 64;
 template <int NC>
-__global__ __launch_bounds__(LINK_TPB) void k_link_update(double *__restrict__ links, const double *__restrict__ e,
-                                                          double dt, int V, int reunit,
-                                                          const double2 *__restrict__ phase, double2 *__restrict__ u64,
-                                                          float2 *__restrict__ u32)
+__device__ __forceinline__ void link_update_lane(unsigned lane, double *__restrict__ links, const double *__restrict__ e,
+                                                 double dt, int V, int reunit, const double2 *__restrict__ phase,
+                                                 double2 *__restrict__ u64, float2 *__restrict__ u32)
 {
     constexpr int LPL = NC == 2 ? 1 : 4;  // lanes per link
-    const int i = (int)(blockIdx.x * (LINK_TPB / LPL) + threadIdx.x / LPL);
+    const int i = (int)(lane / LPL);
     if (i >= 3 * V) return;  // the lanes of a link leave together
     const int s = i / 3, mu = i - 3 * s;  // link (s, mu) at index mu + 3 s
     constexpr int NG = NC * NC - 1;
@@ -1204,9 +1215,10 @@ __global__ __launch_bounds__(LINK_TPB) void k_link_update(double *__restrict__ l
         if (u64) {
             const int iu = mu * V + s;
             const cd ph = phase_of(phase, iu);
-            const cd m[4] = {{n3, n2}, {n1, n0}, {-n1, n0}, {n3, -n2}};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) put_stencil_entry(ph, m[k], u64, u32, (size_t)iu * 4 + k);
+            put_stencil_entry<false>(ph, cd{n3, n2}, u64, u32, (size_t)iu * 4);
+            put_stencil_entry<true>(ph, cd{n1, n0}, u64, u32, (size_t)iu * 4 + 1);
+            put_stencil_entry<true>(ph, cd{-n1, n0}, u64, u32, (size_t)iu * 4 + 2);
+            put_stencil_entry<false>(ph, cd{n3, -n2}, u64, u32, (size_t)iu * 4 + 3);
         }
     } else {
         const int col = threadIdx.x % 4 < 3 ? threadIdx.x % 4 : 0;  // the fourth lane repeats the first
@@ -1231,9 +1243,15 @@ __global__ __launch_bounds__(LINK_TPB) void k_link_update(double *__restrict__ l
             const int iu = mu * V + s;
             const cd ph = phase_of(phase, iu);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) put_stencil_entry(ph, r[k], u64, u32, (size_t)iu * 9 + 3 * k + col);
+            for (int k = 0; k < 3; ++k) put_stencil_entry<false>(ph, r[k], u64, u32, (size_t)iu * 9 + 3 * k + col);
         }
     }
+}
+template <int NC>
+__global__ __launch_bounds__(LINK_TPB) void k_link_update(GaugeHalf g)
+{
+    link_update_lane<NC>(blockIdx.x * LINK_TPB + threadIdx.x, g.links, g.efield, g.dt, g.V, g.reunit,
+                         (const double2 *)g.phase, (double2 *)g.ul64, (float2 *)g.ul32);
 }
 
 __device__ __forceinline__ int nbr(int s, int dmu, int step, int n0, int n1, int n2)
@@ -1253,12 +1271,12 @@ __device__ __forceinline__ int nbr(int s, int dmu, int step, int n0, int n1, int
 // 15 x 12 x 10, where a lane per link left most CUs without a wave, 17.8 -> 15.3 us on 24^3, where the
 // matrices' strided loads bound it).
 template <int NC>
-__global__ __launch_bounds__(LINK_TPB) void k_efield_update(const double *__restrict__ links, double *__restrict__ e,
-                                                            double dt, int n0, int n1, int n2)
+__device__ __forceinline__ void efield_update_lane(unsigned lane, const double *__restrict__ links, double *__restrict__ e,
+                                                   double dt, int n0, int n1, int n2)
 {
     const int V = n0 * n1 * n2;
     const int j = threadIdx.x % 4;
-    const int i = (int)(blockIdx.x * (LINK_TPB / 4) + threadIdx.x / 4);
+    const int i = (int)(lane / 4);
     const bool ok = i < 3 * V;
     const int il = ok ? i : 3 * V - 1;
     const int s = il / 3, mu = il - 3 * s;
@@ -1294,6 +1312,33 @@ __global__ __launch_bounds__(LINK_TPB) void k_efield_update(const double *__rest
 #pragma unroll
     for (int k = 0; k < NG; ++k)
         if (k % 4 == j) o[k] += -2.0 * dt * f[k];
+}
+template <int NC> __global__ __launch_bounds__(LINK_TPB) void k_efield_update(GaugeHalf g)
+{
+    efield_update_lane<NC>(blockIdx.x * LINK_TPB + threadIdx.x, g.links, g.efield, g.dt, g.n0, g.n1, g.n2);
+}
+
+// A Wilson half step and a gauge half step in one launch: the first gauge.blocks workgroups (a multiple of the
+// XCDs, so that the others keep theirs) update the links (into other stencil links than the ones being
+// read) or the E field, the rest are the stencil's.  The two do not depend on each other, and on small
+// lattices each is a launch that leaves most of the chip idle.
+template <int NC, typename T, int MB>
+__global__ __launch_bounds__(TPB) void k_hop_gauge(HopArgs a, GaugeHalf g, int n0, int n1, int n2)
+{
+    if (blockIdx.x < (unsigned)g.blocks) {
+        const unsigned lane = blockIdx.x * TPB + threadIdx.x;
+        if (g.what == GAUGE_LINKS_HALF)
+            link_update_lane<NC>(lane, g.links, g.efield, g.dt, g.V, g.reunit, (const double2 *)g.phase, (double2 *)g.ul64,
+                                 (float2 *)g.ul32);
+        else
+            efield_update_lane<NC>(lane, g.links, g.efield, g.dt, n0, n1, n2);
+        return;
+    }
+    const int V = n0 * n1 * n2;
+    int m, blk;
+    Site p;
+    if (!lane_coords<MB>(a, blockIdx.x - g.blocks, gridDim.x - g.blocks, n0, n1, V, m, p, blk)) return;
+    hop_site<NC, T, T, MB, EPI_AXPY>(a, n0, n1, n2, p, blk * V, 0, m);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1896,6 +1941,26 @@ void hop_ens_wpe(const HopArgs &b, int wpe, hipStream_t st)
     hop_ens_wpe_epi<NC, TI, TO, MB, EPI_ANY>(b, wpe, st);
 }
 
+// the launch arguments of one lattice: lane coordinates, and the traversal where the launch splits evenly;
+// false when the lanes exceed 32 bits
+bool lattice_args(const Geom &g, const HopArgs &a, HopArgs &b, unsigned &nb)
+{
+    const long total = (long)a.nblk * g.V * g.mb;
+    if (total >= (1l << 31)) return false;
+    nb = nblocks(total);
+    b = a;
+    b.dv_V = make_fastdiv((unsigned)g.V);
+    b.dv_per = make_fastdiv((unsigned)((long)a.nblk * g.V / NUM_XCD));
+    b.dv_v8 = make_fastdiv((unsigned)(g.V / NUM_XCD));
+    b.dv_n01 = make_fastdiv((unsigned)(g.n0 * g.n1));
+    b.dv_n0 = make_fastdiv((unsigned)g.n0);
+    // the XCD traversals need whole workgroups spread evenly over the XCDs
+    const bool even = total % ((long)TPB * NUM_XCD) == 0;
+    if (b.trav == TRAV_BOXES && (!even || g.V % NUM_XCD != 0 || (!b.order && b.box.dv_x.d == 0))) b.trav = TRAV_LEX;
+    if (b.trav == TRAV_MODES && !even) b.trav = TRAV_LEX;
+    return true;
+}
+
 template <int NC, typename TI, typename TO>
 hipError_t hop_mb(const Geom &g, const HopArgs &a, int wpe, hipStream_t st)
 {
@@ -1909,23 +1974,28 @@ hipError_t hop_mb(const Geom &g, const HopArgs &a, int wpe, hipStream_t st)
         }
         return hipGetLastError();
     }
-    const long total = (long)a.nblk * g.V * g.mb;
-    if (total >= (1l << 31)) return hipErrorInvalidValue;  // lanes are counted in 32 bits
-    const unsigned nb = nblocks(total);
-    HopArgs b = a;
-    b.dv_V = make_fastdiv((unsigned)g.V);
-    b.dv_per = make_fastdiv((unsigned)((long)a.nblk * g.V / NUM_XCD));
-    b.dv_v8 = make_fastdiv((unsigned)(g.V / NUM_XCD));
-    b.dv_n01 = make_fastdiv((unsigned)(g.n0 * g.n1));
-    b.dv_n0 = make_fastdiv((unsigned)g.n0);
-    // the XCD traversals need whole workgroups spread evenly over the XCDs
-    const bool even = total % ((long)TPB * NUM_XCD) == 0;
-    if (b.trav == TRAV_BOXES && (!even || g.V % NUM_XCD != 0 || (!b.order && b.box.dv_x.d == 0))) b.trav = TRAV_LEX;
-    if (b.trav == TRAV_MODES && !even) b.trav = TRAV_LEX;
+    HopArgs b;
+    unsigned nb;
+    if (!lattice_args(g, a, b, nb)) return hipErrorInvalidValue;
     switch (g.mb) {
     case 16: hop_wpe<NC, TI, TO, 16>(b, nb, wpe, g, st); break;
     case 32: hop_wpe<NC, TI, TO, 32>(b, nb, wpe, g, st); break;
     case 64: hop_wpe<NC, TI, TO, 64>(b, nb, wpe, g, st); break;
+    default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+template <int NC, typename T>
+hipError_t hop_gauge_mb(const Geom &g, const HopArgs &a, const GaugeHalf &h, hipStream_t st)
+{
+    HopArgs b;
+    unsigned nb;
+    if (!lattice_args(g, a, b, nb) || h.blocks % NUM_XCD != 0) return hipErrorInvalidValue;
+    nb += (unsigned)h.blocks;
+    switch (g.mb) {
+    case 16: k_hop_gauge<NC, T, 16><<<nb, TPB, 0, st>>>(b, h, g.n0, g.n1, g.n2); break;
+    case 32: k_hop_gauge<NC, T, 32><<<nb, TPB, 0, st>>>(b, h, g.n0, g.n1, g.n2); break;
+    case 64: k_hop_gauge<NC, T, 64><<<nb, TPB, 0, st>>>(b, h, g.n0, g.n1, g.n2); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -2208,24 +2278,35 @@ hipError_t launch_ucc_to_links(const Geom &g, const double *ucc, double *ul64, f
     return hipGetLastError();
 }
 
-hipError_t launch_link_update(const Geom &g, double *links, const double *efield, double dt, int reunit,
-                              const double *phase, double *ul64, float *ul32, hipStream_t st)
+// lanes of a gauge half step: SU(2) links one each, SU(3) links and E fields four
+static long gauge_lanes(const Geom &g, int what) { return 3L * g.V * (what == GAUGE_LINKS_HALF && g.nc == 2 ? 1 : 4); }
+
+GaugeHalf gauge_half_args(const Geom &g, int what, double *links, double *efield, double dt, int reunit, const double *phase,
+                          double *ul64, float *ul32)
 {
-    const unsigned nb = (unsigned)((3L * g.V * (g.nc == 2 ? 1 : 4) + LINK_TPB - 1) / LINK_TPB);
-    const auto ph = (const double2 *)phase;
-    if (g.nc == 2)
-        k_link_update<2><<<nb, LINK_TPB, 0, st>>>(links, efield, dt, g.V, reunit, ph, (double2 *)ul64, (float2 *)ul32);
-    else
-        k_link_update<3><<<nb, LINK_TPB, 0, st>>>(links, efield, dt, g.V, reunit, ph, (double2 *)ul64, (float2 *)ul32);
+    const long nb = (gauge_lanes(g, what) + TPB - 1) / TPB;
+    return GaugeHalf{links, efield, phase, ul64, ul32, dt, reunit, g.n0, g.n1, g.n2, g.V, what,
+                     (int)((nb + NUM_XCD - 1) / NUM_XCD * NUM_XCD)};
+}
+
+hipError_t launch_gauge_half(const Geom &g, const GaugeHalf &h, hipStream_t st)
+{
+    const unsigned nb = (unsigned)((gauge_lanes(g, h.what) + LINK_TPB - 1) / LINK_TPB);
+    if (h.what == GAUGE_LINKS_HALF) {
+        if (g.nc == 2) k_link_update<2><<<nb, LINK_TPB, 0, st>>>(h);
+        else k_link_update<3><<<nb, LINK_TPB, 0, st>>>(h);
+    } else {
+        if (g.nc == 2) k_efield_update<2><<<nb, LINK_TPB, 0, st>>>(h);
+        else k_efield_update<3><<<nb, LINK_TPB, 0, st>>>(h);
+    }
     return hipGetLastError();
 }
 
-hipError_t launch_efield_update(const Geom &g, const double *links, double *efield, double dt, hipStream_t st)
+hipError_t launch_hop_gauge(const Geom &g, int prec, const HopArgs &a, const GaugeHalf &h, hipStream_t st)
 {
-    const unsigned nb = (unsigned)((12L * g.V + LINK_TPB - 1) / LINK_TPB);
-    if (g.nc == 2) k_efield_update<2><<<nb, LINK_TPB, 0, st>>>(links, efield, dt, g.n0, g.n1, g.n2);
-    else k_efield_update<3><<<nb, LINK_TPB, 0, st>>>(links, efield, dt, g.n0, g.n1, g.n2);
-    return hipGetLastError();
+    if (a.ens_sys || epi_kind(a) != EPI_AXPY) return hipErrorInvalidValue;
+    if (g.nc == 2) return prec == P64 ? hop_gauge_mb<2, double>(g, a, h, st) : hop_gauge_mb<2, float>(g, a, h, st);
+    return prec == P64 ? hop_gauge_mb<3, double>(g, a, h, st) : hop_gauge_mb<3, float>(g, a, h, st);
 }
 
 size_t mode_dot_partial_len(const Geom &g) { return (size_t)DOT_CHUNKS * g.nblk * g.mb * 2; }
