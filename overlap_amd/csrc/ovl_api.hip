@@ -141,6 +141,10 @@ struct ovl_ctx {
     void *s1_links = nullptr, *s1_vec = nullptr, *s1_cg = nullptr, *s1_ritz = nullptr, *s1_start = nullptr;
     double *s1_part = nullptr;
     void *s1_state = nullptr;
+    // one batch of iterations of the single-vector CG and of the pair of Ritz bounds, instantiated: their
+    // launches are the same in every batch and call (the buffers above are allocated once)
+    hipGraphExec_t cg1_exec = nullptr, ritz_exec = nullptr;
+    int cg1_calls = 0;
 
     // timing
     bool profiling = false;
@@ -1226,21 +1230,38 @@ int mscg(ovl_ctx *c, const Geom &g, const void *in, void *chi, const ovl::CgShif
     return OVL_OK;
 }
 
+// the launches that `body` queues on the context's stream, as an instantiated graph
+template <class F> int capture_launches(ovl_ctx *c, hipGraphExec_t *exec, F body)
+{
+    hipGraph_t graph = nullptr;
+    HIPCHK(c, hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
+    const hipError_t e = body();
+    const hipError_t end = hipStreamEndCapture(c->st, &graph);
+    hipError_t r = e != hipSuccess ? e : end;
+    if (r == hipSuccess) r = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0);
+    if (graph) hipGraphDestroy(graph);
+    if (r != hipSuccess) {
+        *exec = nullptr;
+        return fail(c, OVL_E_HIP, std::string("solver graph: ") + hipGetErrorString(r));
+    }
+    return OVL_OK;
+}
+
 // ---- one vector ([spin][colour][site]) ----
+// states of the CG or of the Ritz solves; after them two ints (non-finite flags of a drop-in's inputs) and
+// the CG's shifts
+constexpr size_t SINGLE_STATES = 2 * std::max(sizeof(ovl::CgMode), ovl::RITZ_SOLVES * sizeof(ovl::RitzState));
 // links, partial results and states of the single-vector kernels
 int ensure_single(ovl_ctx *c)
 {
     const size_t V = (size_t)c->g.V;
     RETCHK(dalloc(c, &c->s1_links, 16 * 3 * V * c->g.nc * c->g.nc));
     RETCHK(dalloc(c, (void **)&c->s1_part, sizeof(double) * ovl::single_partial_len(c->g)));
-    return dalloc(c, &c->s1_state, 2 * std::max(sizeof(ovl::CgMode), ovl::RITZ_SOLVES * sizeof(ovl::RitzState)) + sizeof(int) * 2);
+    return dalloc(c, &c->s1_state, SINGLE_STATES + sizeof(int) * 2 + sizeof(ovl::CgShifts));
 }
 size_t vec1_bytes(const ovl_ctx *c) { return (size_t)c->g.V * c->ncomp * 16; }
-// two ints after the states: non-finite flags of a drop-in's inputs
-int *single_flags(const ovl_ctx *c)
-{
-    return (int *)((char *)c->s1_state + 2 * std::max(sizeof(ovl::CgMode), ovl::RITZ_SOLVES * sizeof(ovl::RitzState)));
-}
+int *single_flags(const ovl_ctx *c) { return (int *)((char *)c->s1_state + SINGLE_STATES); }
+ovl::CgShifts *single_shifts(const ovl_ctx *c) { return (ovl::CgShifts *)(single_flags(c) + 2); }
 
 // the single-vector form of mscg: `in` and the links c->s1_links are set, *chi receives the solution
 int mscg1(ovl_ctx *c, const void *in, const ovl::CgShifts &sh, void **chi, int *nonconv)
@@ -1254,18 +1275,30 @@ int mscg1(ovl_ctx *c, const void *in, const ovl::CgShifts &sh, void **chi, int *
     k.links = c->s1_links;
     k.amass = amass(c);
     k.tol = CG_TOL;
-    k.sh = sh;
+    k.shifts = single_shifts(c);
     k.cap = CG_CAP;
+    HIPCHK(c, hipMemcpyAsync(single_shifts(c), &sh, sizeof sh, hipMemcpyHostToDevice, c->st));
     HIPCHK(c, ovl::launch_cg1_start(c->g, k, c->st));
-    ovl::CgMode m{};
-    constexpr int batch = 8;  // an iteration is four short launches: look every eighth (20 us in 150 us)
-    for (int it = 0;; ++it) {
-        if (it % batch == 0 || it == CG_CAP) {
-            HIPCHK(c, hipMemcpyAsync(&m, (ovl::CgMode *)c->s1_state + (it & 1), sizeof m, hipMemcpyDeviceToHost, c->st));
-            HIPCHK(c, hipStreamSynchronize(c->st));
-            if (!m.act || it == CG_CAP) break;
+    // An iteration is four short launches: look for the end every eighth (20 us in 150).  From the second call
+    // on the batch is a graph: its gaps are a third of the eager launches', its capture costs as much as
+    // it saves in two calls.
+    constexpr int batch = 8;
+    static_assert(CG_CAP % batch == 0, "whole batches");
+    auto iterations = [&]() -> hipError_t {
+        for (int i = 0; i < batch; ++i) {
+            const hipError_t e = ovl::launch_cg1_iteration(c->g, k, i, c->st);
+            if (e != hipSuccess) return e;
         }
-        HIPCHK(c, ovl::launch_cg1_iteration(c->g, k, it, c->st));
+        return hipSuccess;
+    };
+    if (!c->cg1_exec && ++c->cg1_calls >= 2) RETCHK(capture_launches(c, &c->cg1_exec, iterations));
+    ovl::CgMode m{};
+    for (int it = 0;; it += batch) {
+        HIPCHK(c, hipMemcpyAsync(&m, c->s1_state, sizeof m, hipMemcpyDeviceToHost, c->st));
+        HIPCHK(c, hipStreamSynchronize(c->st));
+        if (!m.act || it == CG_CAP) break;
+        if (c->cg1_exec) HIPCHK(c, hipGraphLaunch(c->cg1_exec, c->st));
+        else HIPCHK(c, iterations());
     }
     *nonconv = m.it >= CG_CAP && m.rn > CG_TOL * m.bn;
     *chi = ovl::cg1_chi(c->g, c->s1_cg);
@@ -1670,7 +1703,8 @@ int ovl_destroy(ovl_ctx *c)
                   c->order[0], c->order[1],
                   c->order[2], c->order[3], c->x16, c->w16, c->a16, c->b16, c->x48, c->w48, c->a48, c->b48,
                   c->f32[0], c->f32[1], c->guard_buf[0], c->guard_buf[1]};
-    if (c->step_exec) hipGraphExecDestroy(c->step_exec);
+    for (hipGraphExec_t x : {c->step_exec, c->cg1_exec, c->ritz_exec})
+        if (x) hipGraphExecDestroy(x);
     for (void *p : ps)
         if (p) hipFree(p);
     if (c->holds_copies) ovl::hostcopy_release();
@@ -2138,21 +2172,34 @@ static int ritz_solve(ovl_ctx *c, int solves, const double *sign, double delitr,
     std::vector<ovl::RitzState> h((size_t)2 * solves);
     HIPCHK(c, hipMemsetAsync(c->s1_state, 0, sizeof(ovl::RitzState) * h.size(), c->st));
     HIPCHK(c, ovl::launch_ritz_start(c->g, k, c->st));
-    // an iteration is five short launches; once all solves are done they return at once
-    constexpr int batch = 16;
-    for (int it = 0;; ++it) {
-        if (it > 0 && it % batch == 0) {
-            HIPCHK(c, hipMemcpyAsync(h.data(), c->s1_state, sizeof(ovl::RitzState) * h.size(), hipMemcpyDeviceToHost, c->st));
-            HIPCHK(c, hipStreamSynchronize(c->st));
-            bool all = true;
-            for (int q = 0; q < solves; ++q) all = all && h[2 * q + (it & 1)].done;
-            if (all) {
-                for (int q = 0; q < solves; ++q) eig[q] = h[2 * q + (it & 1)].xy_r;
-                return OVL_OK;
-            }
+    // An iteration is five short launches; once all solves are done they return at once.  The pair of bounds
+    // takes hundreds of iterations, so a batch of them is a graph (a third of the gaps of eager launches);
+    // its length is even and divides the 100 iterations between restarts, which stay outside.
+    constexpr int batch = 20;
+    const bool graph = solves == 2 && nrestart % batch == 0;
+    auto iterations = [&](int n, int first) -> hipError_t {
+        for (int i = 0; i < n; ++i) {
+            const hipError_t e = ovl::launch_ritz_iteration(c->g, k, first + i, c->st);
+            if (e != hipSuccess) return e;
         }
-        HIPCHK(c, ovl::launch_ritz_iteration(c->g, k, it, it % nrestart == 0, c->st));
-        c->hop_launches += 2;
+        return hipSuccess;
+    };
+    if (graph && !c->ritz_exec) RETCHK(capture_launches(c, &c->ritz_exec, [&] { return iterations(batch, 0); }));
+    for (int it = 0;;) {
+        if (it % nrestart == 0) HIPCHK(c, ovl::launch_ritz_restart(c->g, k, it, c->st));
+        const int n = graph ? batch : std::min(batch, nrestart - it % nrestart);
+        if (graph) HIPCHK(c, hipGraphLaunch(c->ritz_exec, c->st));
+        else HIPCHK(c, iterations(n, it));
+        it += n;
+        c->hop_launches += 2 * n;
+        HIPCHK(c, hipMemcpyAsync(h.data(), c->s1_state, sizeof(ovl::RitzState) * h.size(), hipMemcpyDeviceToHost, c->st));
+        HIPCHK(c, hipStreamSynchronize(c->st));
+        bool all = true;
+        for (int q = 0; q < solves; ++q) all = all && h[2 * q + (it & 1)].done;
+        if (all) {
+            for (int q = 0; q < solves; ++q) eig[q] = h[2 * q + (it & 1)].xy_r;
+            return OVL_OK;
+        }
     }
 }
 

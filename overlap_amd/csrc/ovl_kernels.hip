@@ -1734,20 +1734,27 @@ __global__ __launch_bounds__(TPB) void k_mode_dot(const double2 *__restrict__ a,
     }
 }
 
-// sum over the chunks, one wavefront per mode (two partial results per lane, then the wave's tree)
+// sum over the chunks in their order, one wavefront per mode: the lanes fetch the partial results together
+// (a lane that walked them itself waited for 128 loads, 10 us), two lanes add the real and imaginary parts.
+// The order is part of the results: the FP16 scales of the mixed sign are the norms' next power of two,
+// and norms of one sit on the edge of it.
 __global__ __launch_bounds__(64) void k_mode_dot_finish(const double2 *__restrict__ partial, double2 *__restrict__ out,
                                                         int nmodes_pad)
 {
+    __shared__ double sh[2][DOT_CHUNKS];
     const int i = blockIdx.x;
-    double r = 0, im = 0;
     for (int c = threadIdx.x; c < DOT_CHUNKS; c += 64) {
         const double2 p = partial[(size_t)c * nmodes_pad + i];
-        r += p.x;
-        im += p.y;
+        sh[0][c] = p.x;
+        sh[1][c] = p.y;
     }
-    r = wave_sum(r);
-    im = wave_sum(im);
-    if (threadIdx.x == 0) out[i] = make_double2(r, im);
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        double r = 0;
+#pragma unroll 16
+        for (int c = 0; c < DOT_CHUNKS; ++c) r += sh[threadIdx.x][c];
+        reinterpret_cast<double *>(out)[2 * i + threadIdx.x] = r;
+    }
 }
 
 // currents (OverlapCurrents.cpp:137-228), per (site, mode) bilinears summed over the modes of a block.

@@ -555,7 +555,7 @@ struct Cg1Args {
     Lat1 g;
     long n;
     int nb_hop, nb_pt, nbmax, par;
-    CgShifts sh;
+    const CgShifts *sh;
     double tol;
     int cap;
 };
@@ -597,6 +597,7 @@ template <int NC, bool SECOND> __global__ __launch_bounds__(TPB1) void k_cg1_hop
     const bool ok = site1(a.g.V, s, sp);
     double2 r[2][NC];
     hop1_site<NC>(SECOND ? a.w : a.ps, a.links, a.g, s, sp, r[0], r[1]);
+    const double dz0 = a.sh->dz[0];
     double t[1] = {0.0};
     if (ok)
 #pragma unroll
@@ -607,8 +608,8 @@ template <int NC, bool SECOND> __global__ __launch_bounds__(TPB1) void k_cg1_hop
                 double2 v = r[k][c];
                 if (SECOND) {
                     const double2 p = a.ps[i];
-                    v.x += a.sh.dz[0] * p.x;
-                    v.y += a.sh.dz[0] * p.y;
+                    v.x += dz0 * p.x;
+                    v.y += dz0 * p.y;
                     a.q[i] = v;
                     t[0] += p.x * v.x + p.y * v.y;
                 } else {
@@ -662,7 +663,7 @@ __global__ __launch_bounds__(TPB1) void k_cg1_shifts(Cg1Args a)
     __shared__ double cf[CG_SHIFTS][3];
     if (k < CG_SHIFTS) {
         double z = o.z[k], gc = o.gc[k], f[3];
-        cg_shift_scalars(o.rn, o.a0, o.betam, a.sh, k, al0, rr[0], z, gc, f);
+        cg_shift_scalars(o.rn, o.a0, o.betam, *a.sh, k, al0, rr[0], z, gc, f);
         cf[k][0] = f[0];
         cf[k][1] = f[1];
         cf[k][2] = f[2];
@@ -846,7 +847,7 @@ Cg1Args cg1_args(const Geom &g, const Cg1Call &c)
     a.nb_hop = hop_blocks(g);
     a.nb_pt = point_blocks(n);
     a.nbmax = std::max(a.nb_hop, a.nb_pt);
-    a.sh = c.sh;
+    a.sh = (const CgShifts *)c.shifts;
     a.tol = c.tol;
     a.cap = c.cap;
     return a;
@@ -925,17 +926,21 @@ template <int NC> static void ritz_iteration_nc(const RitzArgs &a, int solves, h
     k_ritz_direction<<<pt, TPB1, 0, st>>>(a);
 }
 
-hipError_t launch_ritz_iteration(const Geom &g, const RitzCall &c, int iter, bool restart, hipStream_t st)
+hipError_t launch_ritz_restart(const Geom &g, const RitzCall &c, int iter, hipStream_t st)
 {
     RitzArgs a = ritz_args(g, c);
     a.par = iter & 1;
-    if (g.nc == 2) {
-        if (restart) ritz_restart_nc<2>(a, c.solves, st);
-        ritz_iteration_nc<2>(a, c.solves, st);
-    } else {
-        if (restart) ritz_restart_nc<3>(a, c.solves, st);
-        ritz_iteration_nc<3>(a, c.solves, st);
-    }
+    if (g.nc == 2) ritz_restart_nc<2>(a, c.solves, st);
+    else ritz_restart_nc<3>(a, c.solves, st);
+    return hipGetLastError();
+}
+
+hipError_t launch_ritz_iteration(const Geom &g, const RitzCall &c, int iter, hipStream_t st)
+{
+    RitzArgs a = ritz_args(g, c);
+    a.par = iter & 1;
+    if (g.nc == 2) ritz_iteration_nc<2>(a, c.solves, st);
+    else ritz_iteration_nc<3>(a, c.solves, st);
     return hipGetLastError();
 }
 
