@@ -65,9 +65,10 @@ typedef struct {
     int traversal;       /* order in which the stencil launches walk (mode, site) lanes over the 8 XCDs:
                             0 = automatic (ovl_autotune picks among the others),
                             1 = lexicographic (hardware round-robin of workgroups over XCDs),
-                            2 = one spatial box of sites per XCD (every mode block in turn),
-                            3 = 1/8 of the mode blocks per XCD over the whole lattice (y slabs,
-                                z-major); needs a multiple of 8 mode blocks */
+                            2 = one spatial box of sites per XCD (every mode block in turn); a
+                                lattice without eight equal boxes walks as 3,
+                            3 = a contiguous 1/8 of the (mode block, site) lanes per XCD (y slabs,
+                                z-major): whole mode blocks where their number divides by 8 */
 } ovl_params;
 
 /* sign function eps(h_W) options */

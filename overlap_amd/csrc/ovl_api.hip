@@ -468,7 +468,14 @@ int set_traversal(ovl_ctx *c, int prec, int trav, int slabs)
         return OVL_OK;
     }
     if (trav == ovl::TRAV_QUEUE) trav = ovl::TRAV_LEX;
-    if (trav == ovl::TRAV_BOXES && !c->boxes_ok) trav = ovl::TRAV_LEX;
+    // a lattice without eight equal boxes gives every XCD a contiguous eighth of the workgroups; dealt out one
+    // by one they fetched every plane on all eight XCDs (us per Clenshaw degree, dealt and contiguous:
+    // SU(3) 21 x 23 x 22, 64 modes 286 and 220 in FP64, 143 and 105 in FP32; 11 x 14 x 9, 40 modes 50.5
+    // and 37.7, 25.3 and 21.9; SU(2) 9^3, 8 modes 13.2 and 12.1, 9.2 and 8.2)
+    if (trav == ovl::TRAV_BOXES && !c->boxes_ok) {
+        trav = ovl::TRAV_MODES;
+        slabs = 1;
+    }
     slabs = std::max(1, std::min(slabs, c->g.n1));
     if (trav == ovl::TRAV_LEX) slabs = 1;
     if (c->order_set[prec] && trav == c->trav[prec] && slabs == c->slabs[prec]) return OVL_OK;

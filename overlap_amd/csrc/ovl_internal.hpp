@@ -83,7 +83,7 @@ struct HopArgs {
     void *out2;        // optional second output: out2_scale * (sh*h_W(in) + sx*G(x)), before b1/b2/tgt
     double out2_scale;
     int nblk;         // blocks covered by this launch
-    int trav;         // lane traversal, TRAV_* (falls back to TRAV_LEX where the launch does not split evenly)
+    int trav;         // lane traversal, TRAV_* (TRAV_BOXES without eight equal boxes runs as TRAV_MODES)
     const int *order; // TRAV_BOXES: XCD k's box is order[k V/8 .. (k+1) V/8) (null = `box`, computed);
                       // TRAV_MODES: site order inside a mode block (null = lexicographic)
     XcdBoxes box;     // TRAV_BOXES without a table

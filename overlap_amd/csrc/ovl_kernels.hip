@@ -293,7 +293,7 @@ __device__ __forceinline__ void store_sp_nt(void *__restrict__ base, int V, int 
 
 // Lane -> (mode m, site s, block blk) for the three traversals (TRAV_*).  The hardware hands
 // workgroup b to XCD b % 8; the XCD traversals undo that round-robin so that XCD k runs the
-// contiguous k-th eighth of the logical lanes:
+// contiguous k-th eighth of the logical workgroups (the grid is rounded up to whole eighths):
 //   TRAV_BOXES: the eighth is XCD k's spatial box of sites (order[k V/8 .. (k+1) V/8)), every
 //     mode block in turn, so x/y/z neighbours are re-read from that XCD's L2 except at the box
 //     faces;
@@ -666,8 +666,8 @@ __device__ __forceinline__ void hop_ens_tile(const HopArgs &a, int2 w)
     hop_site<NC, TI, TO, MB, EPI>(a, d.n0, d.n1, d.n2, Site{s, rem - y * d.n0, y, z}, d.q0 + blk * d.V, d.l0, m);
 }
 
-// Static table (ens_qctr null): workgroup b runs tile ens_work[b]; the host lays the table out so
-// that the tiles of one system all run on one XCD (whole systems per XCD L2, balanced by size).
+// Static table (ens_qctr null): workgroup b runs tile ens_work[b]; the host cuts the tiles of all systems,
+// system by system, into eight equal runs, one per XCD.
 // Work queues (ens_qctr set): a persistent grid; workgroup b claims ens_per tiles at a time from the
 // queue of XCD b % 8 until it is empty, so the tiles of an XCD's systems go to whichever of its
 // workgroups is free.  Every workgroup leaves when its queue is exhausted (no workgroup waits on
@@ -1948,8 +1948,7 @@ void hop_ens_wpe(const HopArgs &b, int wpe, hipStream_t st)
     hop_ens_wpe_epi<NC, TI, TO, MB, EPI_ANY>(b, wpe, st);
 }
 
-// the launch arguments of one lattice: lane coordinates, and the traversal where the launch splits evenly;
-// false when the lanes exceed 32 bits
+// the launch arguments of one lattice: lane coordinates and traversal; false when the lanes exceed 32 bits
 bool lattice_args(const Geom &g, const HopArgs &a, HopArgs &b, unsigned &nb)
 {
     const long total = (long)a.nblk * g.V * g.mb;
@@ -1961,10 +1960,10 @@ bool lattice_args(const Geom &g, const HopArgs &a, HopArgs &b, unsigned &nb)
     b.dv_v8 = make_fastdiv((unsigned)(g.V / NUM_XCD));
     b.dv_n01 = make_fastdiv((unsigned)(g.n0 * g.n1));
     b.dv_n0 = make_fastdiv((unsigned)g.n0);
-    // the XCD traversals need whole workgroups spread evenly over the XCDs
-    const bool even = total % ((long)TPB * NUM_XCD) == 0;
-    if (b.trav == TRAV_BOXES && (!even || g.V % NUM_XCD != 0 || (!b.order && b.box.dv_x.d == 0))) b.trav = TRAV_LEX;
-    if (b.trav == TRAV_MODES && !even) b.trav = TRAV_LEX;
+    // The XCD traversals give each XCD an eighth of the workgroups: the grid is rounded up to whole eighths
+    // (the last ones find no lanes).  A box of sites needs eight equal boxes.
+    if (b.trav == TRAV_BOXES && (g.V % NUM_XCD != 0 || (!b.order && b.box.dv_x.d == 0))) b.trav = TRAV_MODES;
+    if (b.trav != TRAV_LEX) nb = (nb + NUM_XCD - 1) / NUM_XCD * NUM_XCD;
     return true;
 }
 
