@@ -10,6 +10,7 @@
 #include <rocsolver/rocsolver.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <complex>
 #include <cstdio>
@@ -388,27 +389,35 @@ HopArgs hop_args(const ovl_ctx *c, int prec)
     return a;
 }
 
-// Site traversal for the XCD-aware stencil launches: the lattice is cut into 8 boxes (one per XCD,
-// px*py*pz = 8 dividing the extents, the split of the smallest box surface); inside a box the shorter of
-// the y/z box extents is cut into `sub` slabs, each walked with x fastest, then that extent, then the
-// other one, so the three planes a site's neighbours span (b_x * slab sites each) fit the XCD's L2.
+// Site traversal for the XCD-aware stencil launches: the lattice is cut into 8 boxes (px*py*pz = 8 dividing the
+// extents), one per XCD; inside a box the shorter of the y/z box extents is cut into `sub` slabs, each walked
+// with x fastest, then that extent, then the other one.  Of the splits with the smallest surface between boxes
+// (a direction that is not cut wraps around inside its box) the one with the smallest plane of that walk is
+// taken, along z where two are alike: the three planes a site's neighbours span are then likeliest to
+// stay in the XCD's L2.  Cubes are cut 2 x 4 x 1 by that; 2 x 2 x 2 has the same surface and planes twice as
+// large (us per Clenshaw step, 2 x 2 x 2 and 2 x 4 x 1: SU(3) 24^3, 64 modes FP64 234 and 231, 48-bit 193 and 187,
+// FP32 115 and 111; SU(2) 32^3, 64 modes 374 and 366, 302 and 293, 169 and 162; SU(3) 32^3, 32 modes 356 and 325,
+// 307 and 287, 150 and 148; SU(2) 16^3 and smaller alike).  1 x 1 x 8: 265, 208, 118; 439, 329, 175; 365, 310, 154.
 // Whole boxes (sub = 1) are computed by the kernel from `box`; slabs have a table.
 bool xcd_boxes(int n0, int n1, int n2, ovl::XcdBoxes *out)
 {
-    long best_cost = -1;
+    bool found = false;
+    std::array<long, 4> best{};
     for (int lx = 0; lx <= 3; ++lx)
         for (int ly = 0; lx + ly <= 3; ++ly) {
             const int px = 1 << lx, py = 1 << ly, pz = 8 >> (lx + ly);
             if (n0 % px || n1 % py || n2 % pz) continue;
             const long bx = n0 / px, by = n1 / py, bz = n2 / pz;
-            const long cost = bx * by + by * bz + bz * bx;
-            if (best_cost >= 0 && cost >= best_cost) continue;
-            best_cost = cost;
+            const long cut = (px > 1 ? by * bz : 0) + (py > 1 ? bz * bx : 0) + (pz > 1 ? bx * by : 0);
             const bool y_mid = by <= bz;
+            const std::array<long, 4> cost{cut, bx * std::min(by, bz), y_mid ? 0 : 1, px};
+            if (found && cost >= best) continue;
+            found = true;
+            best = cost;
             *out = ovl::XcdBoxes{lx, ly, (int)by, (int)bz, y_mid, ovl::make_fastdiv((unsigned)bx),
                                  ovl::make_fastdiv((unsigned)(bx * (y_mid ? by : bz)))};
         }
-    return best_cost >= 0;
+    return found;
 }
 
 std::vector<int> xcd_site_order(int n0, int n1, int n2, int sub)
