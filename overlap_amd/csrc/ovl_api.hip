@@ -2749,19 +2749,6 @@ static int noalloc_scratch(double **out)
     return OVL_OK;
 }
 
-// raw reduction results -> the quantities of ovl_system_observables, in the same arithmetic
-__global__ void k_obs_noalloc_finish(const double *raw, double *obs, double n_adj_v, double three_v)
-{
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    obs[OVL_OBS_E_EL] = raw[0];
-    obs[OVL_OBS_E_MAG] = raw[1];
-    obs[OVL_OBS_GAUSS_MAX] = raw[2];
-    obs[OVL_OBS_GAUSS_RMS] = sqrt(raw[3] / n_adj_v);
-    obs[OVL_OBS_UNIT_MAX] = raw[4];
-    obs[OVL_OBS_UNIT_RMS] = sqrt(raw[5] / three_v);
-    obs[OVL_OBS_NCS_DOT] = 0.125 * raw[6] / (M_PI * M_PI);  // ChernSimonsDerivative.cpp:47
-}
-
 int ovl_observables_noalloc(int nc, const int *n, const double *links, const double *efield, double *obs,
                             void *stream)
 {
@@ -2787,11 +2774,7 @@ int ovl_observables_noalloc(int nc, const int *n, const double *links, const dou
     RETCHK(noalloc_scratch(&s));
     double *raw = s + NOALLOC_RAW;
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    hipError_t e = ovl::launch_observables(g, links, efield, ovl::OBS_LOCAL | ovl::OBS_EDOTB, nullptr, s, raw, st);
-    if (e == hipSuccess) {
-        k_obs_noalloc_finish<<<1, 64, 0, st>>>(raw, obs, (double)(nc * nc - 1) * (double)V, 3.0 * (double)V);
-        e = hipGetLastError();
-    }
+    const hipError_t e = ovl::launch_observables(g, links, efield, ovl::OBS_LOCAL | ovl::OBS_EDOTB, nullptr, s, raw, st, obs);
     if (e != hipSuccess) return free_fail(OVL_E_HIP, std::string("ovl_observables_noalloc: ") + hipGetErrorString(e));
     return OVL_OK;
 }

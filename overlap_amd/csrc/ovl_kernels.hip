@@ -4,6 +4,7 @@
 // covers 64 consecutive (mode, site) lanes of one mode block, so every 16-byte load of a spinor
 // component is one contiguous MB*16-byte segment.  Links are shared by all modes of a site and
 // read once per wavefront (MB = 64) or once per MB-lane group.
+#include "../../include/ovl.h"
 #include "ovl_internal.hpp"
 
 #include <algorithm>
@@ -1401,18 +1402,19 @@ template <int NC> __device__ __forceinline__ void alg_components(const Mat<NC> &
 // g (optional): G^a(x) stored as [site][a]; GAUSS_ONLY leaves the other two out.  24^3 SU(3): 9.7 us where
 // three kernels and their finishing passes took 37 us.
 enum { LOC_EEL = 0, LOC_EMAG, LOC_GMAX, LOC_GSUM, LOC_UMAX, LOC_USUM, LOC_COUNT };
-template <int NC, bool GAUSS_ONLY>
-__global__ __launch_bounds__(TPB) void k_obs_local(const double *__restrict__ links, const double *__restrict__ e,
-                                                   double *partial, double *__restrict__ g, int n0, int n1, int n2)
+template <int NC, bool GAUSS_ONLY, int NT>
+__device__ __forceinline__ void obs_local(int wg, int wgs, const double *__restrict__ links,
+                                          const double *__restrict__ e, double *partial, double *__restrict__ g, int n0,
+                                          int n1, int n2)
 {
     const int V = n0 * n1 * n2;
     constexpr int NG = NC * NC - 1;
     double v[LOC_COUNT] = {0, 0, 0, 0, 0, 0};
     const int mu = threadIdx.x % 4;
     const bool dir = mu < 3;
-    const int stride = (int)gridDim.x * (TPB / 4);
-    // the four lanes of a site share the loop condition
-    for (int s = (int)blockIdx.x * (TPB / 4) + threadIdx.x / 4; s < V; s += stride) {
+    const int stride = wgs * (TPB / 4);
+    // the four lanes of a site share the loop condition; threads beyond TPB only join the reduction
+    for (int s = threadIdx.x < TPB ? wg * (TPB / 4) + (int)threadIdx.x / 4 : V; s < V; s += stride) {
         double comp[NG];
 #pragma unroll
         for (int a = 0; a < NG; ++a) comp[a] = 0;
@@ -1473,16 +1475,24 @@ __global__ __launch_bounds__(TPB) void k_obs_local(const double *__restrict__ li
     v[LOC_EEL] *= 0.5;
     v[LOC_EMAG] *= 0.5;
     const int ism[LOC_COUNT] = {0, 0, 1, 0, 1, 0};
-    block_reduce<LOC_COUNT>(v, ism);
+    block_reduce<LOC_COUNT, NT>(v, ism);
     if (threadIdx.x == 0)
 #pragma unroll
-        for (int k = 0; k < LOC_COUNT; ++k) partial[(size_t)blockIdx.x * LOC_COUNT + k] = v[k];
+        for (int k = 0; k < LOC_COUNT; ++k) partial[(size_t)wg * LOC_COUNT + k] = v[k];
+}
+template <int NC, bool GAUSS_ONLY>
+__global__ __launch_bounds__(TPB) void k_obs_local(const double *__restrict__ links, const double *__restrict__ e,
+                                                   double *partial, double *__restrict__ g, int n0, int n1, int n2)
+{
+    obs_local<NC, GAUSS_ONLY, TPB>((int)blockIdx.x, (int)gridDim.x, links, e, partial, g, n0, n1, n2);
 }
 
-// the partial results of k_obs_local (nl of them; none when 0) and of k_edotb (ne; likewise), summed in a
-// fixed order: out[0 .. LOC_COUNT) and out[LOC_COUNT]
+// the partial results of the local observables (nl of them; none when 0) and of E.B (ne; likewise), summed in a
+// fixed order: out[0 .. LOC_COUNT) and out[LOC_COUNT]; `derived` (optional, with both): the quantities of
+// ovl_system_observables from them
 __global__ __launch_bounds__(TPB) void k_obs_finish(const double *__restrict__ local, int nl,
-                                                    const double *__restrict__ edotb, int ne, double *out)
+                                                    const double *__restrict__ edotb, int ne, double *out,
+                                                    double *derived, double n_adj_v, double three_v)
 {
     const int ism[LOC_COUNT + 1] = {0, 0, 1, 0, 1, 0, 0};
     double v[LOC_COUNT + 1] = {0, 0, 0, 0, 0, 0, 0};
@@ -1499,6 +1509,15 @@ __global__ __launch_bounds__(TPB) void k_obs_finish(const double *__restrict__ l
 #pragma unroll
             for (int k = 0; k < LOC_COUNT; ++k) out[k] = v[k];
         if (ne > 0) out[LOC_COUNT] = v[LOC_COUNT];
+        if (derived) {
+            derived[OVL_OBS_E_EL] = v[RAW_EEL];
+            derived[OVL_OBS_E_MAG] = v[RAW_EMAG];
+            derived[OVL_OBS_GAUSS_MAX] = v[RAW_GMAX];
+            derived[OVL_OBS_GAUSS_RMS] = sqrt(v[RAW_GSUM] / n_adj_v);
+            derived[OVL_OBS_UNIT_MAX] = v[RAW_UMAX];
+            derived[OVL_OBS_UNIT_RMS] = sqrt(v[RAW_USUM] / three_v);
+            derived[OVL_OBS_NCS_DOT] = 0.125 * v[RAW_EDOTB] / (M_PI * M_PI);  // ChernSimonsDerivative.cpp:47
+        }
     }
 }
 
@@ -1584,9 +1603,11 @@ template <int NC> __device__ __forceinline__ Row<NC> row_add(const Row<NC> &x, d
 __device__ __forceinline__ int wrap(int c, int n) { return c < 0 ? c + n : (c >= n ? c - n : c); }  // |offset| <= 2 < n
 
 constexpr int EB_TPB = 5 * 64;  // four quadrants and E
+// two waves per SIMD for SU(3): three or four spill (24^3: 65, 119 and 136 us)
+template <int NC> constexpr int EB_WPE = NC == 3 ? 2 : 4;
 template <int NC>
-__global__ __launch_bounds__(EB_TPB) void k_edotb(const double *__restrict__ links, const double *__restrict__ e,
-                                                  double *partial, int n0, int n1, int n2)
+__device__ __forceinline__ void edotb(int wg, int wgs, const double *__restrict__ links, const double *__restrict__ e,
+                                      double *partial, int n0, int n1, int n2)
 {
     constexpr int NG = NC * NC - 1, PAIRS = 64 / NC;
     constexpr double W4 = 5.0 / 12.0, W6 = -1.0 / 24.0;
@@ -1597,7 +1618,7 @@ __global__ __launch_bounds__(EB_TPB) void k_edotb(const double *__restrict__ lin
     const int pair = used ? lane / NC : PAIRS - 1, row = used ? lane % NC : 0;
     double acc[1] = {0.0};
     const int npairs = 3 * V;
-    for (int base = (int)blockIdx.x * PAIRS; base < npairs; base += (int)gridDim.x * PAIRS) {
+    for (int base = wg * PAIRS; base < npairs; base += wgs * PAIRS) {
         const int gi = base + pair;
         const int gc = gi < npairs ? gi : npairs - 1;  // spare lanes repeat the last pair's work
         const bool ok = used && gi < npairs;
@@ -1701,7 +1722,26 @@ __global__ __launch_bounds__(EB_TPB) void k_edotb(const double *__restrict__ lin
     }
     const int ism[1] = {0};
     block_reduce<1, EB_TPB>(acc, ism);
-    if (threadIdx.x == 0) partial[blockIdx.x] = acc[0];
+    if (threadIdx.x == 0) partial[wg] = acc[0];
+}
+template <int NC>
+__global__ __launch_bounds__(EB_TPB) __attribute__((amdgpu_waves_per_eu(EB_WPE<NC>))) void k_edotb(
+    const double *__restrict__ links, const double *__restrict__ e, double *partial, int n0, int n1, int n2)
+{
+    edotb<NC>((int)blockIdx.x, (int)gridDim.x, links, e, partial, n0, n1, n2);
+}
+
+// The local observables (the first nl workgroups, their fifth wavefront idle) and E.B in one launch: small lattices
+// are bound by the launches.  All seven observables queued, in four launches and in two with k_obs_finish:
+// 14.0 and 8.2 us on 8^3 SU(2), 19.8 and 11.4 us on 8^3 SU(3), 67.3 and 64.5 us on 24^3 SU(3).
+template <int NC>
+__global__ __launch_bounds__(EB_TPB) __attribute__((amdgpu_waves_per_eu(EB_WPE<NC>))) void k_observables(
+    const double *__restrict__ links, const double *__restrict__ e, double *local, int nl, double *eb,
+    double *__restrict__ g, int n0, int n1, int n2)
+{
+    const int wg = (int)blockIdx.x;
+    if (wg < nl) obs_local<NC, false, EB_TPB>(wg, nl, links, e, local, g, n0, n1, n2);
+    else edotb<NC>(wg - nl, (int)gridDim.x - nl, links, e, eb, n0, n1, n2);
 }
 
 // per-mode inner products: partial[chunk][mode] then a fixed-order sum over chunks
@@ -2344,31 +2384,37 @@ hipError_t launch_mode_dot(const Geom &g, const void *a, const void *b, double *
     return hipGetLastError();
 }
 
-// partial results of the observables: LOC_BLOCKS x LOC_COUNT of k_obs_local, then EB_BLOCKS of k_edotb
+// partial results of the observables: LOC_BLOCKS x LOC_COUNT of the local ones, then EB_BLOCKS of E.B
 // (fixed upper limits: the static scratch of ovl_observables_noalloc holds them too)
 constexpr int LOC_BLOCKS = 256, EB_BLOCKS = 2048;
 static_assert(LOC_COUNT + 1 == OBS_RAW, "raw observables");
 size_t reduce_partial_len(const Geom &) { return (size_t)LOC_BLOCKS * LOC_COUNT + EB_BLOCKS; }
 
 hipError_t launch_observables(const Geom &g, const double *links, const double *efield, int what, double *gfield,
-                              double *partial, double *out, hipStream_t st)
+                              double *partial, double *out, hipStream_t st, double *derived)
 {
     const int nl = (int)std::min<long>(LOC_BLOCKS, (4L * g.V + TPB - 1) / TPB);
     const int ne = (int)std::min<long>(EB_BLOCKS, (3L * g.V + 64 / g.nc - 1) / (64 / g.nc));
     double *pe = partial + (size_t)LOC_BLOCKS * LOC_COUNT;
-    if (what & OBS_EDOTB) {
+    const bool all = (what & OBS_LOCAL) && (what & OBS_EDOTB);
+    if (derived && !(all && out)) return hipErrorInvalidValue;
+    if (all) {
+        if (g.nc == 2) k_observables<2><<<nl + ne, EB_TPB, 0, st>>>(links, efield, partial, nl, pe, gfield, g.n0, g.n1, g.n2);
+        else k_observables<3><<<nl + ne, EB_TPB, 0, st>>>(links, efield, partial, nl, pe, gfield, g.n0, g.n1, g.n2);
+    } else if (what & OBS_EDOTB) {
         if (g.nc == 2) k_edotb<2><<<ne, EB_TPB, 0, st>>>(links, efield, pe, g.n0, g.n1, g.n2);
         else k_edotb<3><<<ne, EB_TPB, 0, st>>>(links, efield, pe, g.n0, g.n1, g.n2);
     }
-    if (what & OBS_LOCAL) {
+    if (!all && (what & OBS_LOCAL)) {
         if (g.nc == 2) k_obs_local<2, false><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
         else k_obs_local<3, false><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
-    } else if (what & OBS_GAUSS) {
+    } else if (!all && (what & OBS_GAUSS)) {
         if (g.nc == 2) k_obs_local<2, true><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
         else k_obs_local<3, true><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
     }
     if (out)
-        k_obs_finish<<<1, TPB, 0, st>>>(partial, what & (OBS_LOCAL | OBS_GAUSS) ? nl : 0, pe, what & OBS_EDOTB ? ne : 0, out);
+        k_obs_finish<<<1, TPB, 0, st>>>(partial, what & (OBS_LOCAL | OBS_GAUSS) ? nl : 0, pe, what & OBS_EDOTB ? ne : 0, out,
+                                        derived, (double)(g.nc * g.nc - 1) * (double)g.V, 3.0 * (double)g.V);
     return hipGetLastError();
 }
 
