@@ -8,8 +8,9 @@ namespace ovl {
 
 // Ordered after the work queued on `st`; returns when the copy is complete.  Arrays of at least HOSTCOPY_MIN
 // bytes whose pages do not exist yet go through a ring of pinned buffers that a few host threads empty
-// while the DMA engine fills the next ones; all others, and copies that find the ring in use by another
-// host thread, are a plain hipMemcpyAsync and a synchronisation.
+// while the DMA engine fills the next ones; all others (memory that the HIP runtime knows among them), and
+// copies that find the ring in use by another host thread, are a plain hipMemcpyAsync and a
+// synchronisation.
 hipError_t copy_to_host(void *host, const void *dev, size_t bytes, hipStream_t st);
 
 // The ring and its threads belong to the process: made by the first copy that wants them, given back when
@@ -20,3 +21,7 @@ void hostcopy_release();
 constexpr size_t HOSTCOPY_MIN = (size_t)1 << 20;
 
 }  // namespace ovl
+
+// copies of this process that took the ring (not in ovl.h: which way a copy goes does not show in its result,
+// the tests ask here)
+extern "C" long ovl_hostcopy_ring_copies();
