@@ -1,6 +1,7 @@
 """GPU tests of the way a result takes to the host: which arrays go through the ring of pinned buffers and
 which are copied directly.  The results are the same bytes either way."""
 import ctypes as C
+import mmap
 
 import numpy as np
 import pytest
@@ -48,3 +49,36 @@ def test_pinned_arrays_are_copied_directly(gpu, count, touched):
         read_modes(ctx, out.data_ptr(), count)
         assert ring_copies() == before
         assert np.array_equal(out.numpy(), psi)
+
+
+# fresh anonymous pages: below the line, at it, one ring of 16 chunks, a chunk more, several rings
+@pytest.mark.parametrize("count,rings", [(1, 0), (2, 1), (16, 1), (17, 1), (40, 1)])
+def test_fresh_arrays_take_the_ring(gpu, count, rings):
+    print(f"[case] fresh read-back {count} MiB", flush=True)
+    ctx, psi = context(count)
+    with ctx:
+        fresh = mmap.mmap(-1, count * MIB)
+        buf = (C.c_char * (count * MIB)).from_buffer(fresh)
+        before = ring_copies()
+        read_modes(ctx, C.addressof(buf), count)
+        assert ring_copies() == before + rings
+        assert bytes(buf) == psi.tobytes()
+        read_modes(ctx, C.addressof(buf), count)  # the pages exist now
+        assert ring_copies() == before + rings
+        assert bytes(buf) == psi.tobytes()
+
+
+@pytest.mark.parametrize("n", [(24, 32, 40), (31, 33, 47)])  # links in 96 bytes a site: broken last chunks
+def test_broken_last_chunk(gpu, n):
+    print(f"[case] fresh read-back of links {n}", flush=True)
+    links = cf.su2_links(n, 0.3, cf.rng(n[2]))
+    assert links.nbytes > 2 * MIB and links.nbytes % MIB
+    with ovl.Context(2, n, 1) as ctx:
+        ctx.set_links(links)
+        fresh = mmap.mmap(-1, links.nbytes)
+        buf = (C.c_char * links.nbytes).from_buffer(fresh)
+        before = ring_copies()
+        rc = ovl.lib().ovl_get_links(ctx.h, C.cast(C.c_void_p(C.addressof(buf)), C.POINTER(C.c_double)))
+        assert rc == ovl.OK, rc
+        assert ring_copies() == before + 1
+        assert bytes(buf) == links.tobytes()
