@@ -14,10 +14,14 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <condition_variable>
+#include <cstdlib>
 #include <cstring>
+#include <fstream>
 #include <mutex>
 #include <new>
+#include <string>
 #include <thread>
 #include <vector>
 
@@ -28,12 +32,46 @@ namespace {
 constexpr size_t CHUNK = (size_t)1 << 20;
 constexpr int SLOTS = 16, MAX_WORKERS = 8;
 
-int cpus_allowed()
+// whole CPUs of the quota in a control group's directory (version 2: cpu.max "QUOTA PERIOD", version 1: two
+// files); a large number without one
+int group_quota(const std::string &dir)
+{
+    constexpr int NONE = 1 << 20;
+    double quota = -1, period = -1;
+    std::ifstream max(dir + "/cpu.max");
+    if (max) {
+        std::string q;
+        max >> q >> period;
+        if (q != "max") quota = std::atof(q.c_str());
+    } else {
+        std::ifstream(dir + "/cpu.cfs_quota_us") >> quota;
+        std::ifstream(dir + "/cpu.cfs_period_us") >> period;
+    }
+    if (!(quota > 0 && period > 0)) return NONE;
+    return (int)std::min<double>(NONE, std::max(1.0, std::floor(quota / period)));
+}
+
+// the smallest quota of the process's control group and those above it
+int quota_cpus(const std::string &root)
+{
+    int cpus = std::min(group_quota(root), std::min(group_quota(root + "/cpu"), group_quota(root + "/cpu,cpuacct")));
+    std::ifstream self("/proc/self/cgroup");
+    for (std::string line; std::getline(self, line);) {
+        if (line.compare(0, 3, "0::") != 0) continue;
+        for (std::string path = line.substr(3); path.size() > 1; path.resize(path.rfind('/')))
+            cpus = std::min(cpus, group_quota(root + path));
+    }
+    return cpus;
+}
+
+// More spinning threads than the process may run at once would be stopped by the scheduler in the middle of a
+// copy, so a container's quota counts as much as the affinity mask.
+int cpus_allowed(const char *cgroup_root)
 {
     cpu_set_t set;
     CPU_ZERO(&set);
     if (sched_getaffinity(0, sizeof set, &set) != 0) return 1;
-    return CPU_COUNT(&set);
+    return std::min(CPU_COUNT(&set), quota_cpus(cgroup_root ? cgroup_root : "/sys/fs/cgroup"));
 }
 
 // whether the HIP runtime knows the memory (pinned, managed or device memory): the DMA reaches it without a
@@ -89,7 +127,7 @@ public:
     // null when the process has no second core, or no pinned memory or threads are to be had
     static Ring *make()
     {
-        const int nw = std::min(MAX_WORKERS, cpus_allowed() - 1);
+        const int nw = std::min(MAX_WORKERS, cpus_allowed(nullptr) - 1);
         if (nw < 1) return nullptr;
         Ring *r = new (std::nothrow) Ring;
         if (!r) return nullptr;
@@ -286,3 +324,5 @@ void hostcopy_release()
 }  // namespace ovl
 
 extern "C" long ovl_hostcopy_ring_copies() { return ovl::g_copies.load(std::memory_order_relaxed); }
+
+extern "C" int ovl_hostcopy_cpus(const char *cgroup_root) { return ovl::cpus_allowed(cgroup_root); }

@@ -27,3 +27,7 @@ constexpr size_t HOSTCOPY_MIN = (size_t)2 << 20;
 // copies of this process that took the ring (not in ovl.h: which way a copy goes does not show in its result,
 // the tests ask here)
 extern "C" long ovl_hostcopy_ring_copies();
+
+// the CPUs this process may keep busy: those of its affinity mask, or fewer by the CPU quota of its control
+// group (cgroup_root: where the hierarchy is mounted; null: /sys/fs/cgroup)
+extern "C" int ovl_hostcopy_cpus(const char *cgroup_root);
