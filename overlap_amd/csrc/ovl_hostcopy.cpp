@@ -19,6 +19,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <fstream>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -129,8 +130,9 @@ public:
     {
         const int nw = std::min(MAX_WORKERS, cpus_allowed(nullptr) - 1);
         if (nw < 1) return nullptr;
-        Ring *r = new (std::nothrow) Ring;
-        if (!r) return nullptr;
+        std::unique_ptr<Ring> r(new Ring);
+        r->events_.reserve(SLOTS);
+        r->threads_.reserve((size_t)nw);
         bool ok = hipHostMalloc((void **)&r->pinned_, CHUNK * SLOTS, hipHostMallocDefault) == hipSuccess;
         if (!ok) (void)hipGetLastError();
         for (int k = 0; ok && k < SLOTS; ++k) {
@@ -141,14 +143,12 @@ public:
         ok = ok && hipGetDevice(&r->device_) == hipSuccess;
         if (ok) {
             try {
-                for (int k = 0; k < nw; ++k) r->threads_.emplace_back([r] { r->worker(); });
+                for (int k = 0; k < nw; ++k) r->threads_.emplace_back([p = r.get()] { p->worker(); });
             } catch (...) {  // std::system_error: no more threads
                 ok = !r->threads_.empty();
             }
         }
-        if (ok) return r;
-        delete r;
-        return nullptr;
+        return ok ? r.release() : nullptr;
     }
 
     ~Ring()
@@ -297,9 +297,12 @@ hipError_t copy_to_host(void *host, const void *dev, size_t bytes, hipStream_t s
 {
     if (bytes >= HOSTCOPY_MIN && untouched(host, bytes) && !known_to_hip(host)) {
         std::unique_lock<std::mutex> lock;
-        if (Ring *r = take_ring(lock)) {
-            g_copies.fetch_add(1, std::memory_order_relaxed);
-            return r->to_host((char *)host, (const char *)dev, bytes, st);
+        try {
+            if (Ring *r = take_ring(lock)) {
+                g_copies.fetch_add(1, std::memory_order_relaxed);
+                return r->to_host((char *)host, (const char *)dev, bytes, st);
+            }
+        } catch (const std::bad_alloc &) {  // of the ring or of the job, before any thread has the job
         }
     }
     const hipError_t e = hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);
