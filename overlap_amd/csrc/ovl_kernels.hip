@@ -933,18 +933,28 @@ template <int NC> __device__ __forceinline__ Mat<NC> mid()
     return c;
 }
 
+// first double of link (s, mu) in the reference format.  54 doubles a site in SU(3): a 32-bit product overflows from
+// 2^31 / 54 = 39.8 million sites on
+template <int NC> __host__ __device__ constexpr size_t link_at(int s, int mu)
+{
+    return (size_t)(NC == 2 ? 4 : 18) * (mu + 3 * (size_t)s);
+}
+static_assert(link_at<3>(OVL_NOALLOC_MAX_SITES - 1, 2) + 18 == 54ull * OVL_NOALLOC_MAX_SITES &&
+                  link_at<2>(OVL_NOALLOC_MAX_SITES - 1, 2) + 4 == 12ull * OVL_NOALLOC_MAX_SITES,
+              "the last link of the largest lattice");
+
 // master link (reference format) -> row-major matrix
 template <int NC> __device__ __forceinline__ Mat<NC> get_link(const double *__restrict__ links, int s, int mu)
 {
     Mat<NC> m;
     if constexpr (NC == 2) {
-        const double *u = links + 4 * (mu + 3 * s);  // GetMatrix, SU2/GroupOperations.cpp:213-225
+        const double *u = links + link_at<2>(s, mu);  // GetMatrix, SU2/GroupOperations.cpp:213-225
         m.e[0] = {u[3], u[2]};
         m.e[1] = {u[1], u[0]};
         m.e[2] = {-u[1], u[0]};
         m.e[3] = {u[3], -u[2]};
     } else {
-        const double *u = links + 18 * (mu + 3 * s);
+        const double *u = links + link_at<3>(s, mu);
 #pragma unroll
         for (int i = 0; i < 3; ++i)
 #pragma unroll
@@ -1442,7 +1452,7 @@ __device__ __forceinline__ void obs_local(int wg, int wgs, const double *__restr
                 v[LOC_EMAG] += 4.0 * tr;
                 double nrm;
                 if constexpr (NC == 2) {  // UnitarityNorm (SU2/GroupOperations.cpp:172-184)
-                    const double *u = links + 4 * (mu + 3 * (size_t)s);
+                    const double *u = links + link_at<2>(s, mu);
                     const double c3 = u[3] * u[3] + u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
                     nrm = fabs(c3 - 1.0);
                 } else {
