@@ -254,7 +254,7 @@ int ovl_system_observables(ovl_ctx *ctx, int sys, double *obs);
  * values ovl_system_observables returns for the same fields, bit for bit.  The kernels are queued on
  * `stream` (a hipStream_t of the current device; NULL = its default stream) and the call returns
  * without waiting.  It
- * calls no allocator: the reductions' partial results live in a static 32 KiB array per device,
+ * calls no allocator: the reductions' partial results live in a static 64 KiB array per device,
  * shared by every call on that device, so calls that overlap on one device (other streams, other
  * threads) race and must be ordered by the caller.  At most OVL_NOALLOC_MAX_SITES sites; larger
  * lattices, nc other than 2/3 or an extent below 3 return OVL_E_ARG, and ovl_error(NULL) then gives

@@ -2628,7 +2628,7 @@ static int fetch_out(ovl_ctx *c, double *h, int n)
     return OVL_OK;
 }
 
-// the raw observables `what` (ovl::OBS_*) of system s, one synchronisation
+// the raw observables `what` (one ovl::OBS_*) of system s, one synchronisation
 static int obs_raw(ovl_ctx *c, int s, int what, double *raw)
 {
     if (!c->sys_links_set[s]) return fail(c, OVL_E_STATE, "no gauge links uploaded");
@@ -2660,7 +2660,7 @@ int ovl_energy(ovl_ctx *c, double *e_el, double *e_mag)
     if (!c || !e_el || !e_mag) return OVL_E_ARG;
     RETCHK(single_lattice(c, "ovl_energy"));
     double h[ovl::OBS_RAW];
-    RETCHK(obs_raw(c, 0, ovl::OBS_LOCAL, h));
+    RETCHK(obs_raw(c, 0, ovl::OBS_ENERGY, h));
     *e_el = h[ovl::RAW_EEL];
     *e_mag = h[ovl::RAW_EMAG];
     return OVL_OK;
@@ -2682,7 +2682,7 @@ int ovl_unitarity_violation(ovl_ctx *c, double *vmax, double *vrms)
     if (!c || !vmax || !vrms) return OVL_E_ARG;
     RETCHK(single_lattice(c, "ovl_unitarity_violation"));
     double h[ovl::OBS_RAW];
-    RETCHK(obs_raw(c, 0, ovl::OBS_LOCAL, h));
+    RETCHK(obs_raw(c, 0, ovl::OBS_UNITARITY, h));
     *vmax = h[ovl::RAW_UMAX];
     *vrms = unitarity_rms(c, 0, h);
     return OVL_OK;
@@ -2700,7 +2700,7 @@ int ovl_system_observables(ovl_ctx *c, int sys, double *obs)
     if (!c || !obs) return OVL_E_ARG;
     RETCHK(check_sys(c, sys));
     double h[ovl::OBS_RAW];
-    RETCHK(obs_raw(c, sys, ovl::OBS_LOCAL | ovl::OBS_EDOTB, h));
+    RETCHK(obs_raw(c, sys, ovl::OBS_ALL, h));
     obs[OVL_OBS_E_EL] = h[ovl::RAW_EEL];
     obs[OVL_OBS_E_MAG] = h[ovl::RAW_EMAG];
     obs[OVL_OBS_GAUSS_MAX] = h[ovl::RAW_GMAX];
@@ -2712,13 +2712,13 @@ int ovl_system_observables(ovl_ctx *c, int sys, double *obs)
 }
 
 // ---- allocation-free observables ----
-// The reductions' per-workgroup partial results (ovl::reduce_partial_len doubles) and the four raw
+// The reductions' per-workgroup partial results (ovl::reduce_partial_len doubles) and the seven raw
 // results live in this file-scope device array instead of a context's buffers.  Each device holds
 // its own copy; host code uses only the address hipGetSymbolAddress returns for the current device.
 // Every reduction writes all the partial results its finishing pass reads (a fixed grid), so the
 // array needs no clearing between calls; calls that overlap on one device share it and race.
-constexpr size_t NOALLOC_SCRATCH_DOUBLES = 4096;  // 32 KiB per device
-constexpr size_t NOALLOC_RAW = NOALLOC_SCRATCH_DOUBLES - 8;  // raw results: scratch[NOALLOC_RAW .. +7)
+constexpr size_t NOALLOC_RAW = 8192;  // 64 KiB of partial results per device, then the raw ones: scratch[NOALLOC_RAW .. +7)
+constexpr size_t NOALLOC_SCRATCH_DOUBLES = NOALLOC_RAW + 8;
 static __device__ __align__(256) double scratch[NOALLOC_SCRATCH_DOUBLES];
 
 constexpr int NOALLOC_MAX_DEVICES = 64;
@@ -2774,7 +2774,7 @@ int ovl_observables_noalloc(int nc, const int *n, const double *links, const dou
     RETCHK(noalloc_scratch(&s));
     double *raw = s + NOALLOC_RAW;
     const hipStream_t st = static_cast<hipStream_t>(stream);
-    const hipError_t e = ovl::launch_observables(g, links, efield, ovl::OBS_LOCAL | ovl::OBS_EDOTB, nullptr, s, raw, st, obs);
+    const hipError_t e = ovl::launch_observables(g, links, efield, ovl::OBS_ALL, nullptr, s, raw, st, obs);
     if (e != hipSuccess) return free_fail(OVL_E_HIP, std::string("ovl_observables_noalloc: ") + hipGetErrorString(e));
     return OVL_OK;
 }

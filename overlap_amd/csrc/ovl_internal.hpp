@@ -160,12 +160,13 @@ hipError_t launch_hop_gauge(const Geom &g, int prec, const HopArgs &a, const Gau
 hipError_t launch_mode_dot(const Geom &g, const void *a, const void *b, double *partial, double *out,
                            hipStream_t st);
 size_t mode_dot_partial_len(const Geom &g);
-// Global observables, `what` a sum of OBS_*: the raw results of those asked for go to out[OBS_RAW] (device;
-// null: none) in the order (1/2) sum E^2, magnetic energy, max |G|, sum G^2, max and sum of squares of the
-// unitarity norm, sum E.B.  gfield (optional, with OBS_GAUSS or OBS_LOCAL): G^a(x) stored as [site][a].  derived
-// (optional, device, with OBS_LOCAL, OBS_EDOTB and out): the OVL_OBS_COUNT quantities of ovl_system_observables.
+// Global observables: one of OBS_ENERGY, OBS_GAUSS, OBS_UNITARITY, OBS_EDOTB, or OBS_ALL; the raw results of
+// what is asked for go to their places in out[OBS_RAW] (device; null: none): (1/2) sum E^2, magnetic energy,
+// max |G|, sum G^2, max and sum of squares of the unitarity norm, sum E.B.  gfield (optional, with
+// OBS_GAUSS): G^a(x) stored as [site][a].  derived (optional, device, with OBS_ALL and out): the
+// OVL_OBS_COUNT quantities of ovl_system_observables.
 constexpr int OBS_RAW = 7;
-enum { OBS_LOCAL = 1, OBS_GAUSS = 2, OBS_EDOTB = 4 };
+enum { OBS_ENERGY = 1, OBS_GAUSS = 2, OBS_UNITARITY = 4, OBS_EDOTB = 8, OBS_LOCAL = 7, OBS_ALL = 15 };
 enum { RAW_EEL = 0, RAW_EMAG, RAW_GMAX, RAW_GSUM, RAW_UMAX, RAW_USUM, RAW_EDOTB };
 hipError_t launch_observables(const Geom &g, const double *links, const double *efield, int what, double *gfield,
                               double *partial, double *out, hipStream_t st, double *derived = nullptr);

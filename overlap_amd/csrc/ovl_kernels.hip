@@ -1370,14 +1370,16 @@ __device__ __forceinline__ double wave_max(double v)
     return v;
 }
 
-// block reduction of NV values (sum or max per value) in a workgroup of NT threads; result valid in
-// thread 0
-template <int NV, int NT = TPB> __device__ void block_reduce(double *v, const int *is_max)
+// block reduction of NV values (sum or max per value; those of `mask`) in a workgroup of NT threads; result
+// valid in thread 0
+template <int NV, int NT = TPB>
+__device__ __forceinline__ void block_reduce(double *v, const int *is_max, unsigned mask = (1u << NV) - 1)
 {
     __shared__ double sh[NT / 64][NV];
     const int w = threadIdx.x / 64, l = threadIdx.x % 64;
 #pragma unroll
-    for (int k = 0; k < NV; ++k) v[k] = is_max[k] ? wave_max(v[k]) : wave_sum(v[k]);
+    for (int k = 0; k < NV; ++k)
+        if (mask >> k & 1) v[k] = is_max[k] ? wave_max(v[k]) : wave_sum(v[k]);
     if (l == 0)
 #pragma unroll
         for (int k = 0; k < NV; ++k) sh[w][k] = v[k];
@@ -1409,10 +1411,17 @@ template <int NC> __device__ __forceinline__ void alg_components(const Mat<NC> &
 //   max |G^a| and sum G^2 of G(x) = sum_mu E_mu(x) - U_mu(x-mu)^+ E_mu(x-mu) U_mu(x-mu)
 //                                                             (GaussLawViolation.cpp:13-61)
 //   max and sum of the squares of ||U U^+ - 1||               (UnitarityViolation.cpp:13-51)
-// g (optional): G^a(x) stored as [site][a]; GAUSS_ONLY leaves the other two out.  24^3 SU(3): 9.7 us where
-// three kernels and their finishing passes took 37 us.
+// `what` (a sum of OBS_ENERGY, OBS_GAUSS, OBS_UNITARITY) leaves out the others; each quantity is the same sums
+// either way.  g (optional): G^a(x) stored as [site][a].  24^3 SU(3): 9.7 us for all where three kernels and
+// their finishing passes took 37 us.  Up to LOC_BLOCKS workgroups of 64 sites: see there.
 enum { LOC_EEL = 0, LOC_EMAG, LOC_GMAX, LOC_GSUM, LOC_UMAX, LOC_USUM, LOC_COUNT };
-template <int NC, bool GAUSS_ONLY, int NT>
+// the LOC_* values (bits) that the observables `what` have
+constexpr unsigned loc_mask(int what)
+{
+    return (what & OBS_ENERGY ? 3u << LOC_EEL : 0) | (what & OBS_GAUSS ? 3u << LOC_GMAX : 0) |
+           (what & OBS_UNITARITY ? 3u << LOC_UMAX : 0);
+}
+template <int NC, int WHAT, int NT>
 __device__ __forceinline__ void obs_local(int wg, int wgs, const double *__restrict__ links,
                                           const double *__restrict__ e, double *partial, double *__restrict__ g, int n0,
                                           int n1, int n2)
@@ -1429,15 +1438,17 @@ __device__ __forceinline__ void obs_local(int wg, int wgs, const double *__restr
 #pragma unroll
         for (int a = 0; a < NG; ++a) comp[a] = 0;
         if (dir) {
-            const int sm = nbr(s, mu, -1, n0, n1, n2);
-            const Mat<NC> e0 = alg_to_mat<NC>(e + (size_t)NG * (mu + 3 * (size_t)s));
-            const Mat<NC> e1 = alg_to_mat<NC>(e + (size_t)NG * (mu + 3 * (size_t)sm));
-            const Mat<NC> ub = get_link<NC>(links, sm, mu);
-            Mat<NC> t = mmul<NC>(mmul<NC>(mdag<NC>(ub), e1), ub);
+            if constexpr (WHAT & OBS_GAUSS) {
+                const int sm = nbr(s, mu, -1, n0, n1, n2);
+                const Mat<NC> e0 = alg_to_mat<NC>(e + (size_t)NG * (mu + 3 * (size_t)s));
+                const Mat<NC> e1 = alg_to_mat<NC>(e + (size_t)NG * (mu + 3 * (size_t)sm));
+                const Mat<NC> ub = get_link<NC>(links, sm, mu);
+                Mat<NC> t = mmul<NC>(mmul<NC>(mdag<NC>(ub), e1), ub);
 #pragma unroll
-            for (int k = 0; k < NC * NC; ++k) t.e[k] = {e0.e[k].r - t.e[k].r, e0.e[k].i - t.e[k].i};
-            alg_components<NC>(t, comp);
-            if constexpr (!GAUSS_ONLY) {
+                for (int k = 0; k < NC * NC; ++k) t.e[k] = {e0.e[k].r - t.e[k].r, e0.e[k].i - t.e[k].i};
+                alg_components<NC>(t, comp);
+            }
+            if constexpr (WHAT & OBS_ENERGY) {
                 for (int a = 0; a < NG; ++a) {
                     const double q = e[(size_t)NG * (mu + 3 * (size_t)s) + a];
                     v[LOC_EEL] += q * q;
@@ -1450,6 +1461,8 @@ __device__ __forceinline__ void obs_local(int wg, int wgs, const double *__restr
 #pragma unroll
                 for (int i = 0; i < NC; ++i) tr += 1.0 - p.e[i * NC + i].r;
                 v[LOC_EMAG] += 4.0 * tr;
+            }
+            if constexpr (WHAT & OBS_UNITARITY) {
                 double nrm;
                 if constexpr (NC == 2) {  // UnitarityNorm (SU2/GroupOperations.cpp:172-184)
                     const double *u = links + link_at<2>(s, mu);
@@ -1470,55 +1483,61 @@ __device__ __forceinline__ void obs_local(int wg, int wgs, const double *__restr
                 v[LOC_USUM] += nrm * nrm;
             }
         }
+        if constexpr (WHAT & OBS_GAUSS)
 #pragma unroll
-        for (int a = 0; a < NG; ++a) {
-            comp[a] += __shfl_xor(comp[a], 1, 64);
-            comp[a] += __shfl_xor(comp[a], 2, 64);
-            if (a % 4 == mu) {  // every lane of the site holds G^a: each keeps its share
-                if (g) g[(size_t)NG * s + a] = comp[a];
-                const double q = fabs(comp[a]);
-                v[LOC_GMAX] = fmax(v[LOC_GMAX], q);
-                v[LOC_GSUM] += q * q;
+            for (int a = 0; a < NG; ++a) {
+                comp[a] += __shfl_xor(comp[a], 1, 64);
+                comp[a] += __shfl_xor(comp[a], 2, 64);
+                if (a % 4 == mu) {  // every lane of the site holds G^a: each keeps its share
+                    if (g) g[(size_t)NG * s + a] = comp[a];
+                    const double q = fabs(comp[a]);
+                    v[LOC_GMAX] = fmax(v[LOC_GMAX], q);
+                    v[LOC_GSUM] += q * q;
+                }
             }
-        }
     }
     v[LOC_EEL] *= 0.5;
     v[LOC_EMAG] *= 0.5;
     const int ism[LOC_COUNT] = {0, 0, 1, 0, 1, 0};
-    block_reduce<LOC_COUNT, NT>(v, ism);
+    block_reduce<LOC_COUNT, NT>(v, ism, loc_mask(WHAT));
     if (threadIdx.x == 0)
 #pragma unroll
-        for (int k = 0; k < LOC_COUNT; ++k) partial[(size_t)wg * LOC_COUNT + k] = v[k];
+        for (int k = 0; k < LOC_COUNT; ++k)
+            if (loc_mask(WHAT) >> k & 1) partial[(size_t)wg * LOC_COUNT + k] = v[k];
 }
-template <int NC, bool GAUSS_ONLY>
+template <int NC, int WHAT>
 __global__ __launch_bounds__(TPB) void k_obs_local(const double *__restrict__ links, const double *__restrict__ e,
                                                    double *partial, double *__restrict__ g, int n0, int n1, int n2)
 {
-    obs_local<NC, GAUSS_ONLY, TPB>((int)blockIdx.x, (int)gridDim.x, links, e, partial, g, n0, n1, n2);
+    obs_local<NC, WHAT, TPB>((int)blockIdx.x, (int)gridDim.x, links, e, partial, g, n0, n1, n2);
 }
 
-// the partial results of the local observables (nl of them; none when 0) and of E.B (ne; likewise), summed in a
-// fixed order: out[0 .. LOC_COUNT) and out[LOC_COUNT]; `derived` (optional, with both): the quantities of
-// ovl_system_observables from them
+// the partial results of the local observables of WHAT (nl workgroups') and of E.B (ne, with OBS_EDOTB), summed in
+// a fixed order: out[0 .. LOC_COUNT) and out[LOC_COUNT]; `derived` (optional, with all of them): the
+// quantities of ovl_system_observables from them
+template <int WHAT>
 __global__ __launch_bounds__(TPB) void k_obs_finish(const double *__restrict__ local, int nl,
                                                     const double *__restrict__ edotb, int ne, double *out,
                                                     double *derived, double n_adj_v, double three_v)
 {
+    constexpr unsigned MASK = loc_mask(WHAT) | (WHAT & OBS_EDOTB ? 1u << LOC_COUNT : 0);
     const int ism[LOC_COUNT + 1] = {0, 0, 1, 0, 1, 0, 0};
     double v[LOC_COUNT + 1] = {0, 0, 0, 0, 0, 0, 0};
-    for (int b = threadIdx.x; b < nl; b += TPB)
+    if constexpr (loc_mask(WHAT) != 0)
+        for (int b = threadIdx.x; b < nl; b += TPB)
 #pragma unroll
-        for (int k = 0; k < LOC_COUNT; ++k) {
-            const double p = local[(size_t)b * LOC_COUNT + k];
-            v[k] = ism[k] ? fmax(v[k], p) : v[k] + p;
-        }
-    for (int b = threadIdx.x; b < ne; b += TPB) v[LOC_COUNT] += edotb[b];
-    block_reduce<LOC_COUNT + 1>(v, ism);
+            for (int k = 0; k < LOC_COUNT; ++k)
+                if (MASK >> k & 1) {
+                    const double p = local[(size_t)b * LOC_COUNT + k];
+                    v[k] = ism[k] ? fmax(v[k], p) : v[k] + p;
+                }
+    if constexpr ((WHAT & OBS_EDOTB) != 0)
+        for (int b = threadIdx.x; b < ne; b += TPB) v[LOC_COUNT] += edotb[b];
+    block_reduce<LOC_COUNT + 1>(v, ism, MASK);
     if (threadIdx.x == 0) {
-        if (nl > 0)
 #pragma unroll
-            for (int k = 0; k < LOC_COUNT; ++k) out[k] = v[k];
-        if (ne > 0) out[LOC_COUNT] = v[LOC_COUNT];
+        for (int k = 0; k <= LOC_COUNT; ++k)
+            if (MASK >> k & 1) out[k] = v[k];
         if (derived) {
             derived[OVL_OBS_E_EL] = v[RAW_EEL];
             derived[OVL_OBS_E_MAG] = v[RAW_EMAG];
@@ -1741,17 +1760,24 @@ __global__ __launch_bounds__(EB_TPB) __attribute__((amdgpu_waves_per_eu(EB_WPE<N
     edotb<NC>((int)blockIdx.x, (int)gridDim.x, links, e, partial, n0, n1, n2);
 }
 
-// The local observables (the first nl workgroups, their fifth wavefront idle) and E.B in one launch: small lattices
-// are bound by the launches.  All seven observables queued, in four launches and in two with k_obs_finish:
-// 14.0 and 8.2 us on 8^3 SU(2), 19.8 and 11.4 us on 8^3 SU(3), 67.3 and 64.5 us on 24^3 SU(3).
+// The local observables (the first nb workgroups, their fifth wavefront idle, take the nl shares of k_obs_local in
+// turn, so that the sums are its sums) and E.B in one launch: small lattices are bound by the launches.  All
+// seven observables queued, in four launches and in two with k_obs_finish: 14.0 and 8.2 us on 8^3 SU(2), 19.8 and
+// 11.4 us on 8^3 SU(3), 67.3 and 64.5 us on 24^3 SU(3).  More than OBS_BLOCKS workgroups only displace those of E.B
+// (a workgroup for each of up to 1020 shares: SU(2) 48^3 93 -> 102 us, SU(3) 32^3 134 -> 140 us).
+constexpr int OBS_BLOCKS = 256;
 template <int NC>
 __global__ __launch_bounds__(EB_TPB) __attribute__((amdgpu_waves_per_eu(EB_WPE<NC>))) void k_observables(
-    const double *__restrict__ links, const double *__restrict__ e, double *local, int nl, double *eb,
+    const double *__restrict__ links, const double *__restrict__ e, double *local, int nl, int nb, double *eb,
     double *__restrict__ g, int n0, int n1, int n2)
 {
     const int wg = (int)blockIdx.x;
-    if (wg < nl) obs_local<NC, false, EB_TPB>(wg, nl, links, e, local, g, n0, n1, n2);
-    else edotb<NC>(wg - nl, (int)gridDim.x - nl, links, e, eb, n0, n1, n2);
+    if (wg < nb)
+        for (int w = wg; w < nl; w += nb) {
+            obs_local<NC, OBS_LOCAL, EB_TPB>(w, nl, links, e, local, g, n0, n1, n2);
+            __syncthreads();  // the reduction's LDS is free again
+        }
+    else edotb<NC>(wg - nb, (int)gridDim.x - nb, links, e, eb, n0, n1, n2);
 }
 
 // per-mode inner products: partial[chunk][mode] then a fixed-order sum over chunks
@@ -2395,37 +2421,52 @@ hipError_t launch_mode_dot(const Geom &g, const void *a, const void *b, double *
 }
 
 // partial results of the observables: LOC_BLOCKS x LOC_COUNT of the local ones, then EB_BLOCKS of E.B
-// (fixed upper limits: the static scratch of ovl_observables_noalloc holds them too)
-constexpr int LOC_BLOCKS = 256, EB_BLOCKS = 2048;
+// (fixed upper limits: the static scratch of ovl_observables_noalloc holds them too).  A workgroup of the local ones
+// has 64 sites at a time; with 256 of them at most, lattices from 32^3 on left the chip half empty (SU(2) 64^3, a
+// call with its synchronisation: energy 62.8 us and Gauss law 48.4 us; with 1024 workgroups and nothing
+// else computed 37.3 and 38.8; the unitarity norm 61.7 and 27.0).
+constexpr int LOC_BLOCKS = 1024, EB_BLOCKS = 2048;
 static_assert(LOC_COUNT + 1 == OBS_RAW, "raw observables");
 size_t reduce_partial_len(const Geom &) { return (size_t)LOC_BLOCKS * LOC_COUNT + EB_BLOCKS; }
+
+template <int NC, int WHAT>
+static hipError_t observables(const Geom &g, const double *links, const double *efield, double *gfield, double *partial,
+                              double *out, double *derived, hipStream_t st)
+{
+    const int nl = (int)std::min<long>(LOC_BLOCKS, (4L * g.V + TPB - 1) / TPB);
+    const int nb = std::min(nl, OBS_BLOCKS);
+    const int ne = (int)std::min<long>(EB_BLOCKS, (3L * g.V + 64 / NC - 1) / (64 / NC));
+    double *pe = partial + (size_t)LOC_BLOCKS * LOC_COUNT;
+    if constexpr (WHAT == OBS_ALL)
+        k_observables<NC><<<nb + ne, EB_TPB, 0, st>>>(links, efield, partial, nl, nb, pe, gfield, g.n0, g.n1, g.n2);
+    else if constexpr (WHAT == OBS_EDOTB) k_edotb<NC><<<ne, EB_TPB, 0, st>>>(links, efield, pe, g.n0, g.n1, g.n2);
+    else k_obs_local<NC, WHAT><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
+    if (out)
+        k_obs_finish<WHAT><<<1, TPB, 0, st>>>(partial, nl, pe, ne, out, derived, (double)(NC * NC - 1) * (double)g.V,
+                                              3.0 * (double)g.V);
+    return hipGetLastError();
+}
+
+template <int NC>
+static hipError_t observables_nc(const Geom &g, const double *links, const double *efield, int what, double *gfield,
+                                 double *partial, double *out, double *derived, hipStream_t st)
+{
+    switch (what) {
+    case OBS_ENERGY: return observables<NC, OBS_ENERGY>(g, links, efield, gfield, partial, out, nullptr, st);
+    case OBS_GAUSS: return observables<NC, OBS_GAUSS>(g, links, efield, gfield, partial, out, nullptr, st);
+    case OBS_UNITARITY: return observables<NC, OBS_UNITARITY>(g, links, efield, gfield, partial, out, nullptr, st);
+    case OBS_EDOTB: return observables<NC, OBS_EDOTB>(g, links, efield, gfield, partial, out, nullptr, st);
+    case OBS_ALL: return observables<NC, OBS_ALL>(g, links, efield, gfield, partial, out, derived, st);
+    default: return hipErrorInvalidValue;
+    }
+}
 
 hipError_t launch_observables(const Geom &g, const double *links, const double *efield, int what, double *gfield,
                               double *partial, double *out, hipStream_t st, double *derived)
 {
-    const int nl = (int)std::min<long>(LOC_BLOCKS, (4L * g.V + TPB - 1) / TPB);
-    const int ne = (int)std::min<long>(EB_BLOCKS, (3L * g.V + 64 / g.nc - 1) / (64 / g.nc));
-    double *pe = partial + (size_t)LOC_BLOCKS * LOC_COUNT;
-    const bool all = (what & OBS_LOCAL) && (what & OBS_EDOTB);
-    if (derived && !(all && out)) return hipErrorInvalidValue;
-    if (all) {
-        if (g.nc == 2) k_observables<2><<<nl + ne, EB_TPB, 0, st>>>(links, efield, partial, nl, pe, gfield, g.n0, g.n1, g.n2);
-        else k_observables<3><<<nl + ne, EB_TPB, 0, st>>>(links, efield, partial, nl, pe, gfield, g.n0, g.n1, g.n2);
-    } else if (what & OBS_EDOTB) {
-        if (g.nc == 2) k_edotb<2><<<ne, EB_TPB, 0, st>>>(links, efield, pe, g.n0, g.n1, g.n2);
-        else k_edotb<3><<<ne, EB_TPB, 0, st>>>(links, efield, pe, g.n0, g.n1, g.n2);
-    }
-    if (!all && (what & OBS_LOCAL)) {
-        if (g.nc == 2) k_obs_local<2, false><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
-        else k_obs_local<3, false><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
-    } else if (!all && (what & OBS_GAUSS)) {
-        if (g.nc == 2) k_obs_local<2, true><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
-        else k_obs_local<3, true><<<nl, TPB, 0, st>>>(links, efield, partial, gfield, g.n0, g.n1, g.n2);
-    }
-    if (out)
-        k_obs_finish<<<1, TPB, 0, st>>>(partial, what & (OBS_LOCAL | OBS_GAUSS) ? nl : 0, pe, what & OBS_EDOTB ? ne : 0, out,
-                                        derived, (double)(g.nc * g.nc - 1) * (double)g.V, 3.0 * (double)g.V);
-    return hipGetLastError();
+    if (derived && !(what == OBS_ALL && out)) return hipErrorInvalidValue;
+    return g.nc == 2 ? observables_nc<2>(g, links, efield, what, gfield, partial, out, derived, st)
+                     : observables_nc<3>(g, links, efield, what, gfield, partial, out, derived, st);
 }
 
 hipError_t launch_gauss_restore(const Geom &g, const double *links, const double *gfield, double *efield, double gamma,
