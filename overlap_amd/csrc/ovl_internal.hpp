@@ -147,6 +147,7 @@ struct GaugeHalf {
     float *ul32;
     double dt;
     int reunit, n0, n1, n2, V, what;
+    int lpl;     // lanes per link
     int blocks;  // workgroups of a shared launch
 };
 GaugeHalf gauge_half_args(const Geom &g, int what, double *links, double *efield, double dt, int reunit, const double *phase,

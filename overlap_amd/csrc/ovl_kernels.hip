@@ -1049,17 +1049,27 @@ __device__ __forceinline__ Mat<3> gather_columns(const cd *c)
     return m;
 }
 
+// the same from one lane's three columns
+__device__ __forceinline__ Mat<3> from_columns(const cd (&c)[3][3])
+{
+    Mat<3> m;
+#pragma unroll
+    for (int j = 0; j < 3; ++j)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) m.e[i * 3 + j] = c[j][i];
+    return m;
+}
+
 // 1/k of the Taylor series (a division would be as long as the product it scales)
 __device__ const double inverse_of[21] = {0.0,      1.0,      1.0 / 2,  1.0 / 3,  1.0 / 4,  1.0 / 5,  1.0 / 6,
                                           1.0 / 7,  1.0 / 8,  1.0 / 9,  1.0 / 10, 1.0 / 11, 1.0 / 12, 1.0 / 13,
                                           1.0 / 14, 1.0 / 15, 1.0 / 16, 1.0 / 17, 1.0 / 18, 1.0 / 19, 1.0 / 20};
 
-// column `col` of exp(i c alpha^a t^a): scaling and squaring of the Taylor series (FP64).  The columns of
-// the Horner form are independent, so three of four lanes walk one each: a third of the 20 matrix
-// products' chain per lane, the sums of the one-lane form unchanged.
-__device__ void iexp_column(double c, const double *alpha, int col, cd *r)
+// exp(i c alpha^a t^a) by scaling and squaring of the Taylor series (FP64): the scaled matrix and the number of
+// squarings
+__device__ __forceinline__ int iexp_scale(double c, const double *alpha, Mat<3> &a)
 {
-    Mat<3> a = alg_to_mat<3>(alpha);
+    a = alg_to_mat<3>(alpha);
     double nrm = 0;
 #pragma unroll
     for (int i = 0; i < 9; ++i) {
@@ -1072,7 +1082,11 @@ __device__ void iexp_column(double c, const double *alpha, int col, cd *r)
     const double sc = ldexp(1.0, -sq);
 #pragma unroll
     for (int i = 0; i < 9; ++i) { a.e[i].r *= sc; a.e[i].i *= sc; }
-    // Horner: I + a(1 + a/2(1 + a/3(...)))
+    return sq;
+}
+// column `col` of the series, Horner: I + a(1 + a/2(1 + a/3(...))).  The columns are independent.
+__device__ __forceinline__ void iexp_series(const Mat<3> &a, int col, cd *r)
+{
     const double one[3] = {col == 0 ? 1.0 : 0.0, col == 1 ? 1.0 : 0.0, col == 2 ? 1.0 : 0.0};
 #pragma unroll
     for (int i = 0; i < 3; ++i) r[i] = {one[i], 0.0};
@@ -1081,10 +1095,6 @@ __device__ void iexp_column(double c, const double *alpha, int col, cd *r)
         const double f = inverse_of[k];
 #pragma unroll
         for (int i = 0; i < 3; ++i) r[i] = {__builtin_fma(f, r[i].r, one[i]), f * r[i].i};
-    }
-    for (int k = 0; k < sq; ++k) {  // sq is the same in the four lanes of a link
-        const Mat<3> m = gather_columns(r);
-        mcol<true>(m, r);
     }
 }
 
@@ -1183,17 +1193,18 @@ __global__ __launch_bounds__(TPB) void k_ucc_setup(const double2 *__restrict__ u
 
 // Dynamics.cpp:97-138: U <- exp(i cU E) U with cU = -dt.  With u64 the new stencil links are written in the
 // same pass (the leapfrog's half step: one launch instead of two, and the links are not read again).
-// A workgroup is one wavefront, so that a small lattice spreads over the CUs.  SU(3): four lanes per
-// link, the first three a column each (iexp_column).  With a lane per link and the stencil links apart:
-// 11.1 + 4.8 us on 15 x 12 x 10 (the serial chain in 22 workgroups) and 14.1 + 7.5 us on 24^3 SU(3); now
-// 5.7 and 15.7 us (24^3: 25 MB read and written in 144-byte strides).
+// A workgroup is one wavefront, so that a small lattice spreads over the CUs.  SU(3): LPL = 4 lanes per
+// link, the first three a column each: a third of the chain of 20 matrix products per lane.  With a lane per
+// link and the stencil links apart: 11.1 + 4.8 us on 15 x 12 x 10 (the serial chain in 22 workgroups) and
+// 14.1 + 7.5 us on 24^3 SU(3); so 5.7 and 15.7 us (24^3: 25 MB read and written in 144-byte strides).  LPL = 1, the
+// same sums in one lane, does not pay for the fourth lane and the exchanges of the others: ovl_update_links with
+// LPL = 4 and 1, 24^3 23.1 and 23.5 us, 32^3 33.2 and 31.8, 40^3 54.5 and 44.1, 56^3 123 and 96.
 constexpr int LINK_TPB = 64;
-template <int NC>
+template <int NC, int LPL>
 __device__ __forceinline__ void link_update_lane(unsigned lane, double *__restrict__ links, const double *__restrict__ e,
                                                  double dt, int V, int reunit, const double2 *__restrict__ phase,
                                                  double2 *__restrict__ u64, float2 *__restrict__ u32)
 {
-    constexpr int LPL = NC == 2 ? 1 : 4;  // lanes per link
     const int i = (int)(lane / LPL);
     if (i >= 3 * V) return;  // the lanes of a link leave together
     const int s = i / 3, mu = i - 3 * s;  // link (s, mu) at index mu + 3 s
@@ -1231,11 +1242,51 @@ __device__ __forceinline__ void link_update_lane(unsigned lane, double *__restri
             put_stencil_entry<true>(ph, cd{-n1, n0}, u64, u32, (size_t)iu * 4 + 2);
             put_stencil_entry<false>(ph, cd{n3, -n2}, u64, u32, (size_t)iu * 4 + 3);
         }
+    } else if constexpr (LPL == 1) {
+        double *u = links + 18 * (size_t)i;
+        Mat<3> a;
+        const int sq = iexp_scale(c, al, a);
+        cd r[3][3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) iexp_series(a, j, r[j]);
+        for (int k = 0; k < sq; ++k) {
+            a = from_columns(r);
+#pragma unroll
+            for (int j = 0; j < 3; ++j) mcol<true>(a, r[j]);
+        }
+        a = from_columns(r);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) r[j][k] = {u[6 * j + 2 * k], u[6 * j + 2 * k + 1]};
+            mcol<false>(a, r[j]);
+        }
+        a = from_columns(r);
+        if (reunit) a = reunit3(a);
+#pragma unroll
+        for (int j = 0; j < 3; ++j)
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                u[6 * j + 2 * k] = a.e[3 * k + j].r;
+                u[6 * j + 2 * k + 1] = a.e[3 * k + j].i;
+            }
+        if (u64) {
+            const int iu = mu * V + s;
+            const cd ph = phase_of(phase, iu);
+#pragma unroll
+            for (int k = 0; k < 9; ++k) put_stencil_entry<false>(ph, a.e[k], u64, u32, (size_t)iu * 9 + k);
+        }
     } else {
         const int col = threadIdx.x % 4 < 3 ? threadIdx.x % 4 : 0;  // the fourth lane repeats the first
         double *u = links + 18 * (size_t)i + 6 * col;
+        Mat<3> a;
+        const int sq = iexp_scale(c, al, a);
         cd ex[3], r[3];
-        iexp_column(c, al, col, ex);
+        iexp_series(a, col, ex);
+        for (int k = 0; k < sq; ++k) {  // sq is the same in the four lanes of a link
+            const Mat<3> m = gather_columns(ex);
+            mcol<true>(m, ex);
+        }
 #pragma unroll
         for (int k = 0; k < 3; ++k) r[k] = {u[2 * k], u[2 * k + 1]};
         mcol<false>(gather_columns(ex), r);
@@ -1258,10 +1309,10 @@ __device__ __forceinline__ void link_update_lane(unsigned lane, double *__restri
         }
     }
 }
-template <int NC>
+template <int NC, int LPL>
 __global__ __launch_bounds__(LINK_TPB) void k_link_update(GaugeHalf g)
 {
-    link_update_lane<NC>(blockIdx.x * LINK_TPB + threadIdx.x, g.links, g.efield, g.dt, g.V, g.reunit,
+    link_update_lane<NC, LPL>(blockIdx.x * LINK_TPB + threadIdx.x, g.links, g.efield, g.dt, g.V, g.reunit,
                          (const double2 *)g.phase, (double2 *)g.ul64, (float2 *)g.ul32);
 }
 
@@ -1277,21 +1328,20 @@ __device__ __forceinline__ int nbr(int s, int dmu, int step, int n0, int n1, int
 // E_mu(x) += dt * (-2) sum_{nu != mu} [ReTr(i t^a U_{mu nu}(x)) + ReTr(i t^a U_{mu,-nu}(x))]
 // (Hamilton's equation of H = 1/2 E^2 + 2 sum ReTr(1 - U_plaq) for U' = -i E U; the
 // reference's plaquette macros used by Dynamics.cpp:145-197 are absent)
-// Four lanes per link, one plaquette each (two planes, forward and backward), their components summed
+// Four lanes per link (LPL = 4), one plaquette each (two planes, forward and backward), their components summed
 // from the four lanes: a lane's chain is three matrix products instead of twelve (SU(3): 14.1 -> 7.3 us on
 // 15 x 12 x 10, where a lane per link left most CUs without a wave, 17.8 -> 15.3 us on 24^3, where the
-// matrices' strided loads bound it).
+// matrices' strided loads bound it).  The lanes of a wavefront then walk both the forward and the backward
+// products; with LPL = 1, one lane and the same sums, none does: ovl_update_efield
+// with LPL = 4 and 1, SU(2) 16^3 14.8 and 15.5 us, 24^3 17.3 and 15.9, 32^3 21.3 and 17.9, 64^3 72 and 46.  SU(3)
+// has four lanes throughout: in one lane 24^3 takes 24.5 us instead of 23.7, 48^3 97.6 instead of 88.4.
+
+// sums of ReTr(i t^a U_plaq) (retr_sums) of plaquette j of link (s, mu): plane (mu, the j/2-th other direction), j odd:
+// the backward one
 template <int NC>
-__device__ __forceinline__ void efield_update_lane(unsigned lane, const double *__restrict__ links, double *__restrict__ e,
-                                                   double dt, int n0, int n1, int n2)
+__device__ __forceinline__ void plaquette_sums(const double *__restrict__ links, int s, int mu, int j, int n0, int n1, int n2,
+                                               double *f)
 {
-    const int V = n0 * n1 * n2;
-    const int j = threadIdx.x % 4;
-    const int i = (int)(lane / 4);
-    const bool ok = i < 3 * V;
-    const int il = ok ? i : 3 * V - 1;
-    const int s = il / 3, mu = il - 3 * s;
-    constexpr int NG = NC * NC - 1;
     const int nu = j < 2 ? (mu == 0 ? 1 : 0) : (mu == 2 ? 1 : 2);  // the two other directions, ascending
     const bool back = j & 1;
     const int sp = nbr(s, mu, 1, n0, n1, n2);
@@ -1308,25 +1358,56 @@ __device__ __forceinline__ void efield_update_lane(unsigned lane, const double *
         p = mmul<NC>(p, mdag<NC>(get_link<NC>(links, nbr(s, nu, 1, n0, n1, n2), mu)));
         p = mmul<NC>(p, mdag<NC>(get_link<NC>(links, s, nu)));
     }
-    double f[NG];
     retr_sums<NC>(p, f);
-    const int base = (int)(threadIdx.x & 60);
-#pragma unroll
-    for (int k = 0; k < NG; ++k) {  // in the order of the planes
-        double t = 0;
-#pragma unroll
-        for (int l = 0; l < 4; ++l) t = __builtin_fma(retr_factor(k), __shfl(f[k], base + l, 64), t);
-        f[k] = t;
-    }
-    if (!ok) return;
-    double *o = e + (size_t)NG * i;
-#pragma unroll
-    for (int k = 0; k < NG; ++k)
-        if (k % 4 == j) o[k] += -2.0 * dt * f[k];
 }
-template <int NC> __global__ __launch_bounds__(LINK_TPB) void k_efield_update(GaugeHalf g)
+template <int NC, int LPL>
+__device__ __forceinline__ void efield_update_lane(unsigned lane, const double *__restrict__ links, double *__restrict__ e,
+                                                   double dt, int n0, int n1, int n2)
 {
-    efield_update_lane<NC>(blockIdx.x * LINK_TPB + threadIdx.x, g.links, g.efield, g.dt, g.n0, g.n1, g.n2);
+    const int V = n0 * n1 * n2;
+    const int i = (int)(lane / LPL);
+    constexpr int NG = NC * NC - 1;
+    if constexpr (LPL == 1) {
+        if (i >= 3 * V) return;
+        const int s = i / 3, mu = i - 3 * s;
+        double t[NG];
+#pragma unroll
+        for (int k = 0; k < NG; ++k) t[k] = 0;
+#pragma unroll
+        for (int l = 0; l < 4; ++l) {
+            double f[NG];
+            plaquette_sums<NC>(links, s, mu, l, n0, n1, n2, f);
+#pragma unroll
+            for (int k = 0; k < NG; ++k) t[k] = __builtin_fma(retr_factor(k), f[k], t[k]);
+        }
+        double *o = e + (size_t)NG * i;
+#pragma unroll
+        for (int k = 0; k < NG; ++k) o[k] += -2.0 * dt * t[k];
+    } else {
+        const int j = threadIdx.x % 4;
+        const bool ok = i < 3 * V;
+        const int il = ok ? i : 3 * V - 1;
+        const int s = il / 3, mu = il - 3 * s;
+        double f[NG];
+        plaquette_sums<NC>(links, s, mu, j, n0, n1, n2, f);
+        const int base = (int)(threadIdx.x & 60);
+#pragma unroll
+        for (int k = 0; k < NG; ++k) {  // in the order of the planes
+            double t = 0;
+#pragma unroll
+            for (int l = 0; l < 4; ++l) t = __builtin_fma(retr_factor(k), __shfl(f[k], base + l, 64), t);
+            f[k] = t;
+        }
+        if (!ok) return;
+        double *o = e + (size_t)NG * i;
+#pragma unroll
+        for (int k = 0; k < NG; ++k)
+            if (k % 4 == j) o[k] += -2.0 * dt * f[k];
+    }
+}
+template <int NC, int LPL> __global__ __launch_bounds__(LINK_TPB) void k_efield_update(GaugeHalf g)
+{
+    efield_update_lane<NC, LPL>(blockIdx.x * LINK_TPB + threadIdx.x, g.links, g.efield, g.dt, g.n0, g.n1, g.n2);
 }
 
 // A Wilson half step and a gauge half step in one launch: the first gauge.blocks workgroups (a multiple of the
@@ -1339,10 +1420,10 @@ __global__ __launch_bounds__(TPB) void k_hop_gauge(HopArgs a, GaugeHalf g, int n
     if (blockIdx.x < (unsigned)g.blocks) {
         const unsigned lane = blockIdx.x * TPB + threadIdx.x;
         if (g.what == GAUGE_LINKS_HALF)
-            link_update_lane<NC>(lane, g.links, g.efield, g.dt, g.V, g.reunit, (const double2 *)g.phase, (double2 *)g.ul64,
-                                 (float2 *)g.ul32);
-        else
-            efield_update_lane<NC>(lane, g.links, g.efield, g.dt, n0, n1, n2);
+            link_update_lane<NC, NC == 2 ? 1 : 4>(lane, g.links, g.efield, g.dt, g.V, g.reunit, (const double2 *)g.phase,
+                                                  (double2 *)g.ul64, (float2 *)g.ul32);
+        else if (NC == 2 && g.lpl == 1) efield_update_lane<NC, NC == 2 ? 1 : 4>(lane, g.links, g.efield, g.dt, n0, n1, n2);
+        else efield_update_lane<NC, 4>(lane, g.links, g.efield, g.dt, n0, n1, n2);
         return;
     }
     const int V = n0 * n1 * n2;
@@ -2360,33 +2441,47 @@ hipError_t launch_ucc_to_links(const Geom &g, const double *ucc, double *ul64, f
     return hipGetLastError();
 }
 
-// lanes of a gauge half step: SU(2) links one each, SU(3) links and E fields four
-static long gauge_lanes(const Geom &g, int what) { return 3L * g.V * (what == GAUGE_LINKS_HALF && g.nc == 2 ? 1 : 4); }
+// Lanes per link of a gauge half step: four while they are needed to fill the chip, else one (link_update_lane,
+// efield_update_lane; SU(2) links are always one).  The lines lie where the two cross: SU(2) E fields between 16^3
+// and 18^3 (18^3: 15.8 and 15.7 us), SU(3) links alone at 32^3, with the stencil links, whose stores are better
+// spread over four lanes, between 40^3 and 44^3 (a Wilson step of one FP32 mode with E moving: 40^3 335 and 333 us,
+// 36^3 242 and 247, 44^3 449 and 446).
+constexpr long ONE_LANE_EFIELD_SU2 = 16384, ONE_LANE_LINKS_SU3 = 90000, ONE_LANE_STENCIL_SU3 = 200000;
+static int lanes_per_link(const Geom &g, int what, bool stencil)
+{
+    const long links = 3L * g.V;
+    if (g.nc == 2) return what == GAUGE_LINKS_HALF || links > ONE_LANE_EFIELD_SU2 ? 1 : 4;
+    return what == GAUGE_LINKS_HALF && links > (stencil ? ONE_LANE_STENCIL_SU3 : ONE_LANE_LINKS_SU3) ? 1 : 4;
+}
 
 GaugeHalf gauge_half_args(const Geom &g, int what, double *links, double *efield, double dt, int reunit, const double *phase,
                           double *ul64, float *ul32)
 {
-    const long nb = (gauge_lanes(g, what) + TPB - 1) / TPB;
-    return GaugeHalf{links, efield, phase, ul64, ul32, dt, reunit, g.n0, g.n1, g.n2, g.V, what,
-                     (int)((nb + NUM_XCD - 1) / NUM_XCD * NUM_XCD)};
+    return GaugeHalf{links, efield, phase, ul64, ul32, dt, reunit, g.n0, g.n1, g.n2, g.V, what, lanes_per_link(g, what, ul64 != nullptr), 0};
 }
 
 hipError_t launch_gauge_half(const Geom &g, const GaugeHalf &h, hipStream_t st)
 {
-    const unsigned nb = (unsigned)((gauge_lanes(g, h.what) + LINK_TPB - 1) / LINK_TPB);
+    const unsigned nb = (unsigned)((3L * g.V * h.lpl + LINK_TPB - 1) / LINK_TPB);
     if (h.what == GAUGE_LINKS_HALF) {
-        if (g.nc == 2) k_link_update<2><<<nb, LINK_TPB, 0, st>>>(h);
-        else k_link_update<3><<<nb, LINK_TPB, 0, st>>>(h);
+        if (g.nc == 2) k_link_update<2, 1><<<nb, LINK_TPB, 0, st>>>(h);
+        else if (h.lpl == 1) k_link_update<3, 1><<<nb, LINK_TPB, 0, st>>>(h);
+        else k_link_update<3, 4><<<nb, LINK_TPB, 0, st>>>(h);
     } else {
-        if (g.nc == 2) k_efield_update<2><<<nb, LINK_TPB, 0, st>>>(h);
-        else k_efield_update<3><<<nb, LINK_TPB, 0, st>>>(h);
+        if (g.nc == 3) k_efield_update<3, 4><<<nb, LINK_TPB, 0, st>>>(h);
+        else if (h.lpl == 1) k_efield_update<2, 1><<<nb, LINK_TPB, 0, st>>>(h);
+        else k_efield_update<2, 4><<<nb, LINK_TPB, 0, st>>>(h);
     }
     return hipGetLastError();
 }
 
-hipError_t launch_hop_gauge(const Geom &g, int prec, const HopArgs &a, const GaugeHalf &h, hipStream_t st)
+hipError_t launch_hop_gauge(const Geom &g, int prec, const HopArgs &a, const GaugeHalf &half, hipStream_t st)
 {
     if (a.ens_sys || epi_kind(a) != EPI_AXPY) return hipErrorInvalidValue;
+    GaugeHalf h = half;
+    if (g.nc == 3) h.lpl = 4;  // the exponential in one lane would take the stencil's registers
+    const long nb = (3L * g.V * h.lpl + TPB - 1) / TPB;
+    h.blocks = (int)((nb + NUM_XCD - 1) / NUM_XCD * NUM_XCD);
     if (g.nc == 2) return prec == P64 ? hop_gauge_mb<2, double>(g, a, h, st) : hop_gauge_mb<2, float>(g, a, h, st);
     return prec == P64 ? hop_gauge_mb<3, double>(g, a, h, st) : hop_gauge_mb<3, float>(g, a, h, st);
 }
