@@ -392,17 +392,23 @@ HopArgs hop_args(const ovl_ctx *c, int prec)
 // Site traversal for the XCD-aware stencil launches: the lattice is cut into 8 boxes (px*py*pz = 8 dividing the
 // extents), one per XCD; inside a box the shorter of the y/z box extents is cut into `sub` slabs, each walked
 // with x fastest, then that extent, then the other one.  Of the splits with the smallest surface between boxes
-// (a direction that is not cut wraps around inside its box) the one with the smallest plane of that walk is
-// taken, along z where two are alike: the three planes a site's neighbours span are then likeliest to
-// stay in the XCD's L2.  Cubes are cut 2 x 4 x 1 by that; 2 x 2 x 2 has the same surface and planes twice as
-// large (us per Clenshaw step, 2 x 2 x 2 and 2 x 4 x 1: SU(3) 24^3, 64 modes FP64 234 and 231, 48-bit 193 and 187,
-// FP32 115 and 111; SU(2) 32^3, 64 modes 374 and 366, 302 and 293, 169 and 162; SU(3) 32^3, 32 modes 356 and 325,
-// 307 and 287, 150 and 148; SU(2) 16^3 and smaller alike).  1 x 1 x 8: 265, 208, 118; 439, 329, 175; 365, 310, 154.
+// (a direction that is not cut wraps around inside its box) the one with the smallest plane of that walk is taken, along
+// z where two are alike: the three planes a site's neighbours span are then likeliest to stay in the XCD's L2.
+// Larger cubes are cut 2 x 4 x 1 by that; 2 x 2 x 2 has the same surface and planes twice as large (us per Clenshaw
+// step, 2 x 2 x 2 and 2 x 4 x 1: SU(3) 24^3, 64 modes FP64 234 and 231, 48-bit 193 and 187, FP32 115 and 111; SU(2)
+// 32^3, 64 modes 374 and 366, 302 and 293, 169 and 162; SU(3) 32^3, 32 modes 356 and 325, 307 and 287, 150 and 148;
+// SU(3) 12^3, 32 modes 26.6 and 25.1 in FP64; SU(2) 12^3 alike; SU(2) 16^3, 64 modes in FP64 the other way, 51.9
+// and 53.3).  1 x 1 x 8: 265, 208, 118; 439, 329, 175; 365, 310, 154.
+// Boxes thinner than three sites, all of whose sites are a face's, come last once a launch has two workgroups per CU
+// and more: lattices of extent 8 cut into four lost by them (SU(2) in FP64, 96 degrees of the sign: 8^3 with 256
+// modes 2 x 4 x 1 3139 us, 2 x 2 x 2 2939, 384 modes 4519 and 4168, 8 x 16 x 8 with 256 modes 5480 and 5158; 40 Wilson steps of
+// 8^3 with 256 modes 1370 and 1325).  With fewer workgroups the thin planes are the better ones (40 Wilson steps of 8^3
+// with 48 modes 728 and 780, 128 modes 793 and 847).
 // Whole boxes (sub = 1) are computed by the kernel from `box`; slabs have a table.
-bool xcd_boxes(int n0, int n1, int n2, ovl::XcdBoxes *out)
+bool xcd_boxes(int n0, int n1, int n2, long lanes, ovl::XcdBoxes *out)
 {
     bool found = false;
-    std::array<long, 4> best{};
+    std::array<long, 5> best{};
     for (int lx = 0; lx <= 3; ++lx)
         for (int ly = 0; lx + ly <= 3; ++ly) {
             const int px = 1 << lx, py = 1 << ly, pz = 8 >> (lx + ly);
@@ -410,7 +416,8 @@ bool xcd_boxes(int n0, int n1, int n2, ovl::XcdBoxes *out)
             const long bx = n0 / px, by = n1 / py, bz = n2 / pz;
             const long cut = (px > 1 ? by * bz : 0) + (py > 1 ? bz * bx : 0) + (pz > 1 ? bx * by : 0);
             const bool y_mid = by <= bz;
-            const std::array<long, 4> cost{cut, bx * std::min(by, bz), y_mid ? 0 : 1, px};
+            const bool thin = lanes >= 512l * ovl::STENCIL_TPB && ((px > 1 && bx < 3) || (py > 1 && by < 3) || (pz > 1 && bz < 3));
+            const std::array<long, 5> cost{cut, thin, bx * std::min(by, bz), y_mid ? 0 : 1, px};
             if (found && cost >= best) continue;
             found = true;
             best = cost;
@@ -420,11 +427,9 @@ bool xcd_boxes(int n0, int n1, int n2, ovl::XcdBoxes *out)
     return found;
 }
 
-std::vector<int> xcd_site_order(int n0, int n1, int n2, int sub)
+std::vector<int> xcd_site_order(int n0, int n1, int n2, const ovl::XcdBoxes &q, int sub)
 {
     std::vector<int> order;
-    ovl::XcdBoxes q;
-    if (!xcd_boxes(n0, n1, n2, &q)) return order;
     const int bx = (int)q.dv_x.d, slow = q.y_mid ? q.bz : q.by, mid = q.y_mid ? q.by : q.bz;
     sub = std::max(1, std::min(sub, mid));
     order.reserve((size_t)n0 * n1 * n2);
@@ -497,7 +502,7 @@ int set_traversal(ovl_ctx *c, int prec, int trav, int slabs)
     c->slabs[prec] = slabs;
     c->order_set[prec] = true;
     std::vector<int> ord;
-    if (trav == ovl::TRAV_BOXES && slabs > 1) ord = xcd_site_order(c->g.n0, c->g.n1, c->g.n2, slabs);
+    if (trav == ovl::TRAV_BOXES && slabs > 1) ord = xcd_site_order(c->g.n0, c->g.n1, c->g.n2, c->box, slabs);
     else if (trav == ovl::TRAV_MODES && slabs > 1) ord = slab_site_order(c->g.n0, c->g.n1, c->g.n2, slabs);
     if (ord.empty()) return OVL_OK;
     RETCHK(dalloc(c, (void **)&c->order[prec], sizeof(int) * ord.size()));
@@ -1447,7 +1452,7 @@ static int ctx_init(ovl_ctx *c)
     RETCHK(dalloc(c, (void **)&c->partial, sizeof(double) * c->partial_len));
     RETCHK(dalloc(c, (void **)&c->dout, sizeof(double) * (16 + 2 * (size_t)maxblk * mb)));
     if (!c->ensemble && (c->prm.traversal == 0 || c->prm.traversal == 2))
-        c->boxes_ok = xcd_boxes(c->g.n0, c->g.n1, c->g.n2, &c->box);
+        c->boxes_ok = xcd_boxes(c->g.n0, c->g.n1, c->g.n2, (long)c->g.V * c->g.nblk * mb, &c->box);
     if (!c->ensemble) {
         // traversal 0 (automatic): mode split where the mode blocks divide over the XCDs, else
         // boxes; ovl_autotune may change it
