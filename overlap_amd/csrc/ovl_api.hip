@@ -111,10 +111,7 @@ struct ovl_ctx {
     bool order_set[NUM_PREC] = {false, false, false, false};
     int trav[NUM_PREC] = {ovl::TRAV_LEX, ovl::TRAV_LEX, ovl::TRAV_LEX, ovl::TRAV_LEX};  // lane traversal
     int slabs[NUM_PREC] = {1, 1, 1, 1};         // y slabs (TRAV_MODES) or sub-slabs per box (TRAV_BOXES)
-    // streaming output stores: on from the start in FP64, where they leave the L2 to the neighbours (24^3
-    // SU(3), 64 modes, one Clenshaw step 272 -> 236 us; 16^3 SU(2) 53 -> 51); FP32 loses 1% with them
-    // and the other two do not care
-    int nt_out[NUM_PREC] = {1, 0, 0, 0};
+    int nt_out[NUM_PREC] = {0, 0, 0, 0};        // streaming output stores (streams_fp64)
     int wpe[NUM_PREC] = {1, 1, 1, 1};           // occupancy variant
     bool tuned = false;                         // ovl_set_tuning or ovl_autotune has run
     double step_xmax = 0.0;  // bound of the mode norms during ovl_fermion_update (FP16 scales)
@@ -1412,6 +1409,18 @@ int ovl_device_name(char *buf, int len)
     return OVL_OK;
 }
 
+// Streaming output stores of an untuned context: in FP64 they leave the caches to the neighbours (24^3 SU(3), 64 modes,
+// one Clenshaw step 272 -> 236 us; 24^3 SU(2), 128 modes 330 -> 294; an ensemble of SU(2) 8^3, 12^3 and 16^3, 64 modes 93
+// -> 89).  SU(2) vectors of 64-mode blocks between about 20 and 140 MB are better off where the next launch
+// finds them again (plain and streaming, 96 degrees: 16^3 with 64 modes, 34 MB, 5117 and 5169 us, 128 modes
+// 9094 and 9368, 256 modes, 134 MB, 17138 and 17623; outside 12 x 12 x 8 with 128 modes, 19 MB, 3641 and 3556, 28^3 with
+// 64 modes, 180 MB, 25803 and 22769).  FP32 loses 1% with them and the other two precisions do not care.
+static bool streams_fp64(const ovl_ctx *c)
+{
+    const bool kept = !c->ensemble && c->g.nc == 2 && c->g.mb == 64 && c->field64_bytes >= 20000000 && c->field64_bytes <= 140000000;
+    return !kept;
+}
+
 // Allocations and device tables common to ordinary and ensemble contexts; c->g, c->sys and
 // c->link_sites are filled in.  On failure the caller destroys c.
 static int ctx_init(ovl_ctx *c)
@@ -1451,6 +1460,7 @@ static int ctx_init(ovl_ctx *c)
     c->partial_len = plen;
     RETCHK(dalloc(c, (void **)&c->partial, sizeof(double) * c->partial_len));
     RETCHK(dalloc(c, (void **)&c->dout, sizeof(double) * (16 + 2 * (size_t)maxblk * mb)));
+    c->nt_out[P64] = streams_fp64(c);
     if (!c->ensemble && (c->prm.traversal == 0 || c->prm.traversal == 2))
         c->boxes_ok = xcd_boxes(c->g.n0, c->g.n1, c->g.n2, (long)c->g.V * c->g.nblk * mb, &c->box);
     if (!c->ensemble) {
