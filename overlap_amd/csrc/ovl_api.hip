@@ -212,6 +212,7 @@ int dalloc(ovl_ctx *c, void **p, size_t bytes)
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
         *p = nullptr;
+        (void)hipGetLastError();  // reported here: not again by the next launch
         return fail(c, OVL_E_NOMEM, "hipMalloc of " + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));
     }
     return OVL_OK;
@@ -2355,9 +2356,19 @@ static int wilson_half(ovl_ctx *c, const ovl_step_opts *o, int src, int tgt, con
 // pays there, most on small lattices, where a launch leaves most of the chip idle (us per step with moving
 // links, apart and shared: SU(2) 8^3, 16 modes FP64 24.1 and 16.8; SU(3) 24^3, 64 modes FP64 236 and 219;
 // SU(3) 32^3, 256 modes FP32 1081 and 1057); an overlap step has hundreds of launches per gauge half step.
+// Moving links alone need the second set of stencil links; without room for it the half steps stay apart.
 static bool shares_launches(const ovl_ctx *c, const ovl_step_opts *o)
 {
-    return o->kind == OVL_WILSON && o->gauge != OVL_GAUGE_FROZEN && !c->ensemble;
+    if (o->kind != OVL_WILSON || o->gauge == OVL_GAUGE_FROZEN || c->ensemble) return false;
+    return o->gauge == OVL_GAUGE_FULL || (c->ul64_next && c->ul32_next);
+}
+static void make_next_links(ovl_ctx *c, const ovl_step_opts *o)
+{
+    if (o->kind != OVL_WILSON || o->gauge != OVL_GAUGE_LINKS || c->ensemble) return;
+    const size_t entries = 3 * (size_t)c->link_sites * c->g.nc * c->g.nc;
+    if (dalloc(c, (void **)&c->ul64_next, 16 * entries) == OVL_OK && dalloc(c, (void **)&c->ul32_next, 8 * entries) == OVL_OK)
+        return;
+    for (void **p : {(void **)&c->ul64_next, (void **)&c->ul32_next}) dfree(*p);
 }
 
 // a Wilson half step with its gauge half step in shared launches.  Links alone: the stencil reads the present
@@ -2525,11 +2536,7 @@ static int update_impl(ovl_ctx *c, const ovl_step_opts *o, int nsteps, bool obse
     if (w32)
         for (int f = 0; f < 2; ++f)
             if (!c->f32[f]) RETCHK(dalloc(c, &c->f32[f], c->field32_bytes));
-    if (shares_launches(c, o) && o->gauge == OVL_GAUGE_LINKS) {
-        const size_t entries = 3 * (size_t)c->link_sites * c->g.nc * c->g.nc;
-        RETCHK(dalloc(c, (void **)&c->ul64_next, 16 * entries));
-        RETCHK(dalloc(c, (void **)&c->ul32_next, 8 * entries));
-    }
+    make_next_links(c, o);
     begin_timing(c);
     if (observe_last && nsteps > 0) {
         RETCHK(update_impl(c, req, nsteps - 1, false));
