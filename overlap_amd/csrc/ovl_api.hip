@@ -1802,13 +1802,12 @@ static bool all_finite(const double *p, size_t n)
 static int put_doubles(ovl_ctx *c, double *dst, const double *src, size_t n, const char *what)
 {
     bool ok = true;
-    if (n <= HOST_SCAN) {
+    if (n <= HOST_SCAN || stage(c, n * sizeof(double)) != OVL_OK) {  // without room for the staging too
         if (!all_finite(src, n)) return fail(c, OVL_E_ARG, std::string("non-finite ") + what);
         HIPCHK(c, hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyHostToDevice, c->st));
         HIPCHK(c, hipStreamSynchronize(c->st));
         return OVL_OK;
     }
-    RETCHK(stage(c, n * sizeof(double)));
     HIPCHK(c, hipMemcpyAsync(c->staging, src, n * sizeof(double), hipMemcpyHostToDevice, c->st));
     RETCHK(device_finite(c, c->staging, nullptr, (long)n, &ok));
     if (!ok) return fail(c, OVL_E_ARG, std::string("non-finite ") + what);

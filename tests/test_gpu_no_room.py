@@ -54,3 +54,27 @@ for refused in (0, {refuse} * 3 * 210 * 9):
 for a, b in zip(*outs):
     assert np.array_equal(a, b)
 """, tmp_path)
+
+
+def test_link_upload_without_a_staging_buffer(gpu, tmp_path):
+    print("[case] upload of 2.9 MB of links, staging refused", flush=True)
+    run("""
+n = (18, 20, 19)
+g = cf.rng(62)
+links = cf.su3_links(n, 0.4, g)
+e = cf.efield(n, 3, 0.2, g)
+bad = links.copy()
+bad[-2] = np.nan
+with ovl.Context(3, n, 1) as ctx:
+    shim.shim_refuse(0, links.nbytes)
+    ctx.set_links(links)
+    assert shim.shim_refusals() >= 1
+    ctx.set_efield(e)  # small enough for the host's scan: no staging
+    try:
+        ctx.set_links(bad)
+        raise SystemExit("non-finite links were taken")
+    except ovl.OvlError as err:
+        assert err.code == ovl.E_ARG
+    assert np.array_equal(ctx.get_links(), links) and np.array_equal(ctx.get_efield(), e)
+    ctx.apply_wilson(ovl.PSI, ovl.SCRATCH)
+""", tmp_path)
