@@ -1204,9 +1204,10 @@ ovl::CgShifts zolotarev_shifts(double lmin, double lmax)
 // iteration where an iteration moves more than CG_BATCH_BYTES (about 0.2 ms, ten times the 20 us that
 // the host's look costs) and eight of them below.
 constexpr double CG_BATCH_BYTES = 1e9;
-int mscg(ovl_ctx *c, const Geom &g, const void *in, void *chi, const ovl::CgShifts &sh, int *nonconv)
+int mscg(ovl_ctx *c, const void *in, void *chi, const ovl::CgShifts &sh, int *nonconv)
 {
     constexpr int no = ovl::CG_SHIFTS;
+    const Geom &g = c->g;  // the buffers are allocated once, for all modes of the context
     const size_t fb = (size_t)g.nblk * c->blk64_elems * 16;
     const int nm = g.nblk * g.mb, chunks = ovl::mode_dot_chunks();
     RETCHK(dalloc(c, &c->ms_ps, fb * no));
@@ -1341,18 +1342,17 @@ int check_interval(ovl_ctx *c, double lmin, double lmax)
 int ritz_bounds(ovl_ctx *c, double *lmin, double *lmax);
 
 // -i h_ov in -> out (or out += dt (-i h_ov in)) with the Zolotarev sign, all modes of g
-int zolo_overlap(ovl_ctx *c, const Geom &g, const void *in, void *out, double lmin, double lmax, int axpy, double dt)
+int zolo_overlap(ovl_ctx *c, const void *in, void *out, double lmin, double lmax, int axpy, double dt)
 {
     if (lmin == 0.0 && lmax == 0.0) RETCHK(ritz_bounds(c, &lmin, &lmax));
     RETCHK(check_interval(c, lmin, lmax));
     RETCHK(ensure_stencil(c));
-    RETCHK(dalloc(c, &c->ms_chi, (size_t)g.nblk * c->blk64_elems * 16));
+    RETCHK(dalloc(c, &c->ms_chi, c->field64_bytes));
     int nc = 0;
-    RETCHK(mscg(c, g, in, c->ms_chi, zolotarev_shifts(lmin, lmax), &nc));
+    RETCHK(mscg(c, in, c->ms_chi, zolotarev_shifts(lmin, lmax), &nc));
     // psi = -i h_W chi, combined as OverlapU.cpp:188-201
     const double M = c->prm.m_dw, m = c->prm.m_fermion, s = axpy ? dt : 1.0;
     HopArgs a = hop_args(c, P64);
-    a.nblk = g.nblk;
     a.in = c->ms_chi;
     a.out = out;
     a.sh_i = -s * M * (1.0 - 0.5 * m);
@@ -1363,7 +1363,7 @@ int zolo_overlap(ovl_ctx *c, const Geom &g, const void *in, void *out, double lm
         a.tgt = out;
         a.st_r = 1.0;
     }
-    RETCHK(hop(c, g, P64, P64, a));
+    RETCHK(hop(c, c->g, P64, P64, a));
     return cg_result(c, nc);
 }
 
@@ -2044,7 +2044,7 @@ int ovl_apply_overlap(ovl_ctx *c, int in, int out, const ovl_sign_opts *o)
     if (in == out) return fail(c, OVL_E_ARG, "in and out must be different fields");
     begin_timing(c);
     if (o->method == OVL_SIGN_ZOLOTAREV) {
-        int r = zolo_overlap(c, c->g, c->field[in], c->field[out], o->lmin, o->lmax, 0, 0.0);
+        int r = zolo_overlap(c, c->field[in], c->field[out], o->lmin, o->lmax, 0, 0.0);
         end_timing(c);
         return r;
     }
@@ -2394,7 +2394,7 @@ static int fermion_half(ovl_ctx *c, const ovl_step_opts *o, int src, int tgt, vo
 {
     if (o->kind == OVL_WILSON) return wilson_half(c, o, src, tgt, nullptr);
     if (o->sign.method == OVL_SIGN_ZOLOTAREV)
-        return zolo_overlap(c, c->g, c->field[src], c->field[tgt], o->sign.lmin, o->sign.lmax, 1, o->dt);
+        return zolo_overlap(c, c->field[src], c->field[tgt], o->sign.lmin, o->sign.lmax, 1, o->dt);
     return sign_driver(c, &o->sign, c->field[src], c->field[tgt], FIN_OVERLAP_AXPY, o->dt, c->step_xmax, hpsi);
 }
 
@@ -2891,7 +2891,7 @@ int ovl_currents(ovl_ctx *c, int field, const ovl_sign_opts *o, int first_mode, 
     if (field == OVL_SCRATCH) return fail(c, OVL_E_ARG, "currents use the scratch field for -i h_ov psi");
     RETCHK(single_lattice(c, "ovl_currents"));
     if (o->method == OVL_SIGN_ZOLOTAREV)
-        RETCHK(zolo_overlap(c, c->g, c->field[field], c->field[OVL_SCRATCH], o->lmin, o->lmax, 0, 0.0));
+        RETCHK(zolo_overlap(c, c->field[field], c->field[OVL_SCRATCH], o->lmin, o->lmax, 0, 0.0));
     else
     {
         double xmax;
@@ -3199,7 +3199,7 @@ int ovl_qed_eigenbasis(ovl_ctx *c, const ovl_sign_opts *o, int nb, double q, dou
         HIPCHK(c, hipMemsetAsync(c->field[OVL_SCRATCH], 0, c->field64_bytes, c->st));
         HIPCHK(c, ovl::launch_eig_sources(g, c->field[OVL_SCRATCH], k0, cnt, Dz, c->st));
         if (o->method == OVL_SIGN_ZOLOTAREV)
-            RETCHK(zolo_overlap(c, g, c->field[OVL_SCRATCH], c->field[OVL_PSIMID], zlmin, zlmax, 0, 0.0));
+            RETCHK(zolo_overlap(c, c->field[OVL_SCRATCH], c->field[OVL_PSIMID], zlmin, zlmax, 0, 0.0));
         else
             RETCHK(sign_driver(c, o, c->field[OVL_SCRATCH], c->field[OVL_PSIMID], FIN_OVERLAP, 0.0, 1.0));
         if (nsb > 0) {
