@@ -334,10 +334,9 @@ double hop_alg_bytes(const ovl_ctx *c, const HopArgs &a, int pin, int pout)
     return b;
 }
 
-// gauge: a gauge half step to run in the same launch
-int hop(ovl_ctx *c, const Geom &g, int pin, int pout, const HopArgs &a, const ovl::GaugeHalf *gauge = nullptr)
+// with profiling on, times what `launch` queues as stencil variant `var`
+template <class F> int timed_hop(ovl_ctx *c, int var, F launch)
 {
-    const int var = (pin == P64) ? 0 : (pin == P16 ? 3 : (pin == P48 ? 4 : (pout == P32 ? 1 : 2)));
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (c->profiling && !c->capturing) {
         e0 = next_event(c);
@@ -350,14 +349,27 @@ int hop(ovl_ctx *c, const Geom &g, int pin, int pout, const HopArgs &a, const ov
             c->evused--;  // an unpaired event stays unused
         }
     }
-    if (gauge) HIPCHK(c, ovl::launch_hop_gauge(g, pin, a, *gauge, c->st));
-    else HIPCHK(c, ovl::launch_hop(g, pin, pout, a, c->wpe[pin], c->st));
+    HIPCHK(c, launch());
     if (e1) HIPCHK(c, hipEventRecord(e1, c->st));
-    const double b = hop_alg_bytes(c, a, pin, pout);
-    c->hop_launches++;
-    c->hop_bytes += b;
-    c->var_launches[var]++;
-    c->var_bytes[var] += b;
+    return OVL_OK;
+}
+
+void count_hops(ovl_ctx *c, int var, long long launches, double bytes)
+{
+    c->hop_launches += launches;
+    c->hop_bytes += bytes;
+    c->var_launches[var] += launches;
+    c->var_bytes[var] += bytes;
+}
+
+// gauge: a gauge half step to run in the same launch
+int hop(ovl_ctx *c, const Geom &g, int pin, int pout, const HopArgs &a, const ovl::GaugeHalf *gauge = nullptr)
+{
+    const int var = (pin == P64) ? 0 : (pin == P16 ? 3 : (pin == P48 ? 4 : (pout == P32 ? 1 : 2)));
+    RETCHK(timed_hop(c, var, [&] {
+        return gauge ? ovl::launch_hop_gauge(g, pin, a, *gauge, c->st) : ovl::launch_hop(g, pin, pout, a, c->wpe[pin], c->st);
+    }));
+    count_hops(c, var, 1, hop_alg_bytes(c, a, pin, pout));
     return OVL_OK;
 }
 
@@ -2205,32 +2217,53 @@ static int ritz_solve(ovl_ctx *c, int solves, const double *sign, double delitr,
     HIPCHK(c, ovl::launch_ritz_start(c->g, k, c->st));
     // An iteration is five short launches; once all solves are done they return at once.  The pair of bounds
     // takes hundreds of iterations, so a batch of them is a graph (a third of the gaps of eager launches);
-    // its length is even and divides the 100 iterations between restarts, which stay outside.
+    // its length is even and divides the 100 iterations between restarts, which stay outside.  With profiling on
+    // the launches stay eager and the stencil's are timed.
     constexpr int batch = 20;
-    const bool graph = solves == 2 && nrestart % batch == 0;
+    const bool graph = solves == 2 && nrestart % batch == 0 && !c->profiling;
     auto iterations = [&](int n, int first) -> hipError_t {
         for (int i = 0; i < n; ++i) {
-            const hipError_t e = ovl::launch_ritz_iteration(c->g, k, first + i, c->st);
+            hipError_t e = ovl::launch_ritz_hops(c->g, k, first + i, false, c->st);
+            if (e == hipSuccess) e = ovl::launch_ritz_rest(c->g, k, first + i, false, c->st);
             if (e != hipSuccess) return e;
         }
         return hipSuccess;
     };
+    auto eager = [&](int iter, bool restart) -> int {
+        RETCHK(timed_hop(c, 0, [&] { return ovl::launch_ritz_hops(c->g, k, iter, restart, c->st); }));
+        HIPCHK(c, ovl::launch_ritz_rest(c->g, k, iter, restart, c->st));
+        return OVL_OK;
+    };
     if (graph && !c->ritz_exec) RETCHK(capture_launches(c, &c->ritz_exec, [&] { return iterations(batch, 0); }));
+    long long launches = 0;
     for (int it = 0;;) {
-        if (it % nrestart == 0) HIPCHK(c, ovl::launch_ritz_restart(c->g, k, it, c->st));
+        if (it % nrestart == 0) {
+            RETCHK(eager(it, true));
+            launches += 2;
+        }
         const int n = graph ? batch : std::min(batch, nrestart - it % nrestart);
         if (graph) HIPCHK(c, hipGraphLaunch(c->ritz_exec, c->st));
-        else HIPCHK(c, iterations(n, it));
+        else
+            for (int i = 0; i < n; ++i) RETCHK(eager(it + i, false));
         it += n;
-        c->hop_launches += 2 * n;
+        launches += 2 * n;
         HIPCHK(c, hipMemcpyAsync(h.data(), c->s1_state, sizeof(ovl::RitzState) * h.size(), hipMemcpyDeviceToHost, c->st));
         HIPCHK(c, hipStreamSynchronize(c->st));
         bool all = true;
         for (int q = 0; q < solves; ++q) all = all && h[2 * q + (it & 1)].done;
-        if (all) {
-            for (int q = 0; q < solves; ++q) eig[q] = h[2 * q + (it & 1)].xy_r;
-            return OVL_OK;
+        if (!all) continue;
+        // the bytes of the iterations until each solve was done: two launches of 2 + 4 vectors, 2 + 3 at a
+        // restart, and the links once for the solves that share a launch
+        double vectors = 0, longest = 0;
+        for (int q = 0; q < solves; ++q) {
+            const ovl::RitzState &r = h[2 * q + (it & 1)];
+            const double restarts = (r.iters + nrestart - 1) / nrestart;
+            vectors += 6.0 * r.iters + 5.0 * restarts;
+            longest = std::max(longest, r.iters + restarts);
+            eig[q] = r.xy_r;
         }
+        count_hops(c, 0, launches, vectors * vec1_bytes(c) + 2.0 * longest * 48.0 * c->g.V * c->g.nc * c->g.nc);
+        return OVL_OK;
     }
 }
 

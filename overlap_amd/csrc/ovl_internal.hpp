@@ -221,7 +221,8 @@ size_t single_partial_len(const Geom &g);  // doubles of `part` below
 // Ritz: up to RITZ_SOLVES independent solves (signs sign[0..solves)) advance in the same launches.  `vec`:
 // RITZ_VECS vectors per solve, the first one the start vector; `state`: 2 RitzState per solve, zeroed;
 // iteration `iter` counts from 0, with a restart before the first and after every nrestart iterations (the
-// launches depend on iter by its parity only).  The result of iteration i is state[2 solve + (i + 1) % 2].
+// launches depend on iter by its parity only).  The result of iteration i is state[2 solve + (i + 1) % 2].  Either is its
+// two stencil launches (hops) and then the rest.
 constexpr int RITZ_VECS = 6, RITZ_SOLVES = 2, RITZ_PARTS = 5;
 struct RitzState {
     double xy_r, xy_i, xyn_r, xyn_i, gnormim;
@@ -235,8 +236,8 @@ struct RitzCall {
     int solves, nitlz;
 };
 hipError_t launch_ritz_start(const Geom &g, const RitzCall &c, hipStream_t st);
-hipError_t launch_ritz_restart(const Geom &g, const RitzCall &c, int iter, hipStream_t st);
-hipError_t launch_ritz_iteration(const Geom &g, const RitzCall &c, int iter, hipStream_t st);
+hipError_t launch_ritz_hops(const Geom &g, const RitzCall &c, int iter, bool restart, hipStream_t st);
+hipError_t launch_ritz_rest(const Geom &g, const RitzCall &c, int iter, bool restart, hipStream_t st);
 
 // multi-shift CG of one vector: `work` holds CG_SHIFTS + 4 vectors, `state` 2 CgMode, `shifts` a CgShifts (all
 // device); the launches depend on iter by its parity only; the state after iteration `iter` (from 0) is

@@ -908,39 +908,34 @@ hipError_t launch_ritz_start(const Geom &g, const RitzCall &c, hipStream_t st)
     return hipGetLastError();
 }
 
-template <int NC> static void ritz_restart_nc(const RitzArgs &a, int solves, hipStream_t st)
+template <int NC, bool RESTART> static void ritz_hops_nc(const RitzArgs &a, int solves, hipStream_t st)
 {
-    const dim3 hp(a.nb_hop, solves), pt(a.nb_pt, solves);
-    k_ritz_hop<NC, true><<<hp, TPB1, 0, st>>>(a);
-    k_ritz_hop2<NC, true><<<hp, TPB1, 0, st>>>(a);
-    k_ritz_restart<<<pt, TPB1, 0, st>>>(a);
+    const dim3 hp(a.nb_hop, solves);
+    k_ritz_hop<NC, RESTART><<<hp, TPB1, 0, st>>>(a);
+    k_ritz_hop2<NC, RESTART><<<hp, TPB1, 0, st>>>(a);
 }
 
-template <int NC> static void ritz_iteration_nc(const RitzArgs &a, int solves, hipStream_t st)
-{
-    const dim3 hp(a.nb_hop, solves), pt(a.nb_pt, solves);
-    k_ritz_hop<NC, false><<<hp, TPB1, 0, st>>>(a);
-    k_ritz_hop2<NC, false><<<hp, TPB1, 0, st>>>(a);
-    k_ritz_rotate<<<pt, TPB1, 0, st>>>(a);
-    k_ritz_gradient<<<pt, TPB1, 0, st>>>(a);
-    k_ritz_direction<<<pt, TPB1, 0, st>>>(a);
-}
-
-hipError_t launch_ritz_restart(const Geom &g, const RitzCall &c, int iter, hipStream_t st)
+hipError_t launch_ritz_hops(const Geom &g, const RitzCall &c, int iter, bool restart, hipStream_t st)
 {
     RitzArgs a = ritz_args(g, c);
     a.par = iter & 1;
-    if (g.nc == 2) ritz_restart_nc<2>(a, c.solves, st);
-    else ritz_restart_nc<3>(a, c.solves, st);
+    if (g.nc == 2) restart ? ritz_hops_nc<2, true>(a, c.solves, st) : ritz_hops_nc<2, false>(a, c.solves, st);
+    else restart ? ritz_hops_nc<3, true>(a, c.solves, st) : ritz_hops_nc<3, false>(a, c.solves, st);
     return hipGetLastError();
 }
 
-hipError_t launch_ritz_iteration(const Geom &g, const RitzCall &c, int iter, hipStream_t st)
+hipError_t launch_ritz_rest(const Geom &g, const RitzCall &c, int iter, bool restart, hipStream_t st)
 {
     RitzArgs a = ritz_args(g, c);
     a.par = iter & 1;
-    if (g.nc == 2) ritz_iteration_nc<2>(a, c.solves, st);
-    else ritz_iteration_nc<3>(a, c.solves, st);
+    const dim3 pt(a.nb_pt, c.solves);
+    if (restart) {
+        k_ritz_restart<<<pt, TPB1, 0, st>>>(a);
+    } else {
+        k_ritz_rotate<<<pt, TPB1, 0, st>>>(a);
+        k_ritz_gradient<<<pt, TPB1, 0, st>>>(a);
+        k_ritz_direction<<<pt, TPB1, 0, st>>>(a);
+    }
     return hipGetLastError();
 }
 
