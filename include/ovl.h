@@ -304,7 +304,9 @@ typedef struct {
     double total_ms;          /* event-timed wall time of the call on the stream */
     double hop_ms;            /* summed event time of the stencil kernels */
     long long hop_launches;   /* number of stencil kernel launches */
-    double hop_bytes;         /* algorithmic bytes of those launches */
+    double hop_bytes;         /* algorithmic bytes of those launches; a Wilson step with moving links shares
+                                 its stencil launches with gauge half steps, whose bytes (and time)
+                                 are then counted with them */
     int fp64_steps, fp32_steps, fp16_steps, fp48_steps;
     /* per stencil-kernel variant: [0] FP64 in/out, [1] FP32 in/out, [2] FP32 in / FP64 out,
      * [3] FP16 storage in/out, [4] 48-bit storage in/out */
@@ -334,7 +336,9 @@ int ovl_autotune(ovl_ctx *ctx, char *report, int len);
  * kernel, whose `slabs` is the number of tiles a workgroup claims at a time), y slabs of the
  * traversal, streaming output stores (0/1), occupancy
  * variant (minimum waves per SIMD, 1-4; 5 = one workgroup per CU through an LDS reservation, where
- * the device allows 96 KiB per workgroup).  Setting one replays a saved tuning without the sweep. */
+ * the device allows 96 KiB per workgroup; the launches that a Wilson step with moving links shares with its
+ * gauge half steps have one occupancy and disregard it).  Setting one replays a saved tuning without the
+ * sweep. */
 typedef struct {
     int traversal;
     int slabs;

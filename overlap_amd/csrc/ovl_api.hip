@@ -334,6 +334,15 @@ double hop_alg_bytes(const ovl_ctx *c, const HopArgs &a, int pin, int pout)
     return b;
 }
 
+// algorithmic bytes of a gauge half step: links read and written, E read, stencil links written; or links read, E
+// read and written
+double gauge_alg_bytes(const ovl_ctx *c, const ovl::GaugeHalf &h)
+{
+    const double links = 3.0 * h.V, u = 8.0 * link_reals(c), e = 8.0 * n_adj(c), nn = (double)c->g.nc * c->g.nc;
+    if (h.what == ovl::GAUGE_EFIELD_HALF) return links * (u + 2.0 * e);
+    return links * (2.0 * u + e + (h.ul64 ? 24.0 * nn + (h.phase ? 16.0 : 0.0) : 0.0));
+}
+
 // with profiling on, times what `launch` queues as stencil variant `var`
 template <class F> int timed_hop(ovl_ctx *c, int var, F launch)
 {
@@ -369,7 +378,7 @@ int hop(ovl_ctx *c, const Geom &g, int pin, int pout, const HopArgs &a, const ov
     RETCHK(timed_hop(c, var, [&] {
         return gauge ? ovl::launch_hop_gauge(g, pin, a, *gauge, c->st) : ovl::launch_hop(g, pin, pout, a, c->wpe[pin], c->st);
     }));
-    count_hops(c, var, 1, hop_alg_bytes(c, a, pin, pout));
+    count_hops(c, var, 1, hop_alg_bytes(c, a, pin, pout) + (gauge ? gauge_alg_bytes(c, *gauge) : 0.0));
     return OVL_OK;
 }
 
@@ -2384,10 +2393,13 @@ static int wilson_half(ovl_ctx *c, const ovl_step_opts *o, int src, int tgt, con
     return hop(c, c->g, pr, pr, a, gauge);
 }
 
-// Whether a step's stencil and gauge half steps share launches: the Wilson steps of one lattice.  It always
-// pays there, most on small lattices, where a launch leaves most of the chip idle (us per step with moving
-// links, apart and shared: SU(2) 8^3, 16 modes FP64 24.1 and 16.8; SU(3) 24^3, 64 modes FP64 236 and 219;
-// SU(3) 32^3, 256 modes FP32 1081 and 1057); an overlap step has hundreds of launches per gauge half step.
+// Whether a step's stencil and gauge half steps share launches: the Wilson steps of one lattice.  It pays most on small
+// lattices, where a launch leaves most of the chip idle, and costs nothing to speak of on large ones; an overlap
+// step has hundreds of launches per gauge half step.  The shared launch has one occupancy, whatever the context's
+// waves_per_eu, and that is the better one too.  us per step with moving links, apart with the best and the worst
+// of the five occupancy variants, and shared: SU(2) 8^3, 16 modes 22.5, 45.1, 17.4; 16^3, 32 modes 37.6, 85.9, 33.9;
+// 32^3, 64 modes 345.6, 587.7, 348.5; SU(3) 8^3, 16 modes 32.5, 77.7, 23.5; 16^3, 32 modes 63.6, 159.8, 55.0; 24^3, 64 modes
+// 233.0, 592.5, 221.0, in FP32 130.0, 161.2, 116.7; 15 x 12 x 10, 24 modes FP32 33.9, 54.9, 25.4.
 // Moving links alone need the second set of stencil links; without room for it the half steps stay apart.
 static bool shares_launches(const ovl_ctx *c, const ovl_step_opts *o)
 {

@@ -45,3 +45,36 @@ def test_ritz_bounds_are_counted(gpu, nc, n, nm):
         # an iteration of a solve moves six vectors in its two launches, a restart five
         own_t = ts["own", False]
         assert own_t.hop_launches >= 40 and own_t.hop_bytes >= 40 * 2 * V * 4 * nc * 16
+
+
+@pytest.mark.parametrize("nc,flux", [(2, 0), (2, 1), (3, 0), (3, 2)])
+@pytest.mark.parametrize("prec", [ovl.PREC_FP64, ovl.PREC_FP32])
+def test_shared_launches_count_both(gpu, nc, flux, prec):
+    print(f"[case] timing of shared launches nc={nc} flux={flux} prec={prec}", flush=True)
+    n, nm, steps = (4, 5, 6), 3, 2
+    V = int(np.prod(n))
+    links_b, e_b, nn = 8 * (4 if nc == 2 else 18), 8 * (nc * nc - 1), nc * nc
+    g = cf.rng(970 + nc)
+    with ovl.Context(nc, n, nm, m_fermion=0.1) as ctx:
+        ctx.set_links(cf.su2_links(n, 0.3, g) if nc == 2 else cf.su3_links(n, 0.3, g))
+        ctx.set_efield(cf.efield(n, nc, 0.2, g))
+        ctx.set_u1_flux(flux, 1.0)
+        t = {}
+        for gauge in (ovl.GAUGE_FROZEN, ovl.GAUGE_LINKS, ovl.GAUGE_FULL):
+            for graph in (0, 1):
+                ctx.fermion_update(ovl.StepOpts(kind=ovl.WILSON, dt=0.01, gauge=gauge, sign=ovl.sign_opts(precision=prec),
+                                                use_graph=graph), steps)
+                t[gauge, graph] = ctx.timing()
+                consistent(t[gauge, graph])
+        for graph in (0, 1):
+            frozen = t[ovl.GAUGE_FROZEN, graph]
+            assert frozen.hop_launches == 2 * steps
+            # links: read, written, E read, stencil links (24 bytes an entry) written, phases read
+            half = 3 * V * (2 * links_b + e_b + 24 * nn + (16 if flux else 0))
+            moved = t[ovl.GAUGE_LINKS, graph]
+            assert moved.hop_launches == 2 * steps
+            assert abs(moved.hop_bytes - frozen.hop_bytes - 2 * steps * half) <= 1e-9 * moved.hop_bytes
+            # with E moving its half step shares the launch: links read, E read and written
+            full = t[ovl.GAUGE_FULL, graph]
+            assert full.hop_launches == 2 * steps
+            assert abs(full.hop_bytes - frozen.hop_bytes - 2 * steps * 3 * V * (links_b + 2 * e_b)) <= 1e-9 * full.hop_bytes
