@@ -1,6 +1,7 @@
 // Host side of the C ABI (include/ovl.h): device state, the sign-function drivers and the
-// leapfrog.  Scalar recurrences (Clenshaw coefficients, multi-shift CG and Ritz scalars) run on
-// the host in FP64; every vector operation runs in the gfx950 kernels of ovl_kernels.hip.
+// leapfrog.  Clenshaw coefficients are made on the host in FP64; the scalars of the multi-shift CG and of the
+// Ritz solver stay on the device.  Every vector operation runs in the gfx950 kernels of ovl_kernels.hip
+// (fields of many modes) and ovl_solvers.hip (Krylov solvers, single vectors).
 #include "../../include/ovl.h"
 #include "ovl_hostcopy.hpp"
 #include "ovl_internal.hpp"
@@ -1545,11 +1546,13 @@ static int ctx_init(ovl_ctx *c)
 
 static int pick_mode_block(int mode_block, int n_modes)
 {
-    // the smallest padding, and of equal paddings the larger block: 33 to 63 modes fill two blocks of 32
-    // with as many slots as one of 64, whose sites read their links through scalar loads (40 modes of
-    // 11 x 14 x 9 SU(3), one Clenshaw step: 46.8 / 36.8 / 25.4 / 19.9 us in FP64 / 48-bit / FP32 / FP16
-    // against 53.2 / 43.3 / 26.7 / 20.5); up to 32 modes a block of 64 would be half empty (32 modes of
-    // 24^3 SU(3): 270 us against 156 in FP64)
+    // the larger the block, the fewer link loads (64 modes read them through scalar loads): 64 unless it would be
+    // half empty.  33 to 63 modes fill two blocks of 32 with as many slots (40 modes of 11 x 14 x 9 SU(3), one
+    // Clenshaw step in 64 and 32: 46.8 / 36.8 / 25.4 / 19.9 us in FP64 / 48-bit / FP32 / FP16 against 53.2 / 43.3 / 26.7 /
+    // 20.5); 32 modes in a block of 64: 270 us against 156 in FP64 on 24^3 SU(3).  Blocks of 16 pad 33 to 48 and 65
+    // to 96 modes less and are then the faster ones (48 degrees in FP64, blocks of 16, 32, 64: 40 modes 24^3 SU(3)
+    // 10.5, 13.3, 11.4 ms, 16^3 SU(2) 2.13, 2.61, 2.56, but 11 x 14 x 9 SU(3) 1.93, 2.13, 1.85; 80 modes 24^3 SU(3) 16.9, 20.0, 23.2,
+    // 16^3 SU(2) 3.26, 3.71, 4.56): mode_block 16, or -1, which times them, takes those.
     if (mode_block > 0) return mode_block;
     return n_modes > 32 ? 64 : (n_modes > 16 ? 32 : 16);
 }

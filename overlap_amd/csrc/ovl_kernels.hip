@@ -298,11 +298,10 @@ __device__ __forceinline__ void store_sp_nt(void *__restrict__ base, int V, int 
 //   TRAV_BOXES: the eighth is XCD k's spatial box of sites (order[k V/8 .. (k+1) V/8)), every
 //     mode block in turn, so x/y/z neighbours are re-read from that XCD's L2 except at the box
 //     faces;
-//   TRAV_MODES: the eighth is a contiguous range of (mode block, site-order position) in
-//     block-major order -- nblk/8 whole blocks when there are at least 8, else 1/(8/nblk) of one
-//     block's site order (a z range, or a range of y slabs) -- with sites in the order of `order`
-//     (y slabs, z-major) or lexicographic, so few sites are fetched by two XCDs and the
-//     z-neighbour planes of a slab stay in L2.
+//   TRAV_MODES: the eighth is a contiguous range of (mode block, site-order position) in block-major order --
+//     whole mode blocks where their number divides by eight, else runs that begin and end anywhere in a
+//     block's site order -- with sites in the order of `order` (y slabs, z-major) or lexicographic, so few
+//     sites are fetched by two XCDs and the z-neighbour planes of a slab stay in L2.
 __device__ __forceinline__ unsigned fdiv(unsigned n, const FastDiv &f)
 {
     return f.d <= 1 ? n : (__umulhi(n, f.mul) >> f.shift);
@@ -332,8 +331,9 @@ __device__ __forceinline__ bool lane_coords(const HopArgs &a, unsigned wg, unsig
         const unsigned i = rr - b * a.dv_v8.d;
         blk = (int)b;
         if (!a.order) {
-            // whole boxes: the site follows from the slot (no table to read before the first load: 1 to 1.5 us
-            // of every launch's chain)
+            // whole boxes: the site follows from the slot, without a table in memory.  Neither way wins throughout
+            // (96 degrees, computed and from a table: SU(2) 32^3, 32 modes FP64 17.2 and 17.7 ms, SU(3) 32^3, 32 modes
+            // FP32 14.38 and 14.58, SU(3) 24^3, 64 modes 11.25 and 11.23, 12^3, 64 modes 2.02 and 1.98).
             const unsigned slow = fdiv(i, a.box.dv_plane), ip = i - slow * a.box.dv_plane.d;
             const unsigned mid = fdiv(ip, a.box.dv_x);
             const unsigned kx = xc & ((1u << a.box.lx) - 1), ky = (xc >> a.box.lx) & ((1u << a.box.ly) - 1);
@@ -1413,7 +1413,10 @@ template <int NC, int LPL> __global__ __launch_bounds__(LINK_TPB) void k_efield_
 // A Wilson half step and a gauge half step in one launch: the first gauge.blocks workgroups (a multiple of the
 // XCDs, so that the others keep theirs) update the links (into other stencil links than the ones being
 // read) or the E field, the rest are the stencil's.  The two do not depend on each other, and on small
-// lattices each is a launch that leaves most of the chip idle.
+// lattices each is a launch that leaves most of the chip idle.  The stencil keeps its registers (VGPRs, 16/32- and
+// 64-mode blocks, as k_hop and here: SU(2) FP64 234, 162 and 236, 164; FP32 124, 82 and 126, 122; SU(3) FP64 398, 244 and
+// 396, 246; FP32 203, 125 and 204, 127), so only SU(2) in FP32 with 64-mode blocks has fewer waves, four instead of
+// five per SIMD.
 template <int NC, typename T, int MB>
 __global__ __launch_bounds__(TPB) void k_hop_gauge(HopArgs a, GaugeHalf g, int n0, int n1, int n2)
 {

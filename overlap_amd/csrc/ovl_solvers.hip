@@ -10,10 +10,11 @@
 // What bounds them is latency: a vector of 8^3 SU(2) is 64 KB, and every phase of an iteration needs
 // the sum of the one before.  Measured on MI355X against host scalars and 16-mode fields (a launch of
 // two kernels, a copy and a synchronisation per inner product, 124 us per CG iteration and 360 us per
-// Ritz iteration): single-mode overlap operator on 12^3 SU(2) 6.22 -> 1.57 ms (28 us per iteration of
-// four launches, 3.3 - 5.5 us each), Zolotarev step of 16 modes on 8^3 SU(2) with its Ritz bounds 348
-// -> 31 ms (five launches of 4.3 - 5.3 us per pair of Ritz iterations), single-mode Wilson operator on
-// 24^3 SU(3) 627 -> 536 us (stencil 37 -> 6 us; the rest is the 11.3 MB of host arrays).
+// Ritz iteration): single-mode overlap operator on 12^3 SU(2) 6.22 -> 1.35 ms (four launches of 3.3 - 5.5 us
+// per iteration, batches of eight as a graph), Zolotarev step of 16 modes on 8^3 SU(2) with its Ritz bounds 348
+// -> 27 ms (five launches of 4.3 - 5.3 us per pair of Ritz iterations, batches of twenty as a graph),
+// single-mode Wilson operator on 24^3 SU(3) 627 -> 545 us (stencil 37 -> 6 us; the rest is the 11.3 MB of
+// host arrays).
 #include "ovl_internal.hpp"
 
 #include <algorithm>
