@@ -1333,7 +1333,8 @@ __device__ __forceinline__ int nbr(int s, int dmu, int step, int n0, int n1, int
 // 15 x 12 x 10, where a lane per link left most CUs without a wave, 17.8 -> 15.3 us on 24^3, where the
 // matrices' strided loads bound it).  The lanes of a wavefront then walk both the forward and the backward
 // products; with LPL = 1, one lane and the same sums, none does: ovl_update_efield
-// with LPL = 4 and 1, SU(2) 16^3 14.8 and 15.5 us, 24^3 17.3 and 15.9, 32^3 21.3 and 17.9, 64^3 72 and 46.  SU(3)
+// with LPL = 4 and 1, SU(2) 16^3 14.8 and 15.5 us, 24^3 17.3 and 15.9, 32^3 21.3 and 17.9, 64^3 72 and 46 (48^3 29.2
+// and 64^3 43.2 in workgroups of one wavefront, 28.4 and 42.1 in workgroups of four).  SU(3)
 // has four lanes throughout: in one lane 24^3 takes 24.5 us instead of 23.7, 48^3 97.6 instead of 88.4.
 
 // sums of ReTr(i t^a U_plaq) (retr_sums) of plaquette j of link (s, mu): plane (mu, the j/2-th other direction), j odd:
@@ -1405,9 +1406,9 @@ __device__ __forceinline__ void efield_update_lane(unsigned lane, const double *
             if (k % 4 == j) o[k] += -2.0 * dt * f[k];
     }
 }
-template <int NC, int LPL> __global__ __launch_bounds__(LINK_TPB) void k_efield_update(GaugeHalf g)
+template <int NC, int LPL, int NT> __global__ __launch_bounds__(NT) void k_efield_update(GaugeHalf g)
 {
-    efield_update_lane<NC, LPL>(blockIdx.x * LINK_TPB + threadIdx.x, g.links, g.efield, g.dt, g.n0, g.n1, g.n2);
+    efield_update_lane<NC, LPL>(blockIdx.x * NT + threadIdx.x, g.links, g.efield, g.dt, g.n0, g.n1, g.n2);
 }
 
 // A Wilson half step and a gauge half step in one launch: the first gauge.blocks workgroups (a multiple of the
@@ -2471,9 +2472,10 @@ hipError_t launch_gauge_half(const Geom &g, const GaugeHalf &h, hipStream_t st)
         else if (h.lpl == 1) k_link_update<3, 1><<<nb, LINK_TPB, 0, st>>>(h);
         else k_link_update<3, 4><<<nb, LINK_TPB, 0, st>>>(h);
     } else {
-        if (g.nc == 3) k_efield_update<3, 4><<<nb, LINK_TPB, 0, st>>>(h);
-        else if (h.lpl == 1) k_efield_update<2, 1><<<nb, LINK_TPB, 0, st>>>(h);
-        else k_efield_update<2, 4><<<nb, LINK_TPB, 0, st>>>(h);
+        // one lane per link fills the chip with workgroups of any size: the larger ones start sooner
+        if (g.nc == 3) k_efield_update<3, 4, LINK_TPB><<<nb, LINK_TPB, 0, st>>>(h);
+        else if (h.lpl == 1) k_efield_update<2, 1, TPB><<<(unsigned)((3L * g.V + TPB - 1) / TPB), TPB, 0, st>>>(h);
+        else k_efield_update<2, 4, LINK_TPB><<<nb, LINK_TPB, 0, st>>>(h);
     }
     return hipGetLastError();
 }
