@@ -1437,10 +1437,17 @@ int ovl_device_name(char *buf, int len)
 // -> 89).  SU(2) vectors of 64-mode blocks between about 20 and 140 MB are better off where the next launch
 // finds them again (plain and streaming, 96 degrees: 16^3 with 64 modes, 34 MB, 5117 and 5169 us, 128 modes
 // 9094 and 9368, 256 modes, 134 MB, 17138 and 17623; outside 12 x 12 x 8 with 128 modes, 19 MB, 3641 and 3556, 28^3 with
-// 64 modes, 180 MB, 25803 and 22769).  FP32 loses 1% with them and the other two precisions do not care.
+// 64 modes, 180 MB, 25803 and 22769).  So are vectors of both groups of 12 to 17.5 MB, two of which about fill the L2s (plain
+// over streaming, 96 degrees in 64-mode blocks: SU(2) 8 x 8 x 24 0.963, 8 x 8 x 28 0.962, 8 x 8 x 32 0.968, 14 x 14 x 8 0.974,
+// 10 x 10 x 20 0.980, 12^3 0.988, 8 x 16 x 16 1.017; SU(3) 8 x 8 x 16 0.949, 10^3 0.963, 9 x 10 x 14 0.972, 11^3 0.975, 6 x 14 x 15
+// 0.978, 8 x 8 x 22, 17.3 MB, 0.970, 8 x 8 x 20 1.010; outside, SU(2) 8 x 8 x 16, 8.4 MB, 1.014, 12 x 12 x 15, 17.7 MB, 1.019, 9 x 9 x 27, 17.9
+// MB, 1.067, SU(3) 12 x 12 x 10, 17.7 MB, 1.010, 8 x 8 x 24, 18.9 MB, 1.026, 16 x 8 x 16, 25.2 MB, 1.079).  FP32 loses 1% with
+// them and the other two precisions do not care.
 static bool streams_fp64(const ovl_ctx *c)
 {
-    const bool kept = !c->ensemble && c->g.nc == 2 && c->g.mb == 64 && c->field64_bytes >= 20000000 && c->field64_bytes <= 140000000;
+    if (c->ensemble || c->g.mb != 64) return true;
+    const double mb = 1e-6 * (double)c->field64_bytes;
+    const bool kept = (mb >= 12 && mb <= 17.5) || (c->g.nc == 2 && mb >= 20 && mb <= 140);
     return !kept;
 }
 

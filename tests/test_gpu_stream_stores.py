@@ -14,6 +14,18 @@ pytestmark = pytest.mark.gpu
                                             (2, (26, 26, 26), 64, 1), (2, (16, 16, 16), 32, 1), (3, (12, 12, 12), 64, 1),
                                             (2, (4, 4, 4), 64, 1)])
 def test_stores_of_a_new_context(gpu, nc, n, nm, stream):
+    check_stores(nc, n, nm, stream)
+
+
+# vectors of both groups around 12 and 17.5 MB: 11.9, 12.0, 16.9 and 17.6; 11.9, 12.0, 17.3 and 17.5
+@pytest.mark.parametrize("nc,n,nm,stream", [(2, (12, 11, 11), 64, 1), (2, (7, 14, 15), 64, 0), (2, (17, 11, 11), 33, 0),
+                                            (2, (13, 11, 15), 64, 1), (3, (11, 11, 8), 64, 1), (3, (10, 7, 14), 64, 0),
+                                            (3, (9, 12, 13), 40, 0), (3, (12, 7, 17), 64, 1)])
+def test_stores_of_vectors_that_pair_in_the_caches(gpu, nc, n, nm, stream):
+    check_stores(nc, n, nm, stream)
+
+
+def check_stores(nc, n, nm, stream):
     print(f"[case] stores nc={nc} n={n} modes={nm}", flush=True)
     links = np.zeros((int(np.prod(n)) * 3, 4 if nc == 2 else 18))
     links[:, [3] if nc == 2 else [0, 8, 16]] = 1.0
